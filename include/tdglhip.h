@@ -200,13 +200,14 @@ typedef struct {
 typedef struct {
   int64_t steps;        /* steps taken by this handle */
   int64_t calls;        /* tdgl_step calls (cycles) */
-  int64_t pcg_iters;    /* PCG iterations summed over steps */
+  int64_t pcg_iters;    /* PCG iterations summed over steps (a solve by sectors: the most of one sector) */
   int32_t last_iters;   /* iterations of the last solve (PCGSolver.iters) */
   double device_ms;     /* device time of the steps, HIP events */
   int64_t device_bytes; /* device memory held by the handle */
   int64_t graph_cycles; /* tdgl_step calls replayed from a captured graph */
   int64_t rollbacks;    /* captured cycles redone eagerly (a solve needed more iterations) */
-  int32_t pcg_budget;   /* PCG iterations per solve in the captured cycle */
+  int32_t pcg_budget;   /* PCG iterations per solve in the captured cycle (a solve by sectors runs to its end on
+                           the device whatever they are: what the general iteration would hold) */
   int64_t captures;     /* graphs captured and instantiated (the last four are kept and replayed) */
   int32_t folded;       /* 1: the Float32 preconditioner runs its parity-folded transforms */
 } tdgl_stats;
@@ -253,7 +254,9 @@ int tdgl_step_noalloc(tdgl_handle *h, int32_t n, double H, double HJ);
  * box_kc changes how the PCG's block partials fall, the z pass's kernel how its sums are grouped
  * and the folds how the preconditioner rounds (each agrees with the others to the PCG tolerance);
  * the m tiles, the vector ALUs' waves, qparts and zcol change no result.  cand[] lists every candidate
- * timed (us per launch of the kernels it shapes; per PCG iteration for fold and zcol). */
+ * timed (us per launch of the kernels it shapes; per PCG iteration for fold and zcol).  A stepper whose
+ * steps solve by sectors (D constant along x and mirror-symmetric) keeps doing so: of the choices only
+ * box_kc, the blocks of its residual kernel, reaches its steps. */
 #define TDGL_TUNE_MAX 16
 enum { TDGL_TUNE_BOX_KC = 1, TDGL_TUNE_PLANE_MT = 2, TDGL_TUNE_ZMODES_WAVES = 3, TDGL_TUNE_FOLD = 4,
        TDGL_TUNE_ZCOL = 5, TDGL_TUNE_QPARTS = 6 };

@@ -189,8 +189,8 @@ hipError_t launch_copies(const CopyList &c, hipStream_t s);
 // ---------------------------------------------------------------- implicit solve (implicit.jl)
 // Scalars, flags and reduction partials of one PCG solve
 // SC_TOLI, SC_NBI: the relative tolerance and the starting residual norm of an inner Float32
-// solve of the refinement (d.pcg_refine)
-enum { SC_NB = 0, SC_RZ0, SC_RZ1, SC_TOL, SC_TOLI, SC_NBI, SC_COUNT };
+// solve of the refinement (d.pcg_refine); SC_RR: ||r||² at the start of a solve by sectors
+enum { SC_NB = 0, SC_RZ0, SC_RZ1, SC_TOL, SC_TOLI, SC_NBI, SC_RR, SC_COUNT };
 // classes of a step for the captured PCG's budgets (PcgArgs::cls): with the open boundary, the
 // steps since its last recomputation of h_δ (0 .. PCG_NCLS - 2, then the rest), whose solves start
 // further from their extrapolated guesses the nearer they are to it; without it, one class
@@ -664,6 +664,55 @@ hipError_t launch_pcg_resid32(const PcgArgs &a, hipStream_t s);
 // x += d32, gated by fl[gate_fl]
 hipError_t launch_pcg_xupdate(const PcgArgs &a, hipStream_t s);
 hipError_t launch_pcg_finish(const PcgArgs &a, hipStream_t s);   // φ = θ + x, the cycle's counts
+
+// ---------------------------------------------------------------------------- the PCG by sectors (sect.hip)
+// The sectors (2 py + pz) of a mode mx < nx: half extents [0 node, 1 edge][parity] along y and z, the
+// elements of a sector, where sector s starts (its modes follow each other) and its components within it
+struct SectDims {
+  int nx, ny, nz;
+  int hy[2][2], hz[2][2];
+  int size[4], oc[3][4];
+  long long off[4], total;
+};
+// the x transform between node-shaped vectors and the sectors (k_sect_fwd, k_sect_inv)
+struct SectX {
+  SectDims q;
+  int L[3][3];              // the components' extents
+  View v[3];                // fwd: the vector read; inv: φ
+  View th[3], x[3];         // inv: θ and the solution x += value
+  double *S;                // the sectors
+  const double *B[2][2];    // half-size x bases [0 V, 1 U][parity], 16 ceil(h / 16) square: fwd (mode, i), inv (i, mode)
+  const int *gate;          // fwd: off unless *gate
+  int nparts;               // fwd: partials of r·r (PART_RR) summed into SC_RR
+  int cls;                  // inv: the step's class (FL_ITMAXC)
+  PcgDev d;
+  int jg, kg;               // set by the launcher
+};
+bool sect_x_fits(const SectX &p);
+hipError_t launch_sect_fwd(SectX p, hipStream_t s);
+hipError_t launch_sect_inv(SectX p, hipStream_t s);
+// the flexible CG of every sector, each in one block (k_sect_cg): A d = r from d = 0
+constexpr int SECT_T = 512;  // threads of a block at most
+struct SectCG {
+  SectDims q;
+  const double *R;          // the sectors of r
+  double *X;                // d
+  PcgDev d;
+  const double *sx;         // singular values along x
+  const float *sfx, *sfy, *sfz;
+  // Float32 half-size bases, zero-padded: [parity][0 node, 1 edge][0 forward (mode, position), weighted; 1 back
+  // (position, mode)], row-major of order yp / zp; edge modes at the place of the node mode of their wave number
+  const float *yb[2][2][2], *zb[2][2][2];
+  int yp, zp;
+  const unsigned char *code[3];  // D on the half domain: component c at j + hy[c == 1][c == 1] k, indices into pal
+  const double *pal;        // DPAL_MAX values a component
+  double ca, a;             // curl-curl coefficient of the operator, a of the preconditioner
+  double share;             // 1 / the number of sectors
+  int maxit;
+  int np, trows;            // set by the launcher: P's elements, T's rows
+};
+bool sect_cg_fits(const SectCG &a);
+hipError_t launch_sect_cg(SectCG a, hipStream_t s);
 hipError_t launch_pcg_cycle_reset(PcgDev d, hipStream_t s);
 
 }  // namespace tdgl

@@ -1,0 +1,682 @@
+// sect.hip — the insulating PCG solved sector by sector.
+//
+// The conductivity of the field solve is constant along x and mirror-symmetric in y and z (the bar and
+// its padding, implicit.jl:126-140), so A = D + aK keeps three symmetries that the general PCG does not
+// use: the x transform of the separable bases (V on nodes, U on edges) turns every x difference into a
+// product with the mode's singular value, and the mirrors split the (y, z) plane of a mode into four
+// parity sectors.  The solve is then 4 (Nx - 1) independent problems on quarter planes, each small
+// enough for one workgroup's LDS and registers: k_sect_fwd takes the residual to the sectors, k_sect_cg
+// runs the whole flexible CG of a sector in one launch, k_sect_inv takes the solution back.  The general
+// iteration's six launches and 860 MB of HBM traffic (290 us on 256x128x32 cells, 20 to 24 a step; 50 us,
+// launch-bound, on 96x48x24) become one launch a solve, whose iterations leave the CU only for the bases and
+// the solution: a time step took 7.86 -> 1.97 ms on 256x128x32 cells, 458 -> 193 us on 96x48x24, 610 -> 224 us on
+// 128x64x16 with KWT, 327 -> 117 us on 53x27x9.
+//
+// A sector holds values on the half domain (the rest follows by parity): component c of mode mx at
+// (j, k), j fastest, X (c = 0) then Y then Z.  With (py, pz) the parities of the sector's y and z wave
+// numbers, a component is node-like (cosine) along an axis other than its own and edge-like (sine, the
+// opposite parity) along its own.  A half axis of n nodes holds ceil(n/2) (even) or floor(n/2) (odd)
+// nodes and ceil(n/2) - 1 or floor(n/2) edges; sums over a whole axis weigh each point by 2, a centre
+// point by 1.  A difference across the centre takes the mirrored value (SectGhost).
+#include "kernels.h"
+
+namespace tdgl {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ v4d ld4d(const double *p) {
+  const v2d lo = *(const v2d *)p, hi = *(const v2d *)(p + 2);
+  return v4d{lo.x, lo.y, hi.x, hi.y};
+}
+__device__ __forceinline__ double wave_sum_d(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// ---------------------------------------------------------------------------- the x transforms
+// Bound: 2 (Lx / 2) flop in FP64 per element on the matrix cores (the fold along x halves the dense
+// product) against 16 B.  A block takes SX_J positions along y at one z and their mirror images, folds
+// them into the four sectors and the two x parities in LDS and multiplies by the half-size x bases
+// (padded to whole 16 x 16 tiles, read through L2); wave w owns the m tiles w, w + waves, ...
+constexpr int SX_J = 8, SX_COLS = 4 * SX_J;
+constexpr int SX_WAVES = 16;
+
+__device__ __forceinline__ int sx_stride(int qs) { return qs + 2; }  // LDS rows of 4 (mod 8) words
+
+struct SxIdx {
+  int c, k, j0;
+};
+__device__ __forceinline__ SxIdx sx_idx(const SectX &p, int b) {
+  const int per = p.jg * p.kg;
+  SxIdx r;
+  r.c = b / per;
+  const int q = b - r.c * per;
+  r.k = q / p.jg;
+  r.j0 = (q - r.k * p.jg) * SX_J;
+  return r;
+}
+
+__device__ __forceinline__ void sect_fwd_body(const SectX &p, int b) {
+  extern __shared__ __align__(16) unsigned char sx_smem[];
+  double *F = (double *)sx_smem;  // [x parity][column][i]
+  const SxIdx ix = sx_idx(p, b);
+  const int c = ix.c, k = ix.k, j0 = ix.j0, tid = threadIdx.x, nth = blockDim.x;
+  const int L0 = p.L[c][0], L1 = p.L[c][1], L2 = p.L[c][2];
+  const int hx = (L0 + 1) / 2, hy = (L1 + 1) / 2, hz = (L2 + 1) / 2;
+  if (k >= hz || j0 >= hy) return;
+  const int mt = (hx + 15) / 16, QS = 16 * mt, IS = sx_stride(QS);
+  const View v = p.v[c];
+  const double *base = (const double *)v.p;
+  const int ks = L2 - 1 - k;
+  for (int t = tid; t < QS * SX_J; t += nth) {
+    const int i = t % QS, jj = t / QS, j = j0 + jj;
+    double f[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    if (i < hx && j < hy) {
+      const int is = L0 - 1 - i, js = L1 - 1 - j;
+      const double *r00 = base + (size_t)v.s1 * j + (size_t)v.s2 * k, *r10 = base + (size_t)v.s1 * js + (size_t)v.s2 * k;
+      const double *r01 = base + (size_t)v.s1 * j + (size_t)v.s2 * ks, *r11 = base + (size_t)v.s1 * js + (size_t)v.s2 * ks;
+      const double a[2][4] = {{r00[i], r10[i], r01[i], r11[i]}, {r00[is], r10[is], r01[is], r11[is]}};
+      double s[2][4];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const double e0 = a[x][0] + a[x][1], o0 = a[x][0] - a[x][1], e1 = a[x][2] + a[x][3], o1 = a[x][2] - a[x][3];
+        s[x][0] = 0.25 * (e0 + e1);  // y even, z even
+        s[x][1] = 0.25 * (e0 - e1);  // y even, z odd
+        s[x][2] = 0.25 * (o0 + o1);  // y odd, z even
+        s[x][3] = 0.25 * (o0 - o1);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f[0][q] = is == i ? s[0][q] : s[0][q] + s[1][q];
+        f[1][q] = is == i ? 0.0 : s[0][q] - s[1][q];
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) F[(x * SX_COLS + q * SX_J + jj) * IS + i] = f[x][q];
+  }
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
+  const int wx = c == 0 ? 1 : 0;
+  for (int m = w; m < mt; m += nw)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      v4d acc[2] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}};
+      const double *A = p.B[wx][x] + (size_t)(16 * m + lr) * QS + 4 * lk;
+      const double *B0 = F + (x * SX_COLS + lr) * IS + 4 * lk, *B1 = B0 + 16 * IS;
+      v4d a = ld4d(A);
+      for (int g = 0; g < mt; ++g) {
+        const v4d an = ld4d(A + 16 * min(g + 1, mt - 1));
+        const v4d b0 = ld4d(B0 + 16 * g), b1 = ld4d(B1 + 16 * g);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b0[u], acc[0], 0, 0, 0);
+          acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b1[u], acc[1], 0, 0, 0);
+        }
+        a = an;
+      }
+      // element r of lane l: mode 2 (16 m + 4 r + lk) + x of the column's sector and position
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int col = 16 * t + lr, q = col / SX_J, j = j0 + col % SX_J;
+        const int py = (q >> 1) ^ (c == 1 ? 1 : 0), pz = (q & 1) ^ (c == 2 ? 1 : 0), s = 2 * py + pz;
+        const int ly = p.q.hy[c == 1 ? 1 : 0][py], lz = p.q.hz[c == 2 ? 1 : 0][pz];
+        if (j >= ly || k >= lz) continue;
+        double *o = p.S + p.q.off[s] + p.q.oc[c][s] + j + (size_t)ly * k;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int mode = 2 * (16 * m + 4 * r + lk) + x;
+          if (mode < L0) o[(size_t)(mode + wx) * p.q.size[s]] = acc[t][r];
+        }
+      }
+    }
+}
+
+// r to the sectors; block 0 also leaves ||r||² (the partials of the residual kernel) in SC_RR
+__global__ void __launch_bounds__(64 * SX_WAVES) k_sect_fwd(SectX p) {
+  if (p.gate && !*p.gate) return;
+  if (blockIdx.x == 0 && p.nparts > 0) {
+    __shared__ double sh[SX_WAVES];
+    const double *part = p.d.part + (size_t)PART_RR * 2 * MAX_PART;
+    double s = 0.0;
+    for (int e = threadIdx.x; e < p.nparts; e += blockDim.x) s += part[2 * e];
+    s = wave_sum_d(s);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += sh[q];
+      p.d.sc[SC_RR] = t;
+    }
+  }
+  sect_fwd_body(p, (int)blockIdx.x);
+}
+
+// Whether the sectors iterate: the source is not zero and the first residual is above the tolerance
+__device__ __forceinline__ bool sect_active(const PcgDev &d) {
+  const double tol = d.sc[SC_TOL] * d.sc[SC_NB];
+  return d.fl[FL_NZ] && sqrt(d.sc[SC_RR]) > tol;
+}
+
+// The way back: out(i) = E + O and out(L - 1 - i) = E - O of the even and odd x modes, the four sectors
+// summed with the signs of the mirror images.  The product is taken transposed (rows: sector r at
+// position lk, columns: 16 consecutive i), so a lane holds the four sectors of its element and a store
+// covers 16 consecutive doubles.  PCG: x += value, φ = θ + x, and the counts of the solve; with addth
+// (the separable field) φ = θ + value.
+template <bool PCG>
+__device__ __forceinline__ void sect_inv_body(const SectX &p, int b, bool act) {
+  extern __shared__ __align__(16) unsigned char sx_smem[];
+  double *F = (double *)sx_smem;  // [x parity][16 t + 4 sector + j][u]
+  const SxIdx ix = sx_idx(p, b);
+  const int c = ix.c, k = ix.k, j0 = ix.j0, tid = threadIdx.x, nth = blockDim.x;
+  const int L0 = p.L[c][0], L1 = p.L[c][1], L2 = p.L[c][2];
+  const int hx = (L0 + 1) / 2, hy = (L1 + 1) / 2, hz = (L2 + 1) / 2;
+  if (k >= hz || j0 >= hy) return;
+  const int mt = (hx + 15) / 16, QS = 16 * mt, IS = sx_stride(QS);
+  const int wx = c == 0 ? 1 : 0;
+  if (act) {
+    for (int t = tid; t < 2 * QS * SX_COLS; t += nth) {
+      const int jj = t % SX_J, q = (t / SX_J) % 4, mode = t / SX_COLS, j = j0 + jj;
+      const int py = (q >> 1) ^ (c == 1 ? 1 : 0), pz = (q & 1) ^ (c == 2 ? 1 : 0), s = 2 * py + pz;
+      const int ly = p.q.hy[c == 1 ? 1 : 0][py], lz = p.q.hz[c == 2 ? 1 : 0][pz];
+      double v = 0.0;
+      if (mode < L0 && j < ly && k < lz) v = p.S[p.q.off[s] + (size_t)(mode + wx) * p.q.size[s] + p.q.oc[c][s] + j + (size_t)ly * k];
+      F[((mode & 1) * SX_COLS + 16 * (jj >> 2) + 4 * q + (jj & 3)) * IS + (mode >> 1)] = v;
+    }
+    __syncthreads();
+  }
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
+  const View vo = p.v[c], vt = p.th[c], vx = p.x[c];
+  for (int m = w; m < mt; m += nw) {
+    v4d acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[x][t] = v4d{0, 0, 0, 0};
+    if (act)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const double *B = p.B[wx][x] + (size_t)(16 * m + lr) * QS + 4 * lk;
+        const double *A0 = F + (x * SX_COLS + lr) * IS + 4 * lk, *A1 = A0 + 16 * IS;
+        v4d bb = ld4d(B);
+        for (int g = 0; g < mt; ++g) {
+          const v4d bn = ld4d(B + 16 * min(g + 1, mt - 1));
+          const v4d a0 = ld4d(A0 + 16 * g), a1 = ld4d(A1 + 16 * g);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            acc[x][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[u], bb[u], acc[x][0], 0, 0, 0);
+            acc[x][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[u], bb[u], acc[x][1], 0, 0, 0);
+          }
+          bb = bn;
+        }
+      }
+    const int i = 16 * m + lr, is = L0 - 1 - i, ks = L2 - 1 - k;
+    if (i >= hx) continue;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int j = j0 + 4 * t + lk, js = L1 - 1 - j;
+      if (j >= hy) continue;
+#pragma unroll
+      for (int xi = 0; xi < 2; ++xi) {
+        if (xi && is == i) continue;
+        double s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = xi ? acc[0][t][q] - acc[1][t][q] : acc[0][t][q] + acc[1][t][q];
+        const double e = s[0] + s[2], o = s[0] - s[2], e1 = s[1] + s[3], o1 = s[1] - s[3];
+        const double val[4] = {e + e1, o + o1, e - e1, o - o1};  // (j, k), (js, k), (j, ks), (js, ks)
+        const int ii = xi ? is : i;
+#pragma unroll
+        for (int im = 0; im < 4; ++im) {
+          if (((im & 1) && js == j) || ((im & 2) && ks == k)) continue;
+          const int jj = (im & 1) ? js : j, kk = (im & 2) ? ks : k;
+          const size_t oo = (size_t)ii + (size_t)vo.s1 * jj + (size_t)vo.s2 * kk;
+          const size_t ot = (size_t)ii + (size_t)vt.s1 * jj + (size_t)vt.s2 * kk;
+          if (PCG) {
+            const size_t ox = (size_t)ii + (size_t)vx.s1 * jj + (size_t)vx.s2 * kk;
+            const double xn = ((double *)vx.p)[ox] + val[im];
+            if (act) ((double *)vx.p)[ox] = xn;
+            ((double *)vo.p)[oo] = ((const double *)vt.p)[ot] + xn;
+          } else {
+            ((double *)vo.p)[oo] = ((const double *)vt.p)[ot] + val[im];
+          }
+        }
+      }
+    }
+  }
+}
+
+__global__ void __launch_bounds__(64 * SX_WAVES) k_sect_inv(SectX p) {
+  const bool act = sect_active(p.d);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    int *fl = p.d.fl;
+    fl[FL_ITSUM] += fl[FL_IT];
+    if (fl[FL_IT] > fl[FL_ITMAX]) fl[FL_ITMAX] = fl[FL_IT];
+    const int cl = p.cls >= 0 && p.cls < PCG_NCLS ? p.cls : 0;
+    if (fl[FL_IT] > fl[FL_ITMAXC + cl]) fl[FL_ITMAXC + cl] = fl[FL_IT];
+  }
+  sect_inv_body<true>(p, (int)blockIdx.x, act);
+}
+
+static int sx_tiles(const SectX &p) {
+  int mt = 1;
+  for (int c = 0; c < 3; ++c) mt = std::max(mt, cdiv(cdiv(p.L[c][0], 2), 16));
+  return mt;
+}
+static size_t sx_lds(int mt) { return (size_t)2 * SX_COLS * (16 * mt + 2) * sizeof(double); }
+constexpr size_t SECT_LDS_MAX = 160 * 1024;
+bool sect_x_fits(const SectX &p) { return sx_lds(sx_tiles(p)) + 1024 <= SECT_LDS_MAX; }
+static void sx_grid(SectX &p, int &blocks, int &threads, size_t &lds) {
+  p.jg = p.kg = 1;
+  for (int c = 0; c < 3; ++c) {
+    p.jg = std::max(p.jg, cdiv(cdiv(p.L[c][1], 2), SX_J));
+    p.kg = std::max(p.kg, cdiv(p.L[c][2], 2));
+  }
+  const int mt = sx_tiles(p);
+  blocks = 3 * p.jg * p.kg;
+  threads = 64 * std::min(SX_WAVES, std::max(4, mt));
+  lds = sx_lds(mt);
+}
+hipError_t launch_sect_fwd(SectX p, hipStream_t s) {
+  if (g_rec) return hipErrorNotSupported;
+  if (!sect_x_fits(p)) return hipErrorInvalidValue;
+  int nb, nt;
+  size_t lds;
+  sx_grid(p, nb, nt, lds);
+  TDGL_LAUNCH(k_sect_fwd, dim3(nb), dim3(nt), lds, s, p);
+  return hipGetLastError();
+}
+hipError_t launch_sect_inv(SectX p, hipStream_t s) {
+  if (g_rec) return hipErrorNotSupported;
+  if (!sect_x_fits(p)) return hipErrorInvalidValue;
+  int nb, nt;
+  size_t lds;
+  sx_grid(p, nb, nt, lds);
+  TDGL_LAUNCH(k_sect_inv, dim3(nb), dim3(nt), lds, s, p);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------- the CG of a sector
+// One block per sector.  r, Q and z_old of a thread's elements (e = tid + threads i) stay in registers,
+// the direction P in LDS (FP64, its stencil reads neighbours), the preconditioner's work array T in LDS
+// (Float32): rows are the sector's z columns (X's, then Z's, then Y's), j or the y mode along the row.
+// The preconditioner multiplies every row by the half-size y basis (16 x 16 x 4 tiles, the basis from
+// L2), then each wave takes 16 y modes through the z transform, the projector and the inverse z
+// transform in registers (a forward tile leaves in a lane the modes its inverse takes as operand), then
+// the inverse y products.  d += αP goes to global memory (it is the output).
+// The sums are FP64, in a fixed order: the same bits every time.
+// Where it stops: a sector's share of (SECT_TIGHT tol ||b||)² is half an equal share and half its share of
+// the first residual, so the sectors' residuals together are below the tolerance, no sector iterates for
+// the others and one that holds almost nothing stops at once.  What is left is spread over the sectors and
+// not where the general iteration leaves it, and at the tolerance itself the fields came out up to nine
+// times further from a solution to the rounding than that iteration's (2.4e-8 against 2.5e-9 after six
+// cycles of 96x48x24 cells, 9.2e-8 against 2.8e-8 after one of 53x27x9); at an eighth of it they are nearer
+// (1.5e-8 on 53x27x9, 3.3e-8 against 2.0e-7 on 144x17x21, 9e-11 against 6e-10 with KWT) or as near (5.4e-9
+// against 2.5e-9 and 7.1e-9, full length and folded, on 96x48x24), for 15 % more iterations.
+constexpr double SECT_TIGHT = 0.125;
+struct SectGhost {
+  double gn, ge;  // mirrored node past the last (even count, odd parity: -1), mirrored edge (odd count, even parity: -1)
+};
+__device__ __forceinline__ SectGhost sect_ghost(int n, int par) {
+  return SectGhost{(n % 2 == 0 && par) ? -1.0 : 0.0, (n % 2 == 1 && !par) ? -1.0 : 0.0};
+}
+
+// the same value, which the compiler does not know to be: what is derived from it is formed where it is used
+// and not kept in registers through the iterations
+__device__ __forceinline__ int fresh(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+template <int EPT, int ZT, int SM>
+__global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
+  if (!sect_active(a.d)) return;
+  extern __shared__ __align__(16) unsigned char cg_smem[];
+  __shared__ double red[4][SECT_T / 64];
+  __shared__ double pal[3 * DPAL_MAX];
+  const int tid = threadIdx.x, nth = blockDim.x, nw = nth >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
+  const int s = blockIdx.x & 3, mx = blockIdx.x >> 2, py = s >> 1, pz = s & 1;
+  const SectDims &q = a.q;
+  const int n = q.size[s], ly = q.hy[0][py], le = q.hy[1][py], lz = q.hz[0][pz], lze = q.hz[1][pz];
+  const int oY = q.oc[1][s], oZ = q.oc[2][s];
+  double *P = (double *)cg_smem;
+  float *T = (float *)(P + a.np);
+  const int ST = a.yp + 4, CY = lz + lze;
+  const int mt = (ly + 15) / 16, nt1 = (CY + 15) / 16, nt2 = (lz + 15) / 16, ntile = mt * (nt1 + nt2);
+  for (int t = tid; t < a.trows * ST; t += nth) T[t] = 0.0f;
+  if (tid < 3 * DPAL_MAX) pal[tid] = a.pal[tid];
+  const double sv = a.sx[mx], ca = a.ca;
+  const double tolb = a.d.sc[SC_TOL] * a.d.sc[SC_NB];
+  const SectGhost gy = sect_ghost(q.ny, py), gz = sect_ghost(q.nz, pz);
+  const size_t base = (size_t)q.off[s] + (size_t)mx * n;
+
+  // this thread's elements: j | k << 10 | component << 20 | log2 weight << 22 | D code << 24 | live << 28
+  unsigned id[EPT];
+  double r[EPT];
+  float zo[EPT];
+  double rr = 0.0;
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int e = tid + nth * i;
+    id[i] = 0u;
+    r[i] = 0.0;
+    zo[i] = 0.0f;
+    if (e < n) {
+      const int c = e < oY ? 0 : (e < oZ ? 1 : 2), f = e - (c == 0 ? 0 : (c == 1 ? oY : oZ)), row = c == 1 ? le : ly;
+      const int k = f / row, j = f - k * row;
+      const bool cy = c == 1 ? (q.ny % 2 == 0 && py && j == le - 1) : (q.ny % 2 == 1 && !py && j == ly - 1);
+      const bool cz = c == 2 ? (q.nz % 2 == 0 && pz && k == lze - 1) : (q.nz % 2 == 1 && !pz && k == lz - 1);
+      const unsigned wt = (cy ? 0u : 1u) + (cz ? 0u : 1u);
+      const unsigned code = a.code[c][j + q.hy[c == 1][c == 1] * k];
+      id[i] = (unsigned)j | ((unsigned)k << 10) | ((unsigned)c << 20) | (wt << 22) | (code << 24) | (1u << 28);
+      if (!(c == 0 && mx == 0)) r[i] = a.R[base + e];
+      rr += (double)(1u << wt) * (r[i] * r[i]);
+    }
+  }
+  auto sum_of = [&](int slot, double v) {
+    v = wave_sum_d(v);
+    if (l == 0) red[slot][w] = v;
+  };
+  auto total = [&](int slot) {
+    double t = 0.0;
+    for (int k = 0; k < nw; ++k) t += red[slot][k];
+    return t;
+  };
+  sum_of(0, rr);
+  __syncthreads();
+  rr = total(0);
+  const double thr = SECT_TIGHT * SECT_TIGHT * 0.5 * tolb * tolb * (a.share + rr / a.d.sc[SC_RR]);
+  if (!(rr > thr)) {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i)
+      if (id[i] >> 28) a.X[base + tid + nth * i] = 0.0;
+    return;
+  }
+  auto tcol = [&](unsigned v) {  // the element's place in T
+    const int j = v & 1023, k = (v >> 10) & 1023, c = (v >> 20) & 3;
+    return (c == 0 ? k : (c == 1 ? CY + k : lz + k)) * ST + j;
+  };
+  // one pass of the y products over the rows of T: rows x basis, in place
+  auto ypass = [&](const float *BV, const float *BU) {
+    const int la = fresh(lr) * a.yp + 4 * lk, lb = fresh(lr) * ST + 4 * lk;
+    v4f acc[SM];
+#pragma unroll
+    for (int t = 0; t < SM; ++t) {
+      acc[t] = v4f{0, 0, 0, 0};
+      const int tt = w + nw * t;
+      if (tt < ntile) {
+        const int m = tt % mt, nt = tt / mt;
+        const float *A = (nt < nt1 ? BV : BU) + 16 * m * a.yp + la;
+        const float *B = T + (nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1)) * ST + lb;
+        v4f av = *(const v4f *)A;
+        for (int g = 0; g < mt; ++g) {
+          const v4f an = *(const v4f *)(A + 16 * min(g + 1, mt - 1));
+          const v4f bv = *(const v4f *)(B + 16 * g);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc[t], 0, 0, 0);
+          av = an;
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < SM; ++t) {
+      const int tt = w + nw * t;
+      if (tt < ntile) {
+        const int m = tt % mt, nt = tt / mt;
+        const int col0 = nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1);
+        if (col0 + lr < (nt < nt1 ? CY : CY + lz)) *(v4f *)(T + col0 * ST + 16 * m + lb) = acc[t];
+      }
+    }
+    __syncthreads();
+  };
+
+  double rzold = 0.0;
+  int it = 0;
+  for (;;) {
+    // z = M⁻¹ r in Float32
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) id[i] = (unsigned)fresh((int)id[i]);
+#pragma unroll
+    for (int i = 0; i < EPT; ++i)
+      if (id[i] >> 28) T[tcol(id[i])] = (float)r[i];
+    __syncthreads();
+    ypass(a.yb[py][0][0], a.yb[py][1][0]);
+    for (int m = w; m < mt; m += nw) {
+      // 16 y modes: z forward, the projector, z back; k = 16 g + 4 lk + u of the rows (zero past them)
+      v4f Bx[ZT], By[ZT], Bz[ZT];
+      const int lf = fresh(l), lr = lf & 15, lk = lf >> 4;
+      const float *Tq = T + 16 * m + lr;
+#pragma unroll
+      for (int g = 0; g < ZT; ++g)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int k = 16 * g + 4 * lk + u;
+          const float vx = Tq[min(k, lz - 1) * ST], vy = Tq[(CY + min(k, lz - 1)) * ST], vz = Tq[(lz + min(k, lze - 1)) * ST];
+          Bx[g][u] = k < lz ? vx : 0.0f;
+          By[g][u] = k < lz ? vy : 0.0f;
+          Bz[g][u] = k < lze ? vz : 0.0f;
+        }
+      v4f acc[3][ZT];
+#pragma unroll
+      for (int t = 0; t < ZT; ++t) {
+        acc[0][t] = acc[1][t] = acc[2][t] = v4f{0, 0, 0, 0};
+#pragma unroll
+        for (int g = 0; g < ZT; ++g) {
+          const v4f Av = *(const v4f *)(a.zb[pz][0][0] + (16 * t + lr) * a.zp + 16 * g + 4 * lk);
+          const v4f Au = *(const v4f *)(a.zb[pz][1][0] + (16 * t + lr) * a.zp + 16 * g + 4 * lk);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Av[u], Bx[g][u], acc[0][t], 0, 0, 0);
+            acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Av[u], By[g][u], acc[1][t], 0, 0, 0);
+            acc[2][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Au[u], Bz[g][u], acc[2][t], 0, 0, 0);
+          }
+        }
+      }
+      {
+        const int my = 2 * (16 * m + lr) + py;
+        const float k1 = a.sfx[mx], k2 = my < q.ny ? a.sfy[my] : 0.0f;
+        const bool live = my < q.ny, hx = mx > 0, hy = my > 0;
+#pragma unroll
+        for (int t = 0; t < ZT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int mz = 2 * (16 * t + 4 * lk + e) + pz;
+            if (!live || mz >= q.nz) continue;
+            const float k3 = a.sfz[mz], k2s = k1 * k1 + k2 * k2 + k3 * k3;
+            const bool hz = mz > 0;
+            float x1 = hx ? acc[0][t][e] : 0.0f, y1 = hy ? acc[1][t][e] : 0.0f, z1 = hz ? acc[2][t][e] : 0.0f;
+            if (k2s != 0) {  // (I + aK)^{-1} = P_L + P_T / (1 + a |k|²) (implicit.jl:67-78)
+              const float dd = (k1 * x1 + k2 * y1 + k3 * z1) / k2s, f = 1.0f / (1.0f + (float)a.a * k2s);
+              if (hx) x1 = k1 * dd + f * (x1 - k1 * dd);
+              if (hy) y1 = k2 * dd + f * (y1 - k2 * dd);
+              if (hz) z1 = k3 * dd + f * (z1 - k3 * dd);
+            }
+            acc[0][t][e] = x1;
+            acc[1][t][e] = y1;
+            acc[2][t][e] = z1;
+          }
+      }
+      __builtin_amdgcn_wave_barrier();  // the tile's columns are read: their rows take the result
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const int row0 = c == 0 ? 0 : (c == 1 ? CY : lz), rows = c == 2 ? lze : lz;
+        float *To = T + row0 * ST + 16 * m + lr;
+#pragma unroll
+        for (int t = 0; t < ZT; ++t) {
+          v4f o = v4f{0, 0, 0, 0};
+#pragma unroll
+          for (int g = 0; g < ZT; ++g) {
+            const v4f A = *(const v4f *)(a.zb[pz][c == 2 ? 1 : 0][1] + (16 * t + lr) * a.zp + 16 * g + 4 * lk);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) o = __builtin_amdgcn_mfma_f32_16x16x4f32(A[u], acc[c][g][u], o, 0, 0, 0);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int k = 16 * t + 4 * lk + e;
+            if (k < rows) To[k * ST] = o[e];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    ypass(a.yb[py][0][1], a.yb[py][1][1]);
+    // the dots and the direction
+    float z[EPT];
+    double rz = 0.0, rzo = 0.0;
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      z[i] = 0.0f;
+      if (id[i] >> 28) {
+        z[i] = T[tcol(id[i])];
+        const double wr = (double)(1u << ((id[i] >> 22) & 3u)) * r[i];
+        rz += wr * (double)z[i];
+        rzo += wr * (double)zo[i];
+        zo[i] = z[i];
+      }
+    }
+    sum_of(0, rz);
+    sum_of(1, rzo);
+    __syncthreads();
+    rz = total(0);
+    rzo = total(1);
+    const double beta = it > 0 ? (rz - rzo) / rzold : 0.0;
+    rzold = rz;
+#pragma unroll
+    for (int i = 0; i < EPT; ++i)
+      if (id[i] >> 28) {
+        const int e = tid + nth * i;
+        P[e] = it > 0 ? (double)z[i] + beta * P[e] : (double)z[i];
+      }
+    __syncthreads();
+    // Q = (D + aK) P on the half domain
+    double Q[EPT], pq = 0.0;
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      Q[i] = 0.0;
+      const unsigned v = (unsigned)fresh((int)id[i]);
+      if (v >> 28) {
+        const int j = v & 1023, k = (v >> 10) & 1023, c = (v >> 20) & 3;
+        const double *PX = P + j + ly * k, *PY = P + oY + j + le * k, *PZ = P + oZ + j + ly * k;
+        // curl components at edge offsets (dj, dk) of the element: hz and hx need the node past the edge
+        // along y, hy and hx along z
+        auto hzv = [&](int dj) {
+          const double up = j + dj + 1 < ly ? PX[dj + 1] : gy.gn * PX[dj];
+          return sv * PY[dj] - (up - PX[dj]);
+        };
+        auto hyv = [&](int dk) {
+          const double up = k + dk + 1 < lz ? PX[ly * (dk + 1)] : gz.gn * PX[ly * dk];
+          return (up - PX[ly * dk]) - sv * PZ[ly * dk];
+        };
+        auto hxv = [&](int dj, int dk) {
+          const double *z0 = PZ + dj + ly * dk, *y0 = PY + dj + le * dk;
+          const double zu = j + dj + 1 < ly ? z0[1] : gy.gn * z0[0], yu = k + dk + 1 < lz ? y0[le] : gz.gn * y0[0];
+          return (zu - z0[0]) - (yu - y0[0]);
+        };
+        double cur, pc;
+        if (c == 0) {
+          const double hzm = j > 0 ? hzv(-1) : 0.0, hzc = j < le ? hzv(0) : gy.ge * hzm;
+          const double hym = k > 0 ? hyv(-1) : 0.0, hyc = k < lze ? hyv(0) : gz.ge * hym;
+          cur = (hzc - hzm) - (hyc - hym);
+          pc = PX[0];
+        } else if (c == 1) {
+          const double hxm = k > 0 ? hxv(0, -1) : 0.0, hxc = k < lze ? hxv(0, 0) : gz.ge * hxm;
+          cur = (hxc - hxm) + sv * hzv(0);
+          pc = PY[0];
+        } else {
+          const double hxm = j > 0 ? hxv(-1, 0) : 0.0, hxc = j < le ? hxv(0, 0) : gy.ge * hxm;
+          cur = -(sv * hyv(0)) - (hxc - hxm);
+          pc = PZ[0];
+        }
+        Q[i] = pal[DPAL_MAX * c + ((v >> 24) & 15u)] * pc + ca * cur;
+        pq += (double)(1u << ((v >> 22) & 3u)) * (pc * Q[i]);
+      }
+    }
+    sum_of(2, pq);
+    double dv[EPT];
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) dv[i] = (it > 0 && (id[i] >> 28)) ? a.X[base + tid + nth * i] : 0.0;
+    __syncthreads();
+    const double al = rz / total(2);
+    rr = 0.0;
+#pragma unroll
+    for (int i = 0; i < EPT; ++i)
+      if (id[i] >> 28) {
+        const int e = tid + nth * i;
+        a.X[base + e] = dv[i] + al * P[e];
+        r[i] -= al * Q[i];
+        rr += (double)(1u << ((id[i] >> 22) & 3u)) * (r[i] * r[i]);
+      }
+    ++it;
+    sum_of(3, rr);
+    __syncthreads();
+    rr = total(3);
+    if (!(rr > thr) || it >= a.maxit) break;
+  }
+  if (tid == 0) atomicMax(a.d.fl + FL_IT, it);
+}
+
+// The launch of the sectors' CG: threads, elements a thread, y tiles a wave.  8 waves a block, and EPT
+// elements a thread of the sector's size; two blocks share a CU's LDS on the largest grids.
+struct CgPick {
+  bool ok;
+  int threads, ept, zt, sm;
+  size_t lds;
+};
+static CgPick cg_pick(const SectCG &a0, int &np, int &trows) {
+  CgPick k{};
+  const SectDims &q = a0.q;
+  int n = 0, ntile = 0;
+  trows = 0;
+  for (int s = 0; s < 4; ++s) {
+    const int py = s >> 1, pz = s & 1, lz = q.hz[0][pz], lze = q.hz[1][pz], CY = lz + lze;
+    if (q.hy[0][py] < 1 || q.hy[1][py] < 1 || lz < 1 || lze < 1) return k;
+    if (q.hy[0][py] > 1023 || lz > 1023) return k;
+    n = std::max(n, q.size[s]);
+    const int mt = cdiv(q.hy[0][py], 16), nt = cdiv(CY, 16) + cdiv(lz, 16);
+    ntile = std::max(ntile, mt * nt);
+    trows = std::max(trows, CY + 16 * cdiv(lz, 16));
+  }
+  np = (n + 1) / 2 * 2;
+  k.zt = cdiv(q.hz[0][0], 16);
+  const int epts[4] = {2, 4, 8, 11};
+  for (int e : epts) {
+    const int th = 64 * std::max(4, cdiv(n, 64 * e));
+    if (th > SECT_T) continue;
+    k.threads = th;
+    k.ept = e;
+    break;
+  }
+  if (!k.threads) return k;
+  k.sm = cdiv(ntile, k.threads / 64);
+  k.lds = (size_t)np * sizeof(double) + (size_t)trows * (a0.yp + 4) * sizeof(float);
+  k.ok = k.zt <= 3 && k.sm <= 6 && k.lds + 1024 <= SECT_LDS_MAX;
+  k.sm = k.sm <= 3 ? 3 : 6;
+  return k;
+}
+bool sect_cg_fits(const SectCG &a) {
+  int np, tr;
+  return cg_pick(a, np, tr).ok;
+}
+hipError_t launch_sect_cg(SectCG a, hipStream_t s) {
+  if (g_rec) return hipErrorNotSupported;
+  const CgPick k = cg_pick(a, a.np, a.trows);
+  if (!k.ok) return hipErrorInvalidValue;
+  const dim3 grid(4 * a.q.nx), blk(k.threads);
+#define TDGL_CG(E, Z, M)                                              \
+  if (k.ept == E && k.zt == Z && k.sm == M) {                         \
+    TDGL_LAUNCH((k_sect_cg<E, Z, M>), grid, blk, k.lds, s, a);        \
+    return hipGetLastError();                                         \
+  }
+#define TDGL_CG_E(E) TDGL_CG(E, 1, 3) TDGL_CG(E, 2, 3) TDGL_CG(E, 3, 3) TDGL_CG(E, 1, 6) TDGL_CG(E, 2, 6) TDGL_CG(E, 3, 6)
+  TDGL_CG_E(2) TDGL_CG_E(4) TDGL_CG_E(8) TDGL_CG_E(11)
+#undef TDGL_CG_E
+#undef TDGL_CG
+  return hipErrorInvalidValue;
+}
+
+}  // namespace tdgl

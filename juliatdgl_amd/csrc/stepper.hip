@@ -61,11 +61,11 @@ Bases make_bases(int nn) {
 }
 
 // kernel classes of the per-kernel profile (tdgl_profile_get)
-enum { K_STAGE = 0, K_QP, K_FIELD, K_CURL, K_GHOSTS, K_SCATTER, K_TX, K_TX32, K_MODES, K_APPLYA, K_DOT, K_FINISH, K_VEC, K_METER,
+enum { K_STAGE = 0, K_QP, K_FIELD, K_CURL, K_GHOSTS, K_SCATTER, K_TX, K_TX32, K_MODES, K_APPLYA, K_SECT, K_FINISH, K_VEC, K_METER,
        K_FOLD, K_COUNT };
 const char *const K_NAMES[K_COUNT] = {"band_stage", "normal_fluids", "current_field", "links_curl_bc", "neumann_ghosts",
                                       "solve_scatter", "sep_transform_f64", "sep_transform_f32", "sep_modes", "pcg_apply_A",
-                                      "pcg_dot", "pcg_finish", "pcg_vector", "cycle_meter", "sep_fold"};
+                                      "pcg_sectors", "pcg_finish", "pcg_vector", "cycle_meter", "sep_fold"};
 static_assert(K_COUNT == TDGL_NKERNELS, "kernel classes");
 
 // a device or pinned host block of the process's cache
@@ -149,6 +149,7 @@ struct tdgl_handle {
   // the parity-folded Float32 preconditioner: quarters, their two buffers, the half-size bases
   // [axis][0=V,1=U][parity][0=fwd,1=inv]
   bool fold = false;
+  bool general = false;        // general_setup has run
   Quarters q{};
   float *qa = nullptr, *qb = nullptr;
   float *Hq[2][2][2][2] = {};
@@ -167,6 +168,15 @@ struct tdgl_handle {
   double *Hq64[2][2][2][2] = {};
   double *Hp64[2][2][2][2] = {};  // Hq64 zero-padded to whole 16 x 16 tiles (k_qplane64)
   double *zqb64[4] = {};
+  // the PCG by sectors (sect.hip): D constant along x and mirror-symmetric in y and z (TDGL_HIP_SECT=0: the
+  // general iteration); the sectors of r and of the solution lie in T1 and T2
+  bool sect = false;
+  SectDims sq{};
+  double *sxB[2][2][2] = {};   // x half bases [0 V, 1 U][parity][0 forward, 1 back], zero-padded to whole tiles
+  float *syb[2][2][2] = {}, *szb[2][2][2] = {};  // SectCG::yb, zb
+  int syp = 0, szp = 0;
+  unsigned char *scode[3] = {};
+  double *spal = nullptr;
   bool tx_only = false;                   // the separable solve as single-axis passes (a mixed batch)
   int box_kc = 1;                         // levels of k per block of the PCG box kernels
   int plane1 = 1;                         // PlanePass::one of the Float32 launches
@@ -795,6 +805,31 @@ struct SepOut {
   const Vec3f *r32 = nullptr, *zold32 = nullptr;
 };
 
+// The sectors of the solve region (SectDims) of nx x ny x nz nodes
+SectDims sect_dims(int nx, int ny, int nz) {
+  SectDims q{};
+  q.nx = nx;
+  q.ny = ny;
+  q.nz = nz;
+  for (int par = 0; par < 2; ++par) {
+    q.hy[0][par] = par ? ny / 2 : (ny + 1) / 2;
+    q.hz[0][par] = par ? nz / 2 : (nz + 1) / 2;
+    q.hy[1][par] = par ? ny / 2 : (ny + 1) / 2 - 1;
+    q.hz[1][par] = par ? nz / 2 : (nz + 1) / 2 - 1;
+  }
+  for (int s = 0; s < 4; ++s) {
+    const int py = s >> 1, pz = s & 1;
+    const int x = q.hy[0][py] * q.hz[0][pz], y = q.hy[1][py] * q.hz[0][pz], z = q.hy[0][py] * q.hz[1][pz];
+    q.oc[0][s] = 0;
+    q.oc[1][s] = x;
+    q.oc[2][s] = x + y;
+    q.size[s] = x + y + z;
+    q.off[s] = q.total;
+    q.total += (long long)nx * q.size[s];
+  }
+  return q;
+}
+
 // The quarters of the parity folds of the solve region (Quarters): four per component, in the
 // order (component, 2 px + py); qe[4 c + k] their extents
 Quarters quarters_of(const Ranges &rg, int qe[12][3]) {
@@ -1373,11 +1408,90 @@ int implicit_pcg_refine(tdgl_handle *h) {
   return 0;
 }
 
+// ---------------------------------------------------------------------------- the PCG by sectors
+SectX sect_x(tdgl_handle *h, bool inv) {
+  SectX p{};
+  p.q = h->sq;
+  p.d = h->pd;
+  p.cls = h->cur_cls;
+  for (int c = 0; c < 3; ++c)
+    for (int a = 0; a < 3; ++a) p.L[c][a] = h->rg.e[c][a];
+  for (int w = 0; w < 2; ++w)
+    for (int par = 0; par < 2; ++par) p.B[w][par] = h->sxB[w][par][inv];
+  return p;
+}
+SectCG sect_cg(tdgl_handle *h) {
+  SectCG a{};
+  a.q = h->sq;
+  a.R = h->T1;
+  a.X = h->T2;
+  a.d = h->pd;
+  a.sx = h->sd[0];
+  a.sfx = h->sf[0];
+  a.sfy = h->sf[1];
+  a.sfz = h->sf[2];
+  for (int par = 0; par < 2; ++par)
+    for (int w = 0; w < 2; ++w)
+      for (int t = 0; t < 2; ++t) {
+        a.yb[par][w][t] = h->syb[par][w][t];
+        a.zb[par][w][t] = h->szb[par][w][t];
+      }
+  a.yp = h->syp;
+  a.zp = h->szp;
+  for (int c = 0; c < 3; ++c) a.code[c] = h->scode[c];
+  a.pal = h->spal;
+  a.ca = h->d.sxy / (h->d.dx * h->d.dy);
+  a.a = h->d.a;
+  a.share = 1.0 / (4.0 * h->sq.nx);
+  a.maxit = h->d.pcg_maxit;
+  return a;
+}
+
+// _implicit_curl_fast! (implicit.jl:372-446) by sectors: the start and the residual as the general
+// iteration's, the residual to the sectors, the flexible CG of every sector to its own convergence in one
+// launch, the solution's increment back (x += d, φ = θ + x).  Nothing is gated by a budget of iterations,
+// and the host waits for nothing.
+int implicit_pcg_sect(tdgl_handle *h) {
+  const tdgl_desc &d = h->d;
+  const bool extrap = d.pcg_extrap && d.pcg_fast;
+  const int *nz = h->pd.fl + FL_NZ;
+  PcgArgs a = pcg_args(h);
+  a.warm = h->warm;
+  a.extrap = extrap;
+  a.have2 = h->have2;
+  a.nparts_in = field_blocks(h->g);
+  PL(K_VEC, launch_pcg_start(a, h->s));
+  if (!h->warm) {  // cold start: x = M⁻¹ b in Float64
+    SepOut o{&h->x, false, 0};
+    CHK(sep_solve(h, h->B, o, nz, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
+  }
+  h->have2 = h->warm && extrap;
+  h->warm = true;
+  PL(K_APPLYA, launch_pcg_resid(a, h->s));
+  SectX f = sect_x(h, false);
+  for (int c = 0; c < 3; ++c) f.v[c] = node_view(h, h->r.c[c]);
+  f.S = h->T1;
+  f.gate = nz;
+  f.nparts = pcg_box_blocks(h->g, h->box_kc);
+  PL(K_TX, launch_sect_fwd(f, h->s));
+  PL(K_SECT, launch_sect_cg(sect_cg(h), h->s));
+  SectX b = sect_x(h, true);
+  for (int c = 0; c < 3; ++c) {
+    b.v[c] = node_view(h, h->ph[c]);
+    b.th[c] = node_view(h, h->th[c]);
+    b.x[c] = node_view(h, h->x.c[c]);
+  }
+  b.S = h->T2;
+  PL(K_TX, launch_sect_inv(b, h->s));
+  return 0;
+}
+
 // implicit_curl!(s, ::PCGSolver) / _implicit_curl_fast! (implicit.jl:279-446), after the field
 // kernel has written b = φₑ − θ and the partials of b·b, and scaled φ by D.  Eager: the host
 // reads the flags between batches of iterations.  Captured: `budget` iterations, each gated.
 int implicit_pcg(tdgl_handle *h) {
   if (h->refine) return implicit_pcg_refine(h);
+  if (h->sect) return implicit_pcg_sect(h);
   const tdgl_desc &d = h->d;
   const bool fast = d.pcg_fast || d.pcg_f32;
   const bool f32 = d.pcg_f32 != 0;
@@ -1933,7 +2047,9 @@ int destroy_graph(tdgl_handle *h) {
 constexpr int BUDGET_SLACK = 6, BUDGET_RUN = 2, BUDGET_HOLD = 4;
 int cycle_graph(tdgl_handle *h, int n) {
   const bool pcg = h->d.field_mode == TDGL_FIELD_PCG;
-  const GraphKey key{n, h->parity, h->warm ? 1 : 0, h->have2 ? 1 : 0, pcg ? h->budget : 0, 0};
+  // a solve by sectors holds no budget of iterations: nothing to overrun, no start to keep
+  const bool gated = pcg && !h->sect;
+  const GraphKey key{n, h->parity, h->warm ? 1 : 0, h->have2 ? 1 : 0, gated ? h->budget : 0, 0};
   const HostSnap start = snap(h);
   CachedGraph *g = nullptr;
   CachedGraph *const gc0 = h->gc, *const gc1 = h->gc + GRAPH_CACHE_CALL;
@@ -1972,10 +2088,8 @@ int cycle_graph(tdgl_handle *h, int n) {
     restore(h, start);
   }
   g->used = ++h->gtick;
-  if (pcg) {
-    PL(K_VEC, launch_copies(backup_list(h, true), h->s));
-    PL(K_VEC, launch_pcg_cycle_reset(h->pd, h->s));
-  }
+  if (gated) PL(K_VEC, launch_copies(backup_list(h, true), h->s));
+  if (pcg) PL(K_VEC, launch_pcg_cycle_reset(h->pd, h->s));
   HIPCHK(hipGraphLaunch(g->exec, h->s));
   restore(h, g->end);
   if (pcg) {
@@ -2027,12 +2141,12 @@ int d_maxit(tdgl_handle *h) { return h->d.pcg_maxit; }
 int stepwise_graphs(tdgl_handle *h, int n) {
   const HostSnap start = snap(h);
   const int clock0 = h->oclock;
-  PL(K_VEC, launch_copies(backup_list(h, true), h->s));
+  if (!h->sect) PL(K_VEC, launch_copies(backup_list(h, true), h->s));
   PL(K_VEC, launch_pcg_cycle_reset(h->pd, h->s));
   for (int q = 0; q < n; ++q) {
     const int c = step_class(h);
     h->cur_cls = c;
-    const GraphKey key{1, h->parity, h->warm ? 1 : 0, h->have2 ? 1 : 0, h->cbudget[c], c};
+    const GraphKey key{1, h->parity, h->warm ? 1 : 0, h->have2 ? 1 : 0, h->sect ? 0 : h->cbudget[c], c};
     const HostSnap before = snap(h);
     CachedGraph *g = nullptr;
     for (CachedGraph &cg : h->gc)
@@ -2174,6 +2288,242 @@ int check_desc(const tdgl_desc *d, char *why, size_t n) {
   const double cells = (double)(((d->Nx + 1 + 7) / 8) * 8) * (d->Ny + 1) * (d->Nz + 1);
   if (cells > 2.0e9) return no("grid too large for 32-bit indexing");
   return 1;
+}
+
+// The parity-folded Float32 preconditioner of the general iteration (TDGL_HIP_FOLD=0: the full-length
+// transforms): its quarters and half-size bases, where the quarters fit its kernels
+int fold_setup(tdgl_handle *h) {
+  const tdgl_desc &d = h->d;
+  const Ranges &rg = h->rg;
+  // the parity-folded Float32 preconditioner (TDGL_HIP_FOLD=0: the full-length transforms)
+  const char *gf = std::getenv("TDGL_HIP_FOLD"), *gp = std::getenv("TDGL_HIP_PLANE");
+  if (d.field_mode == TDGL_FIELD_PCG && d.pcg_f32 && !(gf && gf[0] == '0') && !(gp && gp[0] == '0') &&
+      d.Nz - 1 >= 2 && d.Nz - 1 <= ZQ_NZ_MAX) {
+    int qe[12][3];
+    const Quarters q = quarters_of(rg, qe);
+    if (plane_fits<float>(qe, 12) && fold_blocks(q) <= MAX_PART) {
+      h->q = q;
+      ALLOC(h->qa, q.total);
+      ALLOC(h->qb, q.total);
+      const int nn[2] = {d.Nx - 1, d.Ny - 1};
+      for (int ax = 0; ax < 2; ++ax) {
+        const Bases b = make_bases(nn[ax]);
+        for (int which = 0; which < 2; ++which) {
+          const std::vector<double> &M = which == 0 ? b.V : b.U;
+          const int L = which == 0 ? nn[ax] : nn[ax] - 1, Lh = (L + 1) / 2;
+          for (int par = 0; par < 2; ++par) {
+            // the columns of parity `par` on the first ceil(L/2) rows: Mh(i, cc) = M(i, 2 cc + par)
+            std::vector<float> hf((size_t)Lh * Lh, 0.0f), hi((size_t)Lh * Lh, 0.0f);
+            for (int i = 0; i < Lh; ++i)
+              for (int cc = 0; cc < Lh; ++cc) {
+                const int col = 2 * cc + par;
+                const float v = col < L ? (float)M[i + (size_t)L * col] : 0.0f;
+                hf[(size_t)i * Lh + cc] = v;  // Mh(i, cc)
+                hi[(size_t)cc * Lh + i] = v;  // Hi[q][m] = Mh(m, q)
+              }
+            ALLOC(h->Hq[ax][which][par][0], hf.size());
+            CHK(upload_vec(h, h->Hq[ax][which][par][0], hf));
+            ALLOC(h->Hq[ax][which][par][1], hi.size());
+            CHK(upload_vec(h, h->Hq[ax][which][par][1], hi));
+            // the same, zero-padded to whole 16 x 16 tiles (k_qplane)
+            const int LP = 16 * cdiv(Lh, 16);
+            for (int t = 0; t < 2; ++t) {
+              const std::vector<float> &src = t == 0 ? hf : hi;
+              std::vector<float> pd((size_t)LP * LP, 0.0f);
+              for (int r = 0; r < Lh; ++r)
+                for (int c = 0; c < Lh; ++c) pd[(size_t)r * LP + c] = src[(size_t)r * Lh + c];
+              ALLOC(h->Hp[ax][which][par][t], pd.size());
+              CHK(upload_vec(h, h->Hp[ax][which][par][t], pd));
+            }
+            h->HpL[ax][which] = Lh;
+          }
+        }
+      }
+      {
+        // the z pass's padded bases: V(n, mz), and U(n, mz - 1) with its zero column and row
+        const int nz = d.Nz - 1, Lu = nz - 1;
+        const Bases b = make_bases(nz);
+        std::vector<float> zb[4];
+        for (int k = 0; k < 4; ++k) zb[k].assign((size_t)nz * nz + ZQ_SLACK, 0.0f);
+        for (int n = 0; n < nz; ++n)
+          for (int mz = 0; mz < nz; ++mz) {
+            const float v = (float)b.V[n + (size_t)nz * mz];
+            const float u = (mz >= 1 && n < Lu) ? (float)b.U[n + (size_t)Lu * (mz - 1)] : 0.0f;
+            zb[0][(size_t)n * nz + mz] = v;
+            zb[1][(size_t)n * nz + mz] = u;
+            zb[2][(size_t)mz * nz + n] = v;
+            zb[3][(size_t)mz * nz + n] = u;
+          }
+        for (int k = 0; k < 4; ++k) {
+          ALLOC(h->zqb[k], zb[k].size());
+          CHK(upload_vec(h, h->zqb[k], zb[k]));
+        }
+        // k_zmodes_mf's image: Vt, Ut (by columns), V, U (by rows), NZP rows of NZP + 4, zero beyond nz
+        const int nzp = 16 * ((nz + 15) / 16), sp = nzp + 4;
+        std::vector<float> img((size_t)zmodes_mf_image(nz), 0.0f);
+        for (int b = 0; b < 4; ++b) {
+          const std::vector<float> &src = zb[b == 0 ? 2 : b == 1 ? 3 : b == 2 ? 0 : 1];
+          for (int r = 0; r < nz; ++r)
+            for (int k = 0; k < nz; ++k) img[((size_t)b * nzp + r) * sp + k] = src[(size_t)r * nz + k];
+        }
+        ALLOC(h->zqmf, img.size());
+        CHK(upload_vec(h, h->zqmf, img));
+      }
+      h->fold = true;
+    }
+  }
+  return 0;
+}
+
+// what only the general iteration reads: D as a palette, the folded preconditioner
+int general_setup(tdgl_handle *h) {
+  const tdgl_desc &d = h->d;
+  const int n = h->g.n;
+  h->general = true;
+  if (d.field_mode == TDGL_FIELD_PCG && !(std::getenv("TDGL_HIP_DPAL") && std::getenv("TDGL_HIP_DPAL")[0] == '0')) {
+    // D as a palette when each component takes at most DPAL_MAX values: one 32-bit code per
+    // node instead of three doubles in the PCG operator (the same values, so the same bits)
+    std::vector<double> pal((size_t)3 * DPAL_MAX, 0.0);
+    std::vector<uint32_t> code((size_t)n, 0u);
+    bool fits = true;
+    for (int c = 0; c < 3 && fits; ++c) {
+      std::vector<double> dd((size_t)n);
+      CHK(hcopy(h, dd.data(), h->D[c], (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
+      std::vector<double> vals;
+      for (size_t e = 0; e < (size_t)n && fits; ++e) {
+        auto it = std::find(vals.begin(), vals.end(), dd[e]);
+        size_t ix = (size_t)(it - vals.begin());
+        if (it == vals.end()) {
+          if (vals.size() == (size_t)DPAL_MAX) {
+            fits = false;
+            break;
+          }
+          vals.push_back(dd[e]);
+        }
+        code[e] |= (uint32_t)ix << (8 * c);
+      }
+      for (size_t k = 0; k < vals.size(); ++k) pal[(size_t)DPAL_MAX * c + k] = vals[k];
+    }
+    if (fits) {
+      ALLOC(h->Dcode, n);
+      CHK(upload_vec(h, h->Dcode, code));
+      ALLOC(h->Dpal, pal.size());
+      CHK(upload_vec(h, h->Dpal, pal));
+      ALLOC(h->Dpal32, pal.size());
+      CHK(upload_vec(h, h->Dpal32, std::vector<float>(pal.begin(), pal.end())));
+    }
+  }
+  return fold_setup(h);
+}
+
+// The solve by sectors where it applies: the Float32-preconditioned PCG with the same coefficient in every
+// direction, D constant along x and equal to its mirror images in y and z on the unknowns (what
+// link_conductivity gives, implicit.jl:126-140), at most DPAL_MAX values of D a component, and a sector that
+// fits a workgroup.  The variables that shape the general iteration select it, as TDGL_HIP_SECT=0 does.
+int sect_setup(tdgl_handle *h) {
+  const tdgl_desc &d = h->d;
+  if (d.field_mode != TDGL_FIELD_PCG || !d.pcg_f32 || d.pcg_refine) return 0;
+  const char *off = std::getenv("TDGL_HIP_SECT");
+  if (off && off[0] == '0') return 0;
+  for (const char *v : {"TDGL_HIP_BUDGET", "TDGL_HIP_FOLD", "TDGL_HIP_QPLANE", "TDGL_HIP_QPARTS", "TDGL_HIP_ZQ_WAVES", "TDGL_HIP_PLANE",
+                        "TDGL_HIP_PLANE1", "TDGL_HIP_ZCOL", "TDGL_HIP_PAPTILE", "TDGL_HIP_ZSWAP", "TDGL_HIP_DPAL", "TDGL_HIP_BOX_KC",
+                        "TDGL_HIP_BOXXCD"})
+    if (std::getenv(v)) return 0;
+  if (!(d.sxy == d.sxz && d.sxy == d.syx && d.sxy == d.syz && d.sxy == d.szx && d.sxy == d.szy && d.dx == d.dy && d.dx == d.dz)) return 0;
+  const int n[3] = {d.Nx - 1, d.Ny - 1, d.Nz - 1};
+  if (n[0] < 2 || n[1] < 3 || n[2] < 3) return 0;
+  h->sq = sect_dims(n[0], n[1], n[2]);
+  const SectDims &q = h->sq;
+  // D on the half domain (its largest extents: even nodes, odd edges) as indices into a palette
+  std::vector<double> pal((size_t)3 * DPAL_MAX, 0.0);
+  std::vector<unsigned char> code[3];
+  const double *Ds[3] = {d.Dx, d.Dy, d.Dz};
+  for (int c = 0; c < 3; ++c) {
+    const int s0 = c == 0 ? d.Nx : d.Nx + 1, s1 = c == 1 ? d.Ny : d.Ny + 1;
+    const int *e = h->rg.e[c];
+    auto at = [&](int i, int j, int k) { return Ds[c][(size_t)(i + 1) + (size_t)s0 * ((j + 1) + (size_t)s1 * (k + 1))]; };
+    const int hy = q.hy[c == 1][c == 1], hz = q.hz[c == 2][c == 2];
+    std::vector<double> vals;
+    code[c].assign((size_t)hy * hz, 0);
+    for (int k = 0; k < e[2]; ++k)
+      for (int j = 0; j < e[1]; ++j) {
+        const double v = at(0, j, k);
+        for (int i = 1; i < e[0]; ++i)
+          if (at(i, j, k) != v) return 0;
+        if (at(0, e[1] - 1 - j, k) != v || at(0, j, e[2] - 1 - k) != v) return 0;
+        if (j >= hy || k >= hz) continue;
+        size_t ix = (size_t)(std::find(vals.begin(), vals.end(), v) - vals.begin());
+        if (ix == vals.size()) {
+          if (vals.size() == (size_t)DPAL_MAX) return 0;
+          vals.push_back(v);
+        }
+        code[c][(size_t)j + (size_t)hy * k] = (unsigned char)ix;
+      }
+    for (size_t k = 0; k < vals.size(); ++k) pal[(size_t)DPAL_MAX * c + k] = vals[k];
+  }
+  h->syp = 16 * cdiv(q.hy[0][0], 16);
+  h->szp = 16 * cdiv(q.hz[0][0], 16);
+  if (!sect_x_fits(sect_x(h, false)) || !sect_cg_fits(sect_cg(h))) return 0;
+  // the tables, in one block
+  std::vector<unsigned char> all;
+  std::vector<std::pair<void *, size_t>> tabs;
+  auto put = [&](void *where, const void *src, size_t bytes) {
+    const size_t o = (all.size() + 255) / 256 * 256;
+    all.resize(o + bytes);
+    std::memcpy(&all[o], src, bytes);
+    tabs.push_back({where, o});
+  };
+  {
+    const Bases b = make_bases(n[0]);
+    for (int w = 0; w < 2; ++w) {
+      const std::vector<double> &M = w == 0 ? b.V : b.U;
+      const int L = n[0] - w, Lh = (L + 1) / 2;
+      // the x passes pad to the tiles of the component's own extent
+      const int LP = 16 * cdiv(Lh, 16);
+      for (int par = 0; par < 2; ++par)
+        for (int t = 0; t < 2; ++t) {
+          std::vector<double> m((size_t)LP * LP, 0.0);
+          for (int i = 0; i < Lh; ++i)
+            for (int cc = 0; cc < Lh; ++cc) {
+              const int col = 2 * cc + par;
+              if (col >= L) continue;
+              const double v = M[i + (size_t)L * col];
+              m[t == 0 ? (size_t)cc * LP + i : (size_t)i * LP + cc] = v;
+            }
+          put(&h->sxB[w][par][t], m.data(), m.size() * sizeof(double));
+        }
+    }
+  }
+  for (int ax = 1; ax < 3; ++ax) {
+    const int nn = n[ax], np = ax == 1 ? h->syp : h->szp;
+    const int(*hh)[2] = ax == 1 ? q.hy : q.hz;
+    const Bases b = make_bases(nn);
+    for (int par = 0; par < 2; ++par)
+      for (int w = 0; w < 2; ++w) {
+        std::vector<float> f((size_t)np * np, 0.0f), g((size_t)np * np, 0.0f);
+        for (int m = 0; 2 * m + par < nn; ++m) {
+          const int k = 2 * m + par;  // the wave number; edges: its column k - 1 (none for 0)
+          if (w == 1 && k == 0) continue;
+          for (int j = 0; j < hh[w][par]; ++j) {
+            const double v = w == 0 ? b.V[j + (size_t)nn * k] : b.U[j + (size_t)(nn - 1) * (k - 1)];
+            const bool centre = w == 0 ? (nn % 2 == 1 && par == 0 && j == hh[0][0] - 1) : (nn % 2 == 0 && par == 1 && j == hh[1][1] - 1);
+            f[(size_t)m * np + j] = (float)(centre ? v : 2.0 * v);
+            g[(size_t)j * np + m] = (float)v;
+          }
+        }
+        float **dst = ax == 1 ? h->syb[par][w] : h->szb[par][w];
+        put(&dst[0], f.data(), f.size() * sizeof(float));
+        put(&dst[1], g.data(), g.size() * sizeof(float));
+      }
+  }
+  for (int c = 0; c < 3; ++c) put(&h->scode[c], code[c].data(), code[c].size());
+  put(&h->spal, pal.data(), pal.size() * sizeof(double));
+  unsigned char *dev = nullptr;
+  ALLOC(dev, all.size());
+  CHK(upload_vec(h, dev, all));
+  for (const auto &t : tabs) *(void **)t.first = dev + t.second;
+  h->sect = true;
+  return 0;
 }
 
 }  // namespace
@@ -2323,7 +2673,9 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
       for (int c = 0; c < 3; ++c) ALLOC(h->B.c[c], n);
       // T1 and T2 also hold the FP64 quarters (a little more than the region: ceil halves)
       int qe[12][3];
-      h->t12cap = std::max((size_t)rg.total, (size_t)quarters_of(rg, qe).total);
+      // and the sectors
+      h->t12cap = std::max({(size_t)rg.total, (size_t)quarters_of(rg, qe).total,
+                            (size_t)sect_dims(d.Nx - 1, d.Ny - 1, d.Nz - 1).total});
       ALLOC(h->T1, h->t12cap);
       ALLOC(h->T2, h->t12cap);
     }
@@ -2479,83 +2831,6 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
       h->plane32 = plane_fits<float>(rg.e, 3);
       h->plane64 = plane_fits<double>(rg.e, 3);
     }
-    // the parity-folded Float32 preconditioner (TDGL_HIP_FOLD=0: the full-length transforms)
-    const char *gf = std::getenv("TDGL_HIP_FOLD");
-    if (d.field_mode == TDGL_FIELD_PCG && d.pcg_f32 && !(gf && gf[0] == '0') && !(gp && gp[0] == '0') &&
-        d.Nz - 1 >= 2 && d.Nz - 1 <= ZQ_NZ_MAX) {
-      int qe[12][3];
-      const Quarters q = quarters_of(rg, qe);
-      if (plane_fits<float>(qe, 12) && fold_blocks(q) <= MAX_PART) {
-        h->q = q;
-        ALLOC(h->qa, q.total);
-        ALLOC(h->qb, q.total);
-        const int nn[2] = {d.Nx - 1, d.Ny - 1};
-        for (int ax = 0; ax < 2; ++ax) {
-          const Bases b = make_bases(nn[ax]);
-          for (int which = 0; which < 2; ++which) {
-            const std::vector<double> &M = which == 0 ? b.V : b.U;
-            const int L = which == 0 ? nn[ax] : nn[ax] - 1, Lh = (L + 1) / 2;
-            for (int par = 0; par < 2; ++par) {
-              // the columns of parity `par` on the first ceil(L/2) rows: Mh(i, cc) = M(i, 2 cc + par)
-              std::vector<float> hf((size_t)Lh * Lh, 0.0f), hi((size_t)Lh * Lh, 0.0f);
-              for (int i = 0; i < Lh; ++i)
-                for (int cc = 0; cc < Lh; ++cc) {
-                  const int col = 2 * cc + par;
-                  const float v = col < L ? (float)M[i + (size_t)L * col] : 0.0f;
-                  hf[(size_t)i * Lh + cc] = v;  // Mh(i, cc)
-                  hi[(size_t)cc * Lh + i] = v;  // Hi[q][m] = Mh(m, q)
-                }
-              ALLOC(h->Hq[ax][which][par][0], hf.size());
-              CHK(upload_vec(h, h->Hq[ax][which][par][0], hf));
-              ALLOC(h->Hq[ax][which][par][1], hi.size());
-              CHK(upload_vec(h, h->Hq[ax][which][par][1], hi));
-              // the same, zero-padded to whole 16 x 16 tiles (k_qplane)
-              const int LP = 16 * cdiv(Lh, 16);
-              for (int t = 0; t < 2; ++t) {
-                const std::vector<float> &src = t == 0 ? hf : hi;
-                std::vector<float> pd((size_t)LP * LP, 0.0f);
-                for (int r = 0; r < Lh; ++r)
-                  for (int c = 0; c < Lh; ++c) pd[(size_t)r * LP + c] = src[(size_t)r * Lh + c];
-                ALLOC(h->Hp[ax][which][par][t], pd.size());
-                CHK(upload_vec(h, h->Hp[ax][which][par][t], pd));
-              }
-              h->HpL[ax][which] = Lh;
-            }
-          }
-        }
-        {
-          // the z pass's padded bases: V(n, mz), and U(n, mz - 1) with its zero column and row
-          const int nz = d.Nz - 1, Lu = nz - 1;
-          const Bases b = make_bases(nz);
-          std::vector<float> zb[4];
-          for (int k = 0; k < 4; ++k) zb[k].assign((size_t)nz * nz + ZQ_SLACK, 0.0f);
-          for (int n = 0; n < nz; ++n)
-            for (int mz = 0; mz < nz; ++mz) {
-              const float v = (float)b.V[n + (size_t)nz * mz];
-              const float u = (mz >= 1 && n < Lu) ? (float)b.U[n + (size_t)Lu * (mz - 1)] : 0.0f;
-              zb[0][(size_t)n * nz + mz] = v;
-              zb[1][(size_t)n * nz + mz] = u;
-              zb[2][(size_t)mz * nz + n] = v;
-              zb[3][(size_t)mz * nz + n] = u;
-            }
-          for (int k = 0; k < 4; ++k) {
-            ALLOC(h->zqb[k], zb[k].size());
-            CHK(upload_vec(h, h->zqb[k], zb[k]));
-          }
-          // k_zmodes_mf's image: Vt, Ut (by columns), V, U (by rows), NZP rows of NZP + 4, zero beyond nz
-          const int nzp = 16 * ((nz + 15) / 16), sp = nzp + 4;
-          std::vector<float> img((size_t)zmodes_mf_image(nz), 0.0f);
-          for (int b = 0; b < 4; ++b) {
-            const std::vector<float> &src = zb[b == 0 ? 2 : b == 1 ? 3 : b == 2 ? 0 : 1];
-            for (int r = 0; r < nz; ++r)
-              for (int k = 0; k < nz; ++k) img[((size_t)b * nzp + r) * sp + k] = src[(size_t)r * nz + k];
-          }
-          ALLOC(h->zqmf, img.size());
-          CHK(upload_vec(h, h->zqmf, img));
-        }
-        h->fold = true;
-      }
-    }
     // the parity-folded FP64 separable solve (TDGL_HIP_FOLD64=0: the full-length transforms)
     // the folds by default where the full-length FP64 planes are too large for the one-round
     // kernel (wider than 160 x 96: they would fall to the vector ALUs); on smaller planes the two
@@ -2628,39 +2903,9 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
         h->fold64 = true;
       }
     }
-    if (d.field_mode == TDGL_FIELD_PCG && !(std::getenv("TDGL_HIP_DPAL") && std::getenv("TDGL_HIP_DPAL")[0] == '0')) {
-      // D as a palette when each component takes at most DPAL_MAX values: one 32-bit code per
-      // node instead of three doubles in the PCG operator (the same values, so the same bits)
-      std::vector<double> pal((size_t)3 * DPAL_MAX, 0.0);
-      std::vector<uint32_t> code((size_t)n, 0u);
-      bool fits = true;
-      for (int c = 0; c < 3 && fits; ++c) {
-        std::vector<double> dd((size_t)n);
-        CHK(hcopy(h, dd.data(), h->D[c], (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-        std::vector<double> vals;
-        for (size_t e = 0; e < (size_t)n && fits; ++e) {
-          auto it = std::find(vals.begin(), vals.end(), dd[e]);
-          size_t ix = (size_t)(it - vals.begin());
-          if (it == vals.end()) {
-            if (vals.size() == (size_t)DPAL_MAX) {
-              fits = false;
-              break;
-            }
-            vals.push_back(dd[e]);
-          }
-          code[e] |= (uint32_t)ix << (8 * c);
-        }
-        for (size_t k = 0; k < vals.size(); ++k) pal[(size_t)DPAL_MAX * c + k] = vals[k];
-      }
-      if (fits) {
-        ALLOC(h->Dcode, n);
-        CHK(upload_vec(h, h->Dcode, code));
-        ALLOC(h->Dpal, pal.size());
-        CHK(upload_vec(h, h->Dpal, pal));
-        ALLOC(h->Dpal32, pal.size());
-        CHK(upload_vec(h, h->Dpal32, std::vector<float>(pal.begin(), pal.end())));
-      }
-    }
+    CHK(sect_setup(h));
+    // a solve by sectors runs no general iteration (the tuner, which times it, sets it up then)
+    if (!h->sect) CHK(general_setup(h));
     if (d.field_mode == TDGL_FIELD_PCG && d.pcg_refine) {
       // FP64 iterative refinement around Float32 inner solves: their vectors, D in Float32
       if (!h->fold || !d.pcg_f32 || !(d.pcg_fast || d.pcg_f32))
@@ -2997,6 +3242,17 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
   HIPCHK(hipMemcpyAsync(h->hp, h->hph, 2 * sizeof(double), hipMemcpyHostToDevice, h->s));
   const HostSnap start = snap(h);
   const int last_iters = h->last_iters;
+  // the shapes are the general iteration's, also where the steps solve by sectors (which have none to choose)
+  struct SectScope {
+    tdgl_handle *h;
+    bool on;
+    ~SectScope() { h->sect = on; }
+  } sect_scope{h, h->sect};
+  h->sect = false;
+  if (!h->general) {
+    CHK(general_setup(h));
+    CHK(flush(h));
+  }
   PL(K_VEC, launch_copies(backup_list(h, true), h->s));
   // what a step rewrites before reading it but the getters return (F of every band, the normal
   // fluids' potentials) goes to the host and back
