@@ -151,6 +151,17 @@ struct FieldArgs {
 hipError_t launch_field(const Geo &g, const FieldArgs &a, hipStream_t s);
 int field_blocks(const Geo &g);
 
+// One stage of several bands, and the field pass with the first, in one launch (k_bands): all of them read
+// the state at the start of the step and none what another writes
+struct BandsArgs {
+  StageArgs st[TDGL_MAX_BANDS];
+  FieldArgs f;
+  int ns;            // bands
+  int field;         // with the field pass
+  int fb, fp, sb, sp;  // set by the launcher: blocks of the field pass and of a band, padded to whole rounds of XCDs
+};
+hipError_t launch_bands(const Geo &g, BandsArgs a, hipStream_t s);
+
 struct CurlArgs {
   const double *ph[3];
   cplx *U[3];

@@ -539,6 +539,47 @@ hipError_t launch_field(const Geo &g, const FieldArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// A stage of every band that has one and, with the first stage, the field pass: launch-bound grids pay one
+// launch (about 5 us in a captured chain) where they paid one a band and one for the field.  The field's
+// blocks come first (they are the longer ones); each part keeps its own order of blocks on the XCDs, so
+// every node's and every partial's bits are those of the separate launches.  A step: 35.2 -> 28.4 us on 12x8x4
+// cells, 76 -> 61 us with three bands on 148x60x10, 219 -> 203 us (128x64x16, KWT), 249 -> 235 us (75x41x13, open);
+// 552 -> 538 us on 256x128x32, where the launches are bound by HBM, and never slower.
+__global__ void __launch_bounds__(256) k_bands(Geo g, BandsArgs a) {
+  int b = blockIdx.x;
+  if (b < a.fp) {
+    if (b >= a.fb) return;
+    const int nx = cdiv_d(g.Nx + 1, 64), ny = cdiv_d(g.Ny + 1, 4);
+    const int l = a.f.xcd ? xcd_run(b, a.fb) : b;
+    field_body(g, a.f, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, g.Nz + 1});
+    return;
+  }
+  b -= a.fp;
+  const int q = b / a.sp;
+  b -= q * a.sp;
+  if (b >= a.sb) return;
+  const StageArgs &st = a.st[q];
+  const int nx = cdiv_d(g.x2 - g.x1, 64), ny = cdiv_d(g.y2 - g.y1, 4);
+  const int l = st.xcd ? xcd_run(b, a.sb) : b;
+  stage_body(g, st, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, g.z2 - g.z1});
+}
+static_assert(sizeof(Geo) + sizeof(BandsArgs) <= 4096, "kernel arguments");
+
+hipError_t launch_bands(const Geo &g, BandsArgs a, hipStream_t s) {
+  if (g_rec) return hipErrorNotSupported;
+  if (a.ns < 0 || a.ns > TDGL_MAX_BANDS) return hipErrorInvalidValue;
+  if (a.field && a.f.part && field_blocks(g) > MAX_PART) return hipErrorInvalidValue;
+  const int ni = g.x2 - g.x1, nj = g.y2 - g.y1, nk = g.z2 - g.z1;
+  a.fb = a.field ? field_blocks(g) : 0;
+  a.sb = (ni > 0 && nj > 0 && nk > 0) ? cdiv(ni, 64) * cdiv(nj, 4) * nk : 0;
+  a.fp = 8 * cdiv(a.fb, 8);
+  a.sp = 8 * std::max(1, cdiv(a.sb, 8));
+  const int nb = a.fp + a.ns * a.sp;
+  if (nb == 0) return hipSuccess;
+  TDGL_LAUNCH(k_bands, dim3(nb), dim3(64, 4, 1), 0, s, g, a);
+  return hipGetLastError();
+}
+
 // Links U = e^{−iφ} (links!, field.jl:105-121), field h = curl φ (curl_h!, :124-137) and the
 // field boundary (field_bc!, :189-228: applied H, slab or bar self-field; the later assignment
 // of the reference wins where two cover one element).

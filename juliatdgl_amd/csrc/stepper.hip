@@ -123,8 +123,8 @@ struct tdgl_handle {
   cplx *U[3] = {}, *V[3] = {};
   double *J[3] = {}, *h[3] = {};
   // workspace
-  cplx *W = nullptr, *W2 = nullptr;
-  double *Om = nullptr;
+  cplx *W[TDGL_MAX_BANDS] = {}, *W2[TDGL_MAX_BANDS] = {};  // per band, so that bands step side by side
+  double *Om[TDGL_MAX_BANDS] = {};   // the frame's rate, per band for the same reason
   // masks and tables
   double *f = nullptr, *tau[3] = {}, *D[3] = {};
   double *bar[6] = {};
@@ -158,6 +158,7 @@ struct tdgl_handle {
   int qplane = 1;              // TDGL_HIP_QPLANE=0: the quarter x-y transforms on k_plane_mf1 / k_plane_mf
   int qparts = 1;              // k_qplane's blocks a quarter plane (its m tiles split; TDGL_HIP_QPARTS)
   int zq_waves = 8;        // the quarter z pass: 4 or 8 waves a block on the vector ALUs, 0 on the matrix cores (k_zmodes_mf)
+  int merge = 1;           // the bands' stages and the field pass in common launches (TDGL_HIP_MERGE=0: each its own)
   int stxcd = 1;           // the stencil kernels' blocks in XCD runs (TDGL_HIP_STENCILXCD=0: the hardware's order)
   float *zqb[4] = {};      // its padded z bases (ZQ_BASES)
   float *zqmf = nullptr;   // the same as k_zmodes_mf's image (zmodes_mf_image floats)
@@ -556,7 +557,7 @@ StageArgs stage_base(tdgl_handle *h, int mu, const tdgl_bandcoef &cf) {
     a.U[c] = h->U[c];
   }
   a.f = h->f;
-  a.Om = h->Om;
+  a.Om = h->Om[mu];
   a.kx = cf.kx;
   a.ky = cf.ky;
   a.kz = cf.kz;
@@ -612,31 +613,51 @@ void stage_qp(tdgl_handle *h, StageArgs &a, int mu) {
     for (int k = 0; k < d.qp_nmodes; ++k) a.qpc[k] = d.qp_P[mu][k];
 }
 
+// The launch arguments of stage j of a band from Y_{j-2} = A and Y_{j-1} = B into C
+StageArgs rkl_stage(tdgl_handle *h, int mu, int ns, int j, const cplx *A, const cplx *B, cplx *C) {
+  const tdgl_desc &d = h->d;
+  const bool kc = d.rkc[mu] != 0;
+  const double q = kc ? d.divisor[mu] : (double)(ns * (ns + 1) / 2);
+  const bool rot = d.rotframe, ex = d.extrap;
+  StageArgs a = stage_base(h, mu, d.bcs[mu]);
+  a.D = C;
+  a.S = B;
+  a.A = A;
+  if (ex && j >= 2) {
+    // the links of the previous stage's fraction c_{j-1} (set after stage j-1, bands.jl:502-513)
+    a.lsrc = rot ? LS_ROTLINKS : LS_ROTFRAC;
+    a.lc = kc ? d.rkc_c[mu][j - 2] : (double)((j - 1) * j) / (double)(ns * (ns + 1));
+  }
+  a.ghost_fly = j >= 2;
+  a.frame = j == 1 ? frame_first(h) : frame_later(h);
+  a.h = d.dt / q;
+  if (j >= 2) {
+    a.combine = 1;
+    a.logcomb = h->noise && d.bcs[mu].gamma2 > 0;   // _logcomb (bands.jl:455)
+    a.cmu = kc ? d.rkc_mu[mu][j - 1] : (2.0 * j - 1) / j;
+    a.cnu = kc ? d.rkc_nu[mu][j - 1] : (1.0 - j) / j;
+  }
+  a.turn = rot && j == ns;
+  if (j == ns) {
+    stage_qp(h, a, mu);
+    a.noise = h->noise;
+  }
+  return a;
+}
+cplx *rkl_buf(tdgl_handle *h, int mu, int ns, int j) {
+  cplx *buf[3] = {h->F[mu], h->W[mu], h->W2[mu]};
+  return buf[(((j - ns) % 3) + 3) % 3];
+}
 // _band_rkl! (bands.jl:464-521): stage j writes buf[(j - ns) mod 3] of (F, W, W2) so that the
 // last stage lands in F and no stage writes a buffer it reads.  The links of stage j >= 2 are
 // V (V Ū)^c_j, or V _cis(R c_j) in the rotating frame, evaluated inside the stage kernel.
 int band_rkl(tdgl_handle *h, int mu, int ns) {
   const tdgl_desc &d = h->d;
-  const bool kc = d.rkc[mu] != 0;
-  const double q = kc ? d.divisor[mu] : (double)(ns * (ns + 1) / 2);
-  const double hh = d.dt / q;
-  const bool rot = d.rotframe, ex = d.extrap;
-  cplx *buf[3] = {h->F[mu], h->W, h->W2};
   const cplx *A = h->G[mu], *B = h->G[mu];
-  const bool lg = h->noise && d.bcs[mu].gamma2 > 0;   // _logcomb (bands.jl:455)
   const bool skq = h->noise && d.noise_sk[mu];         // _skrock (bands.jl:446)
   for (int j = 1; j <= ns; ++j) {
-    cplx *C = buf[(((j - ns) % 3) + 3) % 3];
-    StageArgs a = stage_base(h, mu, d.bcs[mu]);
-    a.D = C;
-    a.S = B;
-    a.A = A;
-    if (ex && j >= 2) {
-      // the links of the previous stage's fraction c_{j-1} (set after stage j-1, bands.jl:502-513)
-      a.lsrc = rot ? LS_ROTLINKS : LS_ROTFRAC;
-      a.lc = kc ? d.rkc_c[mu][j - 2] : (double)((j - 1) * j) / (double)(ns * (ns + 1));
-    }
-    a.ghost_fly = j >= 2;
+    cplx *C = rkl_buf(h, mu, ns, j);
+    StageArgs a = rkl_stage(h, mu, ns, j, A, B, C);
     if (j == 1 && skq) {
       // SK-ROCK's first stage: K₁ = E(Ψⁿ e^{iν₁δθ}) e^{i(κ₁−ν₁)δθ} (bands.jl:482-487)
       SkArgs k{};
@@ -657,19 +678,6 @@ int band_rkl(tdgl_handle *h, int mu, int ns) {
       a.sk_on = 1;
       a.sk_post = d.noise_sk_w[mu][1] - d.noise_sk_w[mu][0];
     }
-    a.frame = j == 1 ? frame_first(h) : frame_later(h);
-    a.h = hh;
-    if (j >= 2) {
-      a.combine = 1;
-      a.logcomb = lg;
-      a.cmu = kc ? d.rkc_mu[mu][j - 1] : (2.0 * j - 1) / j;
-      a.cnu = kc ? d.rkc_nu[mu][j - 1] : (1.0 - j) / j;
-    }
-    a.turn = rot && j == ns;
-    if (j == ns) {
-      stage_qp(h, a, mu);
-      a.noise = h->noise;
-    }
     CHK(stage_launch(h, a));
     A = B;
     B = C;
@@ -685,7 +693,7 @@ int band_substeps(tdgl_handle *h, int mu, int n) {
   const double hh = d.dt / n;
   const cplx *src = h->G[mu];
   for (int m = 1; m <= n; ++m) {
-    cplx *dst = ((n - m) % 2 == 0) ? h->F[mu] : h->W;
+    cplx *dst = ((n - m) % 2 == 0) ? h->F[mu] : h->W[mu];
     StageArgs a = stage_base(h, mu, d.bcs[mu]);
     a.D = dst;
     a.S = src;
@@ -709,6 +717,63 @@ int band_substeps(tdgl_handle *h, int mu, int n) {
   return 0;
 }
 
+// the one Euler step of a band without substeps
+StageArgs euler_stage(tdgl_handle *h, int mu) {
+  const tdgl_desc &d = h->d;
+  StageArgs a = stage_base(h, mu, d.bc[mu]);
+  a.D = h->F[mu];
+  a.S = h->G[mu];
+  a.frame = frame_first(h);
+  a.h = d.dt;
+  a.turn = d.rotframe;
+  stage_qp(h, a, mu);
+  a.noise = h->noise;
+  return a;
+}
+
+// Whether the bands' stages and the field pass go into common launches: Euler steps and stages without SK-ROCK's
+// source or the low-pass sweeps of a noisy frame (which put other launches between them), launched by themselves
+// (not recorded for a batch, not timed one by one)
+bool bands_merge(const tdgl_handle *h) {
+  const tdgl_desc &d = h->d;
+  if (g_rec || h->prof || !h->merge || frame_first(h) == FRAME_RAW) return false;
+  for (int mu = 0; mu < d.nbands; ++mu) {
+    if (h->noise && d.noise_sk[mu]) return false;
+    if (d.stages[mu] == 0 && d.nsub[mu] != 1) return false;
+  }
+  return true;
+}
+
+// update_bands! (bands.jl:330-346) of all bands side by side, stage after stage, the field pass with the first
+int update_bands_merged(tdgl_handle *h, const FieldArgs &fa) {
+  const tdgl_desc &d = h->d;
+  const cplx *A[TDGL_MAX_BANDS], *B[TDGL_MAX_BANDS];
+  int smax = 1;
+  for (int mu = 0; mu < d.nbands; ++mu) {
+    A[mu] = B[mu] = h->G[mu];
+    smax = std::max(smax, d.stages[mu]);
+  }
+  for (int j = 1; j <= smax; ++j) {
+    BandsArgs ba{};
+    ba.field = j == 1;
+    if (j == 1) ba.f = fa;
+    for (int mu = 0; mu < d.nbands; ++mu) {
+      const int ns = d.stages[mu];
+      if (j > std::max(1, ns)) continue;
+      if (ns == 0) {
+        ba.st[ba.ns++] = euler_stage(h, mu);
+        continue;
+      }
+      cplx *C = rkl_buf(h, mu, ns, j);
+      ba.st[ba.ns++] = rkl_stage(h, mu, ns, j, A[mu], B[mu], C);
+      A[mu] = B[mu];
+      B[mu] = C;
+    }
+    LCHK(launch_bands(h->g, ba, h->s));
+  }
+  return 0;
+}
+
 // update_bands! (bands.jl:330-346)
 int update_bands(tdgl_handle *h) {
   const tdgl_desc &d = h->d;
@@ -716,15 +781,7 @@ int update_bands(tdgl_handle *h) {
     if (d.stages[mu] > 0) {
       CHK(band_rkl(h, mu, d.stages[mu]));
     } else if (d.nsub[mu] == 1) {
-      StageArgs a = stage_base(h, mu, d.bc[mu]);
-      a.D = h->F[mu];
-      a.S = h->G[mu];
-      a.frame = frame_first(h);
-      a.h = d.dt;
-      a.turn = d.rotframe;
-      stage_qp(h, a, mu);
-      a.noise = h->noise;
-      CHK(stage_launch(h, a));
+      CHK(stage_launch(h, euler_stage(h, mu)));
     } else {
       CHK(band_substeps(h, mu, d.nsub[mu]));
     }
@@ -1850,7 +1907,8 @@ int step_once(tdgl_handle *h) {
   const tdgl_desc &d = h->d;
   if (d.selffield_bc == TDGL_BC_OPEN) CHK(open_update(h));
   if (d.qp_mode != TDGL_QP_NONE) CHK(qp_potential(h));
-  CHK(update_bands(h));
+  const bool merge = bands_merge(h);
+  if (!merge) CHK(update_bands(h));
   FieldArgs fa{};
   fa.xcd = h->stxcd;
   for (int mu = 0; mu < d.nbands; ++mu) fa.G[mu] = h->G[mu];
@@ -1887,7 +1945,10 @@ int step_once(tdgl_handle *h) {
     fa.kaz = c * d.dz;
     fa.nz = noise_args(h);
   }
-  PL(K_FIELD, launch_field(h->g, fa, h->s));
+  if (merge)
+    CHK(update_bands_merged(h, fa));
+  else
+    PL(K_FIELD, launch_field(h->g, fa, h->s));
   if (d.field_mode == TDGL_FIELD_SEPARABLE) {
     SepOut o{nullptr, true, 0};
     CHK(sep_solve(h, h->B, o, nullptr, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
@@ -2602,14 +2663,18 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
       ALLOC(h->tau[c], n);
     }
     ALLOC(h->f, n);
-    bool stages = false, subs = false;
+    // the bands on substeps one after the other share the first one's
     for (int mu = 0; mu < d.nbands; ++mu) {
-      stages |= d.stages[mu] > 0;
-      subs |= d.stages[mu] == 0 && d.nsub[mu] > 1;
+      if (d.stages[mu] > 0) {
+        ALLOC(h->W[mu], n);
+        ALLOC(h->W2[mu], n);
+      } else if (d.nsub[mu] > 1) {
+        for (int nu = 0; nu < mu && !h->W[mu]; ++nu) h->W[mu] = h->W[nu];
+        if (!h->W[mu]) ALLOC(h->W[mu], n);
+      }
     }
-    if (stages || subs) ALLOC(h->W, n);
-    if (stages) ALLOC(h->W2, n);
-    if (d.rotframe) ALLOC(h->Om, n);
+    if (d.rotframe)
+      for (int mu = 0; mu < d.nbands; ++mu) ALLOC(h->Om[mu], n);
     h->noise = d.noise != 0;
     if (h->noise) {
       ALLOC(h->nctr, 2);
@@ -2819,6 +2884,8 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
     if (qs && qs[0] >= '1' && qs[0] <= '3' && !qs[1]) h->qparts = qs[0] - '0';
     // TDGL_HIP_ZQ_WAVES=4 or 8: the quarter z pass on the vector ALUs with that many waves a block
     // (8 by default), 0: on the matrix cores
+    const char *mg = std::getenv("TDGL_HIP_MERGE");
+    h->merge = mg && mg[0] == '0' ? 0 : 1;
     const char *sx = std::getenv("TDGL_HIP_STENCILXCD");
     h->stxcd = sx && sx[0] == '0' ? 0 : 1;
     const char *zw = std::getenv("TDGL_HIP_ZQ_WAVES");
