@@ -40,17 +40,24 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 // Bound: 2 (Lx / 2) flop in FP64 per element on the matrix cores (the fold along x halves the dense
 // product) against 16 B.  A block takes SX_J positions along y at one z and their mirror images, folds
 // them into the four sectors and the two x parities in LDS and multiplies by the half-size x bases
-// (padded to whole 16 x 16 tiles, read through L2); wave w owns the m tiles w, w + waves, ...
-constexpr int SX_J = 8, SX_COLS = 4 * SX_J;
-constexpr int SX_WAVES = 16;
+// (padded to whole 16 x 16 tiles, read through L2); wave w owns the m tiles w, w + waves, ...  What it waits
+// for is memory: the loads of the images (sixteen in flight a thread), of the bases (three groups ahead) and,
+// on the way back, of θ and x (an image set together: one after the other behind the stores they took 31 us
+// more).  Forward 72 us, back 109 us on 272 x 144 x 48 nodes (104 us each at first; 88 and 217 MB), 12 and 16 us on
+// 100 x 52 x 28.  Four positions a block (half the LDS) took 92 to 102 and 116 to 131 us, 5 to 8 waves no less.
+constexpr int SX_J = 8, SX_COLS = 4 * SX_J, SX_T = SX_COLS / 16;
+constexpr int SX_WAVES = 10;
 
 __device__ __forceinline__ int sx_stride(int qs) { return qs + 2; }  // LDS rows of 4 (mod 8) words
 
 struct SxIdx {
   int c, k, j0;
 };
-__device__ __forceinline__ SxIdx sx_idx(const SectX &p, int b) {
-  const int per = p.jg * p.kg;
+// Blocks in contiguous runs of (j group, k, component) on each XCD (the hardware deals them to the eight in
+// turn): neighbours along j share the lines of a sector's rows, which one L2 then merges
+__device__ __forceinline__ SxIdx sx_idx(const SectX &p, int hw) {
+  const int per = p.jg * p.kg, nb = 3 * per, x = hw & 7, bq = nb >> 3, br = nb & 7;
+  const int b = (x < br ? x * (bq + 1) : br * (bq + 1) + (x - br) * bq) + (hw >> 3);
   SxIdx r;
   r.c = b / per;
   const int q = b - r.c * per;
@@ -71,33 +78,41 @@ __device__ __forceinline__ void sect_fwd_body(const SectX &p, int b) {
   const View v = p.v[c];
   const double *base = (const double *)v.p;
   const int ks = L2 - 1 - k;
-  for (int t = tid; t < QS * SX_J; t += nth) {
-    const int i = t % QS, jj = t / QS, j = j0 + jj;
-    double f[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-    if (i < hx && j < hy) {
-      const int is = L0 - 1 - i, js = L1 - 1 - j;
-      const double *r00 = base + (size_t)v.s1 * j + (size_t)v.s2 * k, *r10 = base + (size_t)v.s1 * js + (size_t)v.s2 * k;
-      const double *r01 = base + (size_t)v.s1 * j + (size_t)v.s2 * ks, *r11 = base + (size_t)v.s1 * js + (size_t)v.s2 * ks;
-      const double a[2][4] = {{r00[i], r10[i], r01[i], r11[i]}, {r00[is], r10[is], r01[is], r11[is]}};
+  // two items a thread at a time, their sixteen loads in flight together
+  for (int t0 = tid; t0 < QS * SX_J; t0 += 2 * nth) {
+    double a[2][2][4];
+    bool ok[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int t = t0 + u * nth, i = t % QS, j = j0 + t / QS;
+      ok[u] = t < QS * SX_J && i < hx && j < hy;
+      const int ic = ok[u] ? i : 0, jc = ok[u] ? j : j0, is = L0 - 1 - ic, js = L1 - 1 - jc;
+      const double *r00 = base + (size_t)v.s1 * jc + (size_t)v.s2 * k, *r10 = base + (size_t)v.s1 * js + (size_t)v.s2 * k;
+      const double *r01 = base + (size_t)v.s1 * jc + (size_t)v.s2 * ks, *r11 = base + (size_t)v.s1 * js + (size_t)v.s2 * ks;
+      a[u][0][0] = r00[ic], a[u][0][1] = r10[ic], a[u][0][2] = r01[ic], a[u][0][3] = r11[ic];
+      a[u][1][0] = r00[is], a[u][1][1] = r10[is], a[u][1][2] = r01[is], a[u][1][3] = r11[is];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int t = t0 + u * nth, i = t % QS, jj = t / QS;
+      if (t >= QS * SX_J) continue;
       double s[2][4];
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        const double e0 = a[x][0] + a[x][1], o0 = a[x][0] - a[x][1], e1 = a[x][2] + a[x][3], o1 = a[x][2] - a[x][3];
+        const double e0 = a[u][x][0] + a[u][x][1], o0 = a[u][x][0] - a[u][x][1], e1 = a[u][x][2] + a[u][x][3],
+                     o1 = a[u][x][2] - a[u][x][3];
         s[x][0] = 0.25 * (e0 + e1);  // y even, z even
         s[x][1] = 0.25 * (e0 - e1);  // y even, z odd
         s[x][2] = 0.25 * (o0 + o1);  // y odd, z even
         s[x][3] = 0.25 * (o0 - o1);
       }
+      const bool ci = L0 - 1 - i == i;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        f[0][q] = is == i ? s[0][q] : s[0][q] + s[1][q];
-        f[1][q] = is == i ? 0.0 : s[0][q] - s[1][q];
+        F[(q * SX_J + jj) * IS + i] = !ok[u] ? 0.0 : (ci ? s[0][q] : s[0][q] + s[1][q]);
+        F[(SX_COLS + q * SX_J + jj) * IS + i] = (!ok[u] || ci) ? 0.0 : s[0][q] - s[1][q];
       }
     }
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) F[(x * SX_COLS + q * SX_J + jj) * IS + i] = f[x][q];
   }
   __syncthreads();
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
@@ -105,23 +120,29 @@ __device__ __forceinline__ void sect_fwd_body(const SectX &p, int b) {
   for (int m = w; m < mt; m += nw)
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
-      v4d acc[2] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}};
-      const double *A = p.B[wx][x] + (size_t)(16 * m + lr) * QS + 4 * lk;
-      const double *B0 = F + (x * SX_COLS + lr) * IS + 4 * lk, *B1 = B0 + 16 * IS;
-      v4d a = ld4d(A);
-      for (int g = 0; g < mt; ++g) {
-        const v4d an = ld4d(A + 16 * min(g + 1, mt - 1));
-        const v4d b0 = ld4d(B0 + 16 * g), b1 = ld4d(B1 + 16 * g);
+      v4d acc[SX_T];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b0[u], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b1[u], acc[1], 0, 0, 0);
-        }
+      for (int t = 0; t < SX_T; ++t) acc[t] = v4d{0, 0, 0, 0};
+      const double *A = p.B[wx][x] + (size_t)(16 * m + lr) * QS + 4 * lk;
+      const double *B0 = F + (x * SX_COLS + lr) * IS + 4 * lk;
+      // the bases come from L2: three groups ahead, an MFMA group takes 512 cycles of its SIMD
+      v4d a = ld4d(A), an = ld4d(A + 16 * min(1, mt - 1)), a2 = ld4d(A + 16 * min(2, mt - 1));
+      for (int g = 0; g < mt; ++g) {
+        const v4d a3 = ld4d(A + 16 * min(g + 3, mt - 1));
+        v4d b[SX_T];
+#pragma unroll
+        for (int t = 0; t < SX_T; ++t) b[t] = ld4d(B0 + 16 * t * IS + 16 * g);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int t = 0; t < SX_T; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[t][u], acc[t], 0, 0, 0);
         a = an;
+        an = a2;
+        a2 = a3;
       }
       // element r of lane l: mode 2 (16 m + 4 r + lk) + x of the column's sector and position
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < SX_T; ++t) {
         const int col = 16 * t + lr, q = col / SX_J, j = j0 + col % SX_J;
         const int py = (q >> 1) ^ (c == 1 ? 1 : 0), pz = (q & 1) ^ (c == 2 ? 1 : 0), s = 2 * py + pz;
         const int ly = p.q.hy[c == 1 ? 1 : 0][py], lz = p.q.hz[c == 2 ? 1 : 0][pz];
@@ -137,7 +158,7 @@ __device__ __forceinline__ void sect_fwd_body(const SectX &p, int b) {
 }
 
 // r to the sectors; block 0 also leaves ||r||² (the partials of the residual kernel) in SC_RR
-__global__ void __launch_bounds__(64 * SX_WAVES) k_sect_fwd(SectX p) {
+__global__ void __launch_bounds__(64 * SX_WAVES, 5) k_sect_fwd(SectX p) {
   if (p.gate && !*p.gate) return;
   if (blockIdx.x == 0 && p.nparts > 0) {
     __shared__ double sh[SX_WAVES];
@@ -179,69 +200,90 @@ __device__ __forceinline__ void sect_inv_body(const SectX &p, int b, bool act) {
   const int mt = (hx + 15) / 16, QS = 16 * mt, IS = sx_stride(QS);
   const int wx = c == 0 ? 1 : 0;
   if (act) {
-    for (int t = tid; t < 2 * QS * SX_COLS; t += nth) {
-      const int jj = t % SX_J, q = (t / SX_J) % 4, mode = t / SX_COLS, j = j0 + jj;
-      const int py = (q >> 1) ^ (c == 1 ? 1 : 0), pz = (q & 1) ^ (c == 2 ? 1 : 0), s = 2 * py + pz;
-      const int ly = p.q.hy[c == 1 ? 1 : 0][py], lz = p.q.hz[c == 2 ? 1 : 0][pz];
-      double v = 0.0;
-      if (mode < L0 && j < ly && k < lz) v = p.S[p.q.off[s] + (size_t)(mode + wx) * p.q.size[s] + p.q.oc[c][s] + j + (size_t)ly * k];
-      F[((mode & 1) * SX_COLS + 16 * (jj >> 2) + 4 * q + (jj & 3)) * IS + (mode >> 1)] = v;
+    // a thread keeps its position and sector and steps through the modes (nth is a multiple of 32), eight loads
+    // in flight
+    const int jj = tid % SX_J, q = (tid / SX_J) % 4, j = j0 + jj, dm = nth / SX_COLS;
+    const int py = (q >> 1) ^ (c == 1 ? 1 : 0), pz = (q & 1) ^ (c == 2 ? 1 : 0), s = 2 * py + pz;
+    const int ly = p.q.hy[c == 1 ? 1 : 0][py], lz = p.q.hz[c == 2 ? 1 : 0][pz];
+    const bool in = j < ly && k < lz;
+    const size_t ms = (size_t)p.q.size[s];
+    const double *src = p.S + p.q.off[s] + (size_t)wx * ms + p.q.oc[c][s] + (in ? (size_t)j + (size_t)ly * k : 0);
+    double *dst = F + (16 * (jj >> 2) + 4 * q + (jj & 3)) * IS;
+    for (int m0 = tid / SX_COLS; m0 < 2 * QS; m0 += 8 * dm) {
+      double f[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) f[u] = src[(size_t)min(m0 + u * dm, L0 - 1) * ms];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int mode = m0 + u * dm;
+        if (mode < 2 * QS) dst[(mode & 1) * SX_COLS * IS + (mode >> 1)] = (in && mode < L0) ? f[u] : 0.0;
+      }
     }
     __syncthreads();
   }
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6, l = tid & 63, lr = l & 15, lk = l >> 4;
   const View vo = p.v[c], vt = p.th[c], vx = p.x[c];
   for (int m = w; m < mt; m += nw) {
-    v4d acc[2][2];
+    v4d acc[2][SX_T];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) acc[x][t] = v4d{0, 0, 0, 0};
+      for (int t = 0; t < SX_T; ++t) acc[x][t] = v4d{0, 0, 0, 0};
     if (act)
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         const double *B = p.B[wx][x] + (size_t)(16 * m + lr) * QS + 4 * lk;
-        const double *A0 = F + (x * SX_COLS + lr) * IS + 4 * lk, *A1 = A0 + 16 * IS;
-        v4d bb = ld4d(B);
+        const double *A0 = F + (x * SX_COLS + lr) * IS + 4 * lk;
+        v4d bb = ld4d(B), bn = ld4d(B + 16 * min(1, mt - 1)), b2 = ld4d(B + 16 * min(2, mt - 1));
         for (int g = 0; g < mt; ++g) {
-          const v4d bn = ld4d(B + 16 * min(g + 1, mt - 1));
-          const v4d a0 = ld4d(A0 + 16 * g), a1 = ld4d(A1 + 16 * g);
+          const v4d b3 = ld4d(B + 16 * min(g + 3, mt - 1));
+          v4d a[SX_T];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            acc[x][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[u], bb[u], acc[x][0], 0, 0, 0);
-            acc[x][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[u], bb[u], acc[x][1], 0, 0, 0);
-          }
+          for (int t = 0; t < SX_T; ++t) a[t] = ld4d(A0 + 16 * t * IS + 16 * g);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int t = 0; t < SX_T; ++t)
+              acc[x][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][u], bb[u], acc[x][t], 0, 0, 0);
           bb = bn;
+          bn = b2;
+          b2 = b3;
         }
       }
     const int i = 16 * m + lr, is = L0 - 1 - i, ks = L2 - 1 - k;
     if (i >= hx) continue;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < SX_T; ++t) {
       const int j = j0 + 4 * t + lk, js = L1 - 1 - j;
       if (j >= hy) continue;
 #pragma unroll
       for (int xi = 0; xi < 2; ++xi) {
         if (xi && is == i) continue;
+        const int ii = xi ? is : i;
+        // the operands of the four images together (a centre row's or plane's image is itself), then the stores
+        double tv[4], xv[4];
+#pragma unroll
+        for (int im = 0; im < 4; ++im) {
+          const int jj = (im & 1) ? js : j, kk = (im & 2) ? ks : k;
+          tv[im] = ((const double *)vt.p)[(size_t)ii + (size_t)vt.s1 * jj + (size_t)vt.s2 * kk];
+          xv[im] = PCG ? ((const double *)vx.p)[(size_t)ii + (size_t)vx.s1 * jj + (size_t)vx.s2 * kk] : 0.0;
+        }
         double s[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) s[q] = xi ? acc[0][t][q] - acc[1][t][q] : acc[0][t][q] + acc[1][t][q];
         const double e = s[0] + s[2], o = s[0] - s[2], e1 = s[1] + s[3], o1 = s[1] - s[3];
         const double val[4] = {e + e1, o + o1, e - e1, o - o1};  // (j, k), (js, k), (j, ks), (js, ks)
-        const int ii = xi ? is : i;
 #pragma unroll
         for (int im = 0; im < 4; ++im) {
           if (((im & 1) && js == j) || ((im & 2) && ks == k)) continue;
           const int jj = (im & 1) ? js : j, kk = (im & 2) ? ks : k;
           const size_t oo = (size_t)ii + (size_t)vo.s1 * jj + (size_t)vo.s2 * kk;
-          const size_t ot = (size_t)ii + (size_t)vt.s1 * jj + (size_t)vt.s2 * kk;
           if (PCG) {
-            const size_t ox = (size_t)ii + (size_t)vx.s1 * jj + (size_t)vx.s2 * kk;
-            const double xn = ((double *)vx.p)[ox] + val[im];
-            if (act) ((double *)vx.p)[ox] = xn;
-            ((double *)vo.p)[oo] = ((const double *)vt.p)[ot] + xn;
+            const double xn = xv[im] + val[im];
+            if (act) ((double *)vx.p)[(size_t)ii + (size_t)vx.s1 * jj + (size_t)vx.s2 * kk] = xn;
+            ((double *)vo.p)[oo] = tv[im] + xn;
           } else {
-            ((double *)vo.p)[oo] = ((const double *)vt.p)[ot] + val[im];
+            ((double *)vo.p)[oo] = tv[im] + val[im];
           }
         }
       }
@@ -249,7 +291,7 @@ __device__ __forceinline__ void sect_inv_body(const SectX &p, int b, bool act) {
   }
 }
 
-__global__ void __launch_bounds__(64 * SX_WAVES) k_sect_inv(SectX p) {
+__global__ void __launch_bounds__(64 * SX_WAVES, 5) k_sect_inv(SectX p) {
   const bool act = sect_active(p.d);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     int *fl = p.d.fl;
