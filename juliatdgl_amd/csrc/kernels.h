@@ -470,10 +470,10 @@ struct FftPass {
   int lines_fast;          // consecutive threads over lines (a line's elements are far apart)
   const double *ghat;
   long long g_s, g_l0, g_l1;
-  int lpb;                 // set by the launcher
+  int lpb;                 // log2 of the lines of a block, set by the launcher
   FftAxis ax;
 };
-hipError_t launch_fft(FftPass p, const int *gate, hipStream_t s);
+hipError_t launch_fft(const FftPass *p, int n, const int *gate, hipStream_t s);  // n <= 3 lattices
 
 struct OpenGreen {         // fac·G on the padded box M0 x M1 x M2 (real)
   double *out;

@@ -70,18 +70,19 @@ hipError_t launch_open_dj(const Geo &g, const OpenDJ &a, hipStream_t s) {
 __device__ __forceinline__ cplx imul_s(cplx v, int s) { return s > 0 ? mk(-v.y, v.x) : mk(v.y, -v.x); }  // (s i) v
 
 // the R-point DFT with exponent sign s, in place
-__device__ __forceinline__ void dft_small(cplx *v, int R, int s) {
-  if (R == 2) {
+template <int R>
+__device__ __forceinline__ void dft_small(cplx (&v)[R], int s) {
+  if constexpr (R == 2) {
     const cplx a = v[0], b = v[1];
     v[0] = cadd(a, b);
     v[1] = csub(a, b);
-  } else if (R == 4) {
+  } else if constexpr (R == 4) {
     const cplx t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]), t2 = cadd(v[1], v[3]), t3 = imul_s(csub(v[1], v[3]), s);
     v[0] = cadd(t0, t2);
     v[1] = cadd(t1, t3);
     v[2] = csub(t0, t2);
     v[3] = csub(t1, t3);
-  } else if (R == 3) {
+  } else if constexpr (R == 3) {
     const double h3 = 0.86602540378443864676;  // √3/2
     const cplx t1 = cadd(v[1], v[2]), t2 = imul_s(rmul(h3, csub(v[1], v[2])), s);
     const cplx m = csub(v[0], rmul(0.5, t1));
@@ -104,105 +105,133 @@ __device__ __forceinline__ void dft_small(cplx *v, int R, int s) {
   }
 }
 
-// Stockham autosort passes over `lines` lines of length M in LDS; returns the buffer holding the
-// result (natural order).  Pass with radix R: butterfly j reads src[j + r M/R], twiddles r by
-// ω^(r (j mod Ns) M/(Ns R)), writes dst[(j/Ns) Ns R + (j mod Ns) + r Ns].
-__device__ cplx *fft_lines(cplx *A, cplx *B, int lines, const FftAxis &ax, int dir) {
-  const int M = ax.M;
-  cplx *src = A, *dst = B;
-  int Ns = 1;
-  for (int s = 0; s < ax.nrad; ++s) {
-    const int R = ax.rad[s], MR = M / R, step = M / (Ns * R);
-    for (int item = threadIdx.x; item < lines * MR; item += blockDim.x) {
-      const int l = item / MR, j = item % MR, k = j % Ns;
-      const cplx *S = src + l * M;
-      cplx *D = dst + l * M;
-      cplx v[5];
-      for (int r = 0; r < R; ++r) v[r] = S[j + r * MR];
-      for (int r = 1; r < R; ++r) {
-        cplx w = ax.tw[r * k * step];
-        if (dir > 0) w.y = -w.y;
-        v[r] = cmul(v[r], w);
-      }
-      dft_small(v, R, dir);
-      const int base = (j / Ns) * Ns * R + k;
-      for (int r = 0; r < R; ++r) D[base + r * Ns] = v[r];
-    }
-    __syncthreads();
-    cplx *t = src;
-    src = dst;
-    dst = t;
-    Ns *= R;
-  }
-  return src;
-}
+// The lines of a block lie interleaved in LDS, element e of line l at A[e LPB + l] with LPB a power of two:
+// a thread keeps its line, consecutive lanes take consecutive lines of the same butterfly (no division by a
+// length, no bank conflict, one twiddle for LPB lanes).
+constexpr int FFT_T = 256;      // threads
+constexpr int FFT_LDS = 2560;   // complex values of a block (40 KB: four blocks a CU)
 
-constexpr int FFT_LDS = 2048;  // complex values per LDS buffer (two buffers)
-
-__global__ void __launch_bounds__(256) k_fft(FftPass p, const int *gate) {
-  if (gate && !*gate) return;
-  extern __shared__ __align__(16) unsigned char fft_smem[];
-  cplx *A = (cplx *)fft_smem, *B = A + FFT_LDS;
-  const int M = p.ax.M, LPB = p.lpb;
-  const int nlines = p.nl0 * p.nl1;
-  const int L0 = blockIdx.x * LPB;
-  const int tot = LPB * M;
-  // load (zero beyond nin and beyond the last line); clamped addresses, selected at the store
-  for (int t0 = threadIdx.x; t0 < tot; t0 += 4 * blockDim.x) {
-    cplx v[4];
-    bool ok[4];
-    int dsti[4];
+// One Stockham autosort pass of radix R, in place: every butterfly of a thread is read into registers before any
+// is written.  Butterfly j reads src[j + r M/R], twiddles r by ω^(r (j mod Ns) M/(Ns R)), writes
+// dst[(j/Ns) Ns R + (j mod Ns) + r Ns].
+template <int R>
+__device__ __forceinline__ void fft_pass(cplx *A, int lg, int M, int Ns, const cplx *tw, int dir) {
+  constexpr int IM = (FFT_LDS / R + FFT_T - 1) / FFT_T;
+  const int MR = M / R, step = MR / Ns, items = MR << lg, l = threadIdx.x & ((1 << lg) - 1);
+  const float inv = 1.0f / (float)Ns;
+  cplx v[IM][R];
+  int base[IM];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int t = t0 + u * blockDim.x;
-      int l, e;
-      if (p.lines_fast) {
-        l = t % LPB;
-        e = t / LPB;
-      } else {
-        l = t / M;
-        e = t % M;
-      }
-      const int L = L0 + l;
-      ok[u] = t < tot && L < nlines && e < p.nin;
-      dsti[u] = t < tot ? l * M + e : -1;
-      const int Lc = L < nlines ? L : nlines - 1, ec = e < p.nin ? e : p.nin - 1;
-      const long long idx = (long long)(Lc % p.nl0) * p.in_l0 + (long long)(Lc / p.nl0) * p.in_l1 + (long long)ec * p.in_s;
-      v[u] = p.in_real ? mk(((const double *)p.in)[idx], 0.0) : ((const cplx *)p.in)[idx];
+  for (int u = 0; u < IM; ++u) {
+    const int item = (int)threadIdx.x + u * FFT_T;
+    base[u] = -1;
+    if (item < items) {
+      const int j = item >> lg, q = (int)(((float)j + 0.5f) * inv), k = j - q * Ns;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[u][r] = A[((j + r * MR) << lg) + l];
+      if (Ns > 1)
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          cplx w = tw[r * k * step];
+          if (dir > 0) w.y = -w.y;
+          v[u][r] = cmul(v[u][r], w);
+        }
+      dft_small<R>(v[u], dir);
+      base[u] = q * Ns * R + k;
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (dsti[u] >= 0) A[dsti[u]] = ok[u] ? v[u] : mk(0.0, 0.0);
   }
   __syncthreads();
-  cplx *R = fft_lines(A, B, LPB, p.ax, p.dir);
+#pragma unroll
+  for (int u = 0; u < IM; ++u)
+    if (base[u] >= 0)
+#pragma unroll
+      for (int r = 0; r < R; ++r) A[((base[u] + r * Ns) << lg) + l] = v[u][r];
+  __syncthreads();
+}
+__device__ void fft_lines(cplx *A, int lg, const FftAxis &ax, int dir) {
+  int Ns = 1;
+  for (int s = 0; s < ax.nrad; ++s) {
+    const int R = ax.rad[s];
+    if (R == 4)
+      fft_pass<4>(A, lg, ax.M, Ns, ax.tw, dir);
+    else if (R == 2)
+      fft_pass<2>(A, lg, ax.M, Ns, ax.tw, dir);
+    else if (R == 3)
+      fft_pass<3>(A, lg, ax.M, Ns, ax.tw, dir);
+    else
+      fft_pass<5>(A, lg, ax.M, Ns, ax.tw, dir);
+    Ns *= R;
+  }
+}
+
+// The passes of up to three lattices in one launch (blockIdx.y).  Bound by the reads and writes of the lines,
+// once a pass (1.35 GB a recomputation at 256 x 128 x 32, 0.28 ms at the rate of a copy), and by the passes'
+// LDS traffic: 2.0 ms a recomputation with the radices known when compiled, in place, four blocks a CU; 9.7 ms
+// with two buffers of 64 KB a block, the radix a runtime loop bound and the index divided by the line's length.
+struct FftSet {
+  FftPass p[3];
+};
+__global__ void __launch_bounds__(FFT_T, 4) k_fft(FftSet f, const int *gate) {
+  if (gate && !*gate) return;
+  const FftPass &p = f.p[blockIdx.y];
+  extern __shared__ __align__(16) unsigned char fft_smem[];
+  cplx *A = (cplx *)fft_smem;
+  __shared__ long long lin[64], lout[64], lgh[64];  // where each line of the block starts
+  const int M = p.ax.M, lg = p.lpb, LPB = 1 << lg;
+  const int nlines = p.nl0 * p.nl1, L0 = blockIdx.x << lg, tid = threadIdx.x;
+  if (L0 >= nlines) return;
+  if (tid < LPB) {
+    const int L = min(L0 + tid, nlines - 1), a = L % p.nl0, b = L / p.nl0;
+    lin[tid] = (long long)a * p.in_l0 + (long long)b * p.in_l1;
+    lout[tid] = (long long)a * p.out_l0 + (long long)b * p.out_l1;
+    lgh[tid] = (long long)a * p.g_l0 + (long long)b * p.g_l1;
+  }
+  __syncthreads();
+  const int tot = M << lg, nl = min(LPB, nlines - L0);
+  const float invM = 1.0f / (float)M, invO = 1.0f / (float)p.nout;
+  // load, zero beyond nin (clamped addresses, selected at the store), five in flight a thread
+  for (int t0 = tid; t0 < tot; t0 += 5 * FFT_T) {
+    cplx v[5];
+    int to[5];
+#pragma unroll
+    for (int u = 0; u < 5; ++u) {
+      const int t = min(t0 + u * FFT_T, tot - 1);
+      const int l = p.lines_fast ? (t & (LPB - 1)) : (int)(((float)t + 0.5f) * invM), e = p.lines_fast ? (t >> lg) : t - l * M;
+      const bool ok = e < p.nin;
+      const long long idx = lin[l] + (long long)(ok ? e : 0) * p.in_s;
+      v[u] = p.in_real ? mk(((const double *)p.in)[idx], 0.0) : ((const cplx *)p.in)[idx];
+      to[u] = (e << lg) + l;
+      if (!ok) v[u] = mk(0.0, 0.0);
+    }
+#pragma unroll
+    for (int u = 0; u < 5; ++u)
+      if (t0 + u * FFT_T < tot) A[to[u]] = v[u];
+  }
+  __syncthreads();
+  fft_lines(A, lg, p.ax, p.dir);
   if (p.ghat) {
     // times Ĝ (real), then back (the z pass of a convolution)
-    for (int t = threadIdx.x; t < tot; t += blockDim.x) {
-      const int l = t / M, e = t % M;
-      const int L = L0 + l;
-      if (L >= nlines) continue;
-      const double gv = p.ghat[(long long)(L % p.nl0) * p.g_l0 + (long long)(L / p.nl0) * p.g_l1 + (long long)e * p.g_s];
-      R[t] = rmul(gv, R[t]);
+    const int l = tid & (LPB - 1), le = FFT_T >> lg;
+    const double *gl = p.ghat + lgh[l];
+    for (int e0 = tid >> lg; e0 < M; e0 += 5 * le) {
+      double g[5];
+#pragma unroll
+      for (int u = 0; u < 5; ++u) g[u] = gl[(long long)min(e0 + u * le, M - 1) * p.g_s];
+#pragma unroll
+      for (int u = 0; u < 5; ++u) {
+        const int e = e0 + u * le;
+        if (e < M) A[(e << lg) + l] = rmul(g[u], A[(e << lg) + l]);
+      }
     }
     __syncthreads();
-    cplx *other = R == A ? B : A;
-    R = fft_lines(R, other, LPB, p.ax, -p.dir);
+    fft_lines(A, lg, p.ax, -p.dir);
   }
   // store the first nout of every line
-  for (int t = threadIdx.x; t < LPB * p.nout; t += blockDim.x) {
-    int l, e;
-    if (p.lines_fast) {
-      l = t % LPB;
-      e = t / LPB;
-    } else {
-      l = t / p.nout;
-      e = t % p.nout;
-    }
-    const int L = L0 + l;
-    if (L >= nlines) continue;
-    const cplx v = R[l * M + e];
-    const long long idx = (long long)(L % p.nl0) * p.out_l0 + (long long)(L / p.nl0) * p.out_l1 + (long long)e * p.out_s;
+  for (int t = tid; t < (p.nout << lg); t += FFT_T) {
+    const int l = p.lines_fast ? (t & (LPB - 1)) : (int)(((float)t + 0.5f) * invO), e = p.lines_fast ? (t >> lg) : t - l * p.nout;
+    if (l >= nl) continue;
+    const cplx v = A[(e << lg) + l];
+    const long long idx = lout[l] + (long long)e * p.out_s;
     if (p.out_real)
       ((double *)p.out)[idx] = v.x * p.scale;
     else
@@ -210,15 +239,26 @@ __global__ void __launch_bounds__(256) k_fft(FftPass p, const int *gate) {
   }
 }
 
-int fft_lpb(int M) { return std::max(1, std::min(64, FFT_LDS / M)); }
+// lines of a block, log2: the most (at most 64) whose elements fit FFT_LDS
+static int fft_lg(int M) {
+  int lg = 0;
+  while (lg < 6 && (M << (lg + 1)) <= FFT_LDS) ++lg;
+  return lg;
+}
 
-hipError_t launch_fft(FftPass p, const int *gate, hipStream_t s) {
+hipError_t launch_fft(const FftPass *p, int n, const int *gate, hipStream_t s) {
   if (g_rec) return hipErrorNotSupported;
-  if (p.ax.M < 1 || p.ax.M > FFT_LDS || p.nin < 1 || p.nin > p.ax.M || p.nout < 1 || p.nout > p.ax.M)
-    return hipErrorInvalidValue;
-  p.lpb = fft_lpb(p.ax.M);
-  const int nlines = p.nl0 * p.nl1;
-  TDGL_LAUNCH(k_fft, dim3(cdiv(nlines, p.lpb)), dim3(256), 2 * FFT_LDS * sizeof(cplx), s, p, gate);
+  if (n < 1 || n > 3) return hipErrorInvalidValue;
+  FftSet f{};
+  int nb = 1;
+  for (int q = 0; q < n; ++q) {
+    f.p[q] = p[q];
+    if (p[q].ax.M < 1 || p[q].ax.M > 2048 || p[q].nin < 1 || p[q].nin > p[q].ax.M || p[q].nout < 1 || p[q].nout > p[q].ax.M)
+      return hipErrorInvalidValue;
+    f.p[q].lpb = fft_lg(p[q].ax.M);
+    nb = std::max(nb, cdiv(p[q].nl0 * p[q].nl1, 1 << f.p[q].lpb));
+  }
+  TDGL_LAUNCH(k_fft, dim3(nb, n), dim3(FFT_T), FFT_LDS * sizeof(cplx), s, f, gate);
   return hipGetLastError();
 }
 

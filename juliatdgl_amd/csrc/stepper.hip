@@ -1618,7 +1618,7 @@ void fft_radices(int M, FftAxis &ax) {
 
 // the five passes of one lattice's convolution: x forward from δJ, y forward, z forward × Ĝ and
 // back, y back, x back into θ_δ (the padding is never stored)
-int open_convolve(tdgl_handle *h, int c, const int *gate) {
+void open_passes(tdgl_handle *h, int c, FftPass ps[5]) {
   const int n0 = h->on[c][0], n1 = h->on[c][1], n2 = h->on[c][2];
   const int M0 = h->oM[c][0], M1 = h->oM[c][1], M2 = h->oM[c][2];
   const long long P = (long long)M0 * M1;
@@ -1640,7 +1640,7 @@ int open_convolve(tdgl_handle *h, int c, const int *gate) {
   p.nout = M0;
   p.dir = -1;
   p.ax = h->oax[c][0];
-  PL(K_CURL, launch_fft(p, gate, h->s));
+  ps[0] = p;
   // y forward: lines (i < M0, k < n2)
   FftPass q{};
   q.in = q.out = h->obuf[c];
@@ -1655,7 +1655,7 @@ int open_convolve(tdgl_handle *h, int c, const int *gate) {
   q.dir = -1;
   q.lines_fast = 1;
   q.ax = h->oax[c][1];
-  PL(K_CURL, launch_fft(q, gate, h->s));
+  ps[1] = q;
   // z: forward, × Ĝ, back; lines (i < M0, j < M1), only the box's planes kept
   FftPass z = q;
   z.in_s = z.out_s = P;
@@ -1670,13 +1670,13 @@ int open_convolve(tdgl_handle *h, int c, const int *gate) {
   z.g_l0 = 1;
   z.g_l1 = M0;
   z.ax = h->oax[c][2];
-  PL(K_CURL, launch_fft(z, gate, h->s));
+  ps[2] = z;
   // y back
   FftPass yb = q;
   yb.nin = M1;
   yb.nout = n1;
   yb.dir = 1;
-  PL(K_CURL, launch_fft(yb, gate, h->s));
+  ps[3] = yb;
   // x back into θ_δ, normalized
   FftPass xb{};
   xb.in = h->obuf[c];
@@ -1695,7 +1695,16 @@ int open_convolve(tdgl_handle *h, int c, const int *gate) {
   xb.nout = n0;
   xb.dir = 1;
   xb.ax = h->oax[c][0];
-  PL(K_CURL, launch_fft(xb, gate, h->s));
+  ps[4] = xb;
+}
+// the convolutions of the three lattices, a launch a pass
+int open_convolve(tdgl_handle *h, const int *gate) {
+  FftPass ps[3][5];
+  for (int c = 0; c < 3; ++c) open_passes(h, c, ps[c]);
+  for (int q = 0; q < 5; ++q) {
+    const FftPass p[3] = {ps[0][q], ps[1][q], ps[2][q]};
+    PL(K_CURL, launch_fft(p, 3, gate, h->s));
+  }
   return 0;
 }
 
@@ -1730,7 +1739,7 @@ int open_update(tdgl_handle *h) {
   dj.dy = d.dy;
   dj.dz = d.dz;
   PL(K_CURL, launch_open_dj(h->g, dj, h->s));
-  for (int c = 0; c < 3; ++c) CHK(open_convolve(h, c, re));
+  CHK(open_convolve(h, re));
   OpenFace f{};
   for (int c = 0; c < 3; ++c) {
     f.theta[c] = h->oth[c];
@@ -1791,7 +1800,7 @@ int open_green(tdgl_handle *h) {
       p.nin = p.nout = M0;
       p.dir = -1;
       p.ax = h->oax[c][0];
-      LCHK(launch_fft(p, nullptr, h->s));
+      LCHK(launch_fft(&p, 1, nullptr, h->s));
       FftPass q{};
       q.in = q.out = G;
       q.scale = 1.0;
@@ -1804,7 +1813,7 @@ int open_green(tdgl_handle *h) {
       q.dir = -1;
       q.lines_fast = 1;
       q.ax = h->oax[c][1];
-      LCHK(launch_fft(q, nullptr, h->s));
+      LCHK(launch_fft(&q, 1, nullptr, h->s));
       FftPass z = q;
       z.out = h->oghat[c];
       z.out_real = 1;
@@ -1815,7 +1824,7 @@ int open_green(tdgl_handle *h) {
       z.nl1 = M1;
       z.nin = z.nout = M2;
       z.ax = h->oax[c][2];
-      LCHK(launch_fft(z, nullptr, h->s));
+      LCHK(launch_fft(&z, 1, nullptr, h->s));
       HIPCHK(hipStreamSynchronize(h->s));
       return 0;
     };
