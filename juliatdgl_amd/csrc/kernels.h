@@ -720,7 +720,7 @@ struct SectCG {
   double ca, a;             // curl-curl coefficient of the operator, a of the preconditioner
   double share;             // 1 / the number of sectors
   int maxit;
-  int np, trows;            // set by the launcher: P's elements, T's rows
+  int np, trows, ng;        // set by the launcher: P's places, T's rows, ghosts
 };
 bool sect_cg_fits(const SectCG &a);
 hipError_t launch_sect_cg(SectCG a, hipStream_t s);

@@ -342,13 +342,20 @@ hipError_t launch_sect_inv(SectX p, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------- the CG of a sector
-// One block per sector.  r, Q and z_old of a thread's elements (e = tid + threads i) stay in registers,
-// the direction P in LDS (FP64, its stencil reads neighbours), the preconditioner's work array T in LDS
-// (Float32): rows are the sector's z columns (X's, then Z's, then Y's), j or the y mode along the row.
+// One block per sector.  r, d, Q and z_old of a thread's elements (e = tid + threads i) stay in registers,
+// the direction P in LDS (FP64, its stencil reads neighbours) with a ring of ghost places that follow the
+// same recurrence with the mirrored z, so that every element's stencil is the same nine or eleven reads, and
+// the preconditioner's work array T in LDS (Float32): rows are the sector's z columns (X's, then Z's, then
+// Y's), j or the y mode along the row.
 // The preconditioner multiplies every row by the half-size y basis (16 x 16 x 4 tiles, the basis from
-// L2), then each wave takes 16 y modes through the z transform, the projector and the inverse z
-// transform in registers (a forward tile leaves in a lane the modes its inverse takes as operand), then
-// the inverse y products.  d += αP goes to global memory (it is the output).
+// L2, its first groups asked for before the barrier), then each wave takes 16 y modes through the z transform,
+// the projector and the inverse z transform in registers (a forward tile leaves in a lane the modes its inverse
+// takes as operand), then the inverse y products.
+// Bound: on 272 x 144 x 48 nodes the matrix products of an iteration are 11.8 k cycles of the 42 k it takes a
+// block there (two share a CU), the rest LDS reads of the stencil, FP64 sums and what ten elements a thread spill
+// past 128 registers; on small planes the chain of ten barriers an iteration, 10 k cycles.  Before the ghosts
+// (branches at every edge) and with d in global memory: 955 us there, now 812; 82 to 54 us on 100 x 52 x 28 nodes,
+// 126 to 78 on 83 x 49 x 21, 38 to 26 on 57 x 31 x 13.
 // The sums are FP64, in a fixed order: the same bits every time.
 // Where it stops: a sector's share of (SECT_TIGHT tol ||b||)² is half an equal share and half its share of
 // the first residual, so the sectors' residuals together are below the tolerance, no sector iterates for
@@ -359,13 +366,6 @@ hipError_t launch_sect_inv(SectX p, hipStream_t s) {
 // (1.5e-8 on 53x27x9, 3.3e-8 against 2.0e-7 on 144x17x21, 9e-11 against 6e-10 with KWT) or as near (5.4e-9
 // against 2.5e-9 and 7.1e-9, full length and folded, on 96x48x24), for 15 % more iterations.
 constexpr double SECT_TIGHT = 0.125;
-struct SectGhost {
-  double gn, ge;  // mirrored node past the last (even count, odd parity: -1), mirrored edge (odd count, even parity: -1)
-};
-__device__ __forceinline__ SectGhost sect_ghost(int n, int par) {
-  return SectGhost{(n % 2 == 0 && par) ? -1.0 : 0.0, (n % 2 == 1 && !par) ? -1.0 : 0.0};
-}
-
 // the same value, which the compiler does not know to be: what is derived from it is formed where it is used
 // and not kept in registers through the iterations
 __device__ __forceinline__ int fresh(int v) {
@@ -373,11 +373,30 @@ __device__ __forceinline__ int fresh(int v) {
   return v;
 }
 
+// one step of a wave's sum through DPP: lanes outside the row mask or the row add 0
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+// the sum of a wave's values, in lane 63
+__device__ __forceinline__ double wave_sum63(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15, 31
+  return dpp_add<0x143, 0xc>(v);
+}
+
 template <int EPT, int ZT, int SM>
 __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   if (!sect_active(a.d)) return;
   extern __shared__ __align__(16) unsigned char cg_smem[];
-  __shared__ double red[4][SECT_T / 64];
+  static_assert(SECT_T == 512, "eight waves");
+  constexpr bool SMALL = EPT <= 4;  // few elements: what every iteration needs stays in registers
+  __shared__ __align__(16) double red[4][8];
   __shared__ double pal[3 * DPAL_MAX];
   const int tid = threadIdx.x, nth = blockDim.x, nw = nth >> 6;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
@@ -387,25 +406,74 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   const int oY = q.oc[1][s], oZ = q.oc[2][s];
   double *P = (double *)cg_smem;
   float *T = (float *)(P + a.np);
+  unsigned *G = (unsigned *)(T + a.trows * (a.yp + 4));
   const int ST = a.yp + 4, CY = lz + lze;
   const int mt = (ly + 15) / 16, nt1 = (CY + 15) / 16, nt2 = (lz + 15) / 16, ntile = mt * (nt1 + nt2);
+  // P: component c at pc[c] + (k + 1) RS + j + 1, a ring of ghost places around each
+  const int RS = ly + 2, pY = (lz + 2) * RS, pZ = 2 * pY;
+  auto pat = [&](int c, int j, int k) { return (c == 0 ? 0 : (c == 1 ? pY : pZ)) + (k + 1) * RS + j + 1; };
+  auto tat = [&](int c, int j, int k) { return (c == 0 ? k : (c == 1 ? CY + k : lz + k)) * ST + j; };  // the place in T
   for (int t = tid; t < a.trows * ST; t += nth) T[t] = 0.0f;
+  for (int t = tid; t < a.np; t += nth) P[t] = 0.0;
   if (tid < 3 * DPAL_MAX) pal[tid] = a.pal[tid];
+  if (tid < 32) red[tid >> 3][tid & 7] = 0.0;
+  float *kz = (float *)(G + a.ng);  // the z wave numbers of this parity
+  for (int t = tid; t < lz; t += nth) kz[t] = 2 * t + pz < q.nz ? a.sfz[2 * t + pz] : 0.0f;
   const double sv = a.sx[mx], ca = a.ca;
   const double tolb = a.d.sc[SC_TOL] * a.d.sc[SC_NB];
-  const SectGhost gy = sect_ghost(q.ny, py), gz = sect_ghost(q.nz, pz);
   const size_t base = (size_t)q.off[s] + (size_t)mx * n;
 
-  // this thread's elements: j | k << 10 | component << 20 | log2 weight << 22 | D code << 24 | live << 28
-  unsigned id[EPT];
-  double r[EPT];
+  // The ghosts, place | source in T << 14 | sign << 28 (1 +, 2 -).  The difference across the boundary is zero
+  // (the outer ring repeats the node, or is a zero edge); across the centre it is the mirrored node (even
+  // count ± the last, odd count the one before the last) or edge (odd count - the last, even count the zero
+  // centre).  A sign of 0 stays the zero that P was filled with.
+  {
+    const int yn = q.ny % 2 ? ly - 2 : ly - 1, zn = q.nz % 2 ? lz - 2 : lz - 1;
+    const int sy = q.ny % 2 ? (py ? 0 : 1) : (py ? -1 : 1), sz = q.nz % 2 ? (pz ? 0 : 1) : (pz ? -1 : 1);
+    const int ey = q.ny % 2 && !py ? -1 : 0, ez = q.nz % 2 && !pz ? -1 : 0;
+    int at = 0;
+    auto run = [&](int cnt, auto entry) {  // entry(i): component, source, place, sign
+      for (int i = (tid + nth - at % nth) % nth; i < cnt; i += nth) entry(i);
+      at += cnt;
+    };
+    int g0 = 0;
+    auto put = [&](int i, int c, int j, int k, int js, int ks, int sg) {
+      G[g0 + i] = (unsigned)pat(c, j, k) | ((unsigned)tat(c, sg ? js : 0, sg ? ks : 0) << 14) | (sg > 0 ? 1u << 28 : (sg < 0 ? 2u << 28 : 0u));
+    };
+    run(lz, [&](int k) { put(k, 0, -1, k, 0, k, 1); });
+    g0 = at;
+    run(lz, [&](int k) { put(k, 0, ly, k, yn, k, sy); });
+    g0 = at;
+    run(ly, [&](int j) { put(j, 0, j, -1, j, 0, 1); });
+    g0 = at;
+    run(ly, [&](int j) { put(j, 0, j, lz, j, zn, sz); });
+    g0 = at;
+    run(lz + 1, [&](int k) { put(k, 1, le, k, le - 1, k < lz ? k : zn, ey * (k < lz ? 1 : sz)); });
+    g0 = at;
+    run(le, [&](int j) { put(j, 1, j, -1, j, 0, 1); });
+    g0 = at;
+    run(le, [&](int j) { put(j, 1, j, lz, j, zn, sz); });
+    g0 = at;
+    run(lze, [&](int k) { put(k, 2, -1, k, 0, k, 1); });
+    g0 = at;
+    run(lze + 1, [&](int k) { put(k, 2, ly, k, yn, k < lze ? k : lze - 1, sy * (k < lze ? 1 : ez)); });
+    g0 = at;
+    run(ly, [&](int j) { put(j, 2, j, lze, j, lze - 1, ez); });
+  }
+  const int ng = 3 * (ly + lz) + 2 * (le + lze) + 2;
+
+  // this thread's elements: place in P | place in T << 14 | log2 weight << 28 | component << 30, and D's codes
+  unsigned id[EPT], code[(EPT + 7) / 8];
+  double r[EPT], d[EPT];
   float zo[EPT];
   double rr = 0.0;
+#pragma unroll
+  for (int i = 0; i < (EPT + 7) / 8; ++i) code[i] = 0u;
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
     const int e = tid + nth * i;
     id[i] = 0u;
-    r[i] = 0.0;
+    r[i] = d[i] = 0.0;
     zo[i] = 0.0f;
     if (e < n) {
       const int c = e < oY ? 0 : (e < oZ ? 1 : 2), f = e - (c == 0 ? 0 : (c == 1 ? oY : oZ)), row = c == 1 ? le : ly;
@@ -413,63 +481,80 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
       const bool cy = c == 1 ? (q.ny % 2 == 0 && py && j == le - 1) : (q.ny % 2 == 1 && !py && j == ly - 1);
       const bool cz = c == 2 ? (q.nz % 2 == 0 && pz && k == lze - 1) : (q.nz % 2 == 1 && !pz && k == lz - 1);
       const unsigned wt = (cy ? 0u : 1u) + (cz ? 0u : 1u);
-      const unsigned code = a.code[c][j + q.hy[c == 1][c == 1] * k];
-      id[i] = (unsigned)j | ((unsigned)k << 10) | ((unsigned)c << 20) | (wt << 22) | (code << 24) | (1u << 28);
+      code[i / 8] |= (unsigned)a.code[c][j + q.hy[c == 1][c == 1] * k] << (4 * (i % 8));
+      id[i] = (unsigned)pat(c, j, k) | ((unsigned)tat(c, j, k) << 14) | (wt << 28) | ((unsigned)c << 30);
       if (!(c == 0 && mx == 0)) r[i] = a.R[base + e];
       rr += (double)(1u << wt) * (r[i] * r[i]);
     }
   }
+  __syncthreads();  // T is zero
   auto sum_of = [&](int slot, double v) {
-    v = wave_sum_d(v);
-    if (l == 0) red[slot][w] = v;
+    v = wave_sum63(v);
+    if (l == 63) red[slot][w] = v;
   };
   auto total = [&](int slot) {
-    double t = 0.0;
-    for (int k = 0; k < nw; ++k) t += red[slot][k];
-    return t;
+    const double *p = red[slot];  // the waves that are not there hold 0
+    return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
   };
+  auto put_r = [&] {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i)
+      if (tid + nth * i < n) T[(id[i] >> 14) & 16383u] = (float)r[i];
+  };
+  auto weight = [&](unsigned v) { return (double)(1u << ((v >> 28) & 3u)); };
   sum_of(0, rr);
+  put_r();
   __syncthreads();
   rr = total(0);
   const double thr = SECT_TIGHT * SECT_TIGHT * 0.5 * tolb * tolb * (a.share + rr / a.d.sc[SC_RR]);
-  if (!(rr > thr)) {
-#pragma unroll
-    for (int i = 0; i < EPT; ++i)
-      if (id[i] >> 28) a.X[base + tid + nth * i] = 0.0;
-    return;
-  }
-  auto tcol = [&](unsigned v) {  // the element's place in T
-    const int j = v & 1023, k = (v >> 10) & 1023, c = (v >> 20) & 3;
-    return (c == 0 ? k : (c == 1 ? CY + k : lz + k)) * ST + j;
-  };
+  const float imt = 1.0f / (float)mt;
   // one pass of the y products over the rows of T: rows x basis, in place
-  auto ypass = [&](const float *BV, const float *BU) {
+  struct First {
+    v4f a, b;  // the first tile's first two groups of the basis
+  };
+  auto tile = [&](int t, int &m, int &nt) __attribute__((always_inline)) {
+    const int tt = w + nw * t;
+    nt = __builtin_amdgcn_readfirstlane((int)(((float)tt + 0.5f) * imt));
+    m = tt - nt * mt;
+    return tt < ntile;
+  };
+  auto first = [&](const float *BV, const float *BU) __attribute__((always_inline)) {
+    First f{v4f{0, 0, 0, 0}, v4f{0, 0, 0, 0}};
+    int m, nt;
+    if (tile(0, m, nt)) {
+      const float *A = (nt < nt1 ? BV : BU) + 16 * m * a.yp + fresh(lr) * a.yp + 4 * lk;
+      f.a = *(const v4f *)A;
+      f.b = *(const v4f *)(A + 16 * min(1, mt - 1));
+    }
+    return f;
+  };
+  auto ypass = [&](const float *BV, const float *BU, const First f) __attribute__((always_inline)) {
     const int la = fresh(lr) * a.yp + 4 * lk, lb = fresh(lr) * ST + 4 * lk;
     v4f acc[SM];
 #pragma unroll
     for (int t = 0; t < SM; ++t) {
       acc[t] = v4f{0, 0, 0, 0};
-      const int tt = w + nw * t;
-      if (tt < ntile) {
-        const int m = tt % mt, nt = tt / mt;
+      int m, nt;
+      if (tile(t, m, nt)) {
         const float *A = (nt < nt1 ? BV : BU) + 16 * m * a.yp + la;
         const float *B = T + (nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1)) * ST + lb;
-        v4f av = *(const v4f *)A;
+        // the basis comes through L2: two groups of sixteen ahead
+        v4f av = t ? *(const v4f *)A : f.a, an = t ? *(const v4f *)(A + 16 * min(1, mt - 1)) : f.b;
         for (int g = 0; g < mt; ++g) {
-          const v4f an = *(const v4f *)(A + 16 * min(g + 1, mt - 1));
+          const v4f aq = *(const v4f *)(A + 16 * min(g + 2, mt - 1));
           const v4f bv = *(const v4f *)(B + 16 * g);
 #pragma unroll
           for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc[t], 0, 0, 0);
           av = an;
+          an = aq;
         }
       }
     }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < SM; ++t) {
-      const int tt = w + nw * t;
-      if (tt < ntile) {
-        const int m = tt % mt, nt = tt / mt;
+      int m, nt;
+      if (tile(t, m, nt)) {
         const int col0 = nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1);
         if (col0 + lr < (nt < nt1 ? CY : CY + lz)) *(v4f *)(T + col0 * ST + 16 * m + lb) = acc[t];
       }
@@ -477,70 +562,86 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
     __syncthreads();
   };
 
-  double rzold = 0.0;
+  const float *const yf[2] = {a.yb[py][0][0], a.yb[py][1][0]}, *const yr[2] = {a.yb[py][0][1], a.yb[py][1][1]};
+  First ff = first(yf[0], yf[1]), fr = ff;
+  if (SMALL) fr = first(yr[0], yr[1]);
+  // the z bases, fragment (t, g) of matrix: 0 V forward, 1 U forward, 2 V back, 3 U back
+  constexpr bool ZREG = SMALL && ZT == 1;
+  auto zfrag = [&](int which, int t, int g, int l) {
+    return *(const v4f *)(a.zb[pz][which & 1][which >> 1] + (16 * t + (l & 15)) * a.zp + 16 * g + 4 * (l >> 4));
+  };
+  v4f zr[4] = {};
+  if (ZREG)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) zr[i] = zfrag(i, 0, 0, l);
+  double dreg[SMALL ? EPT : 1] = {};
+  if (SMALL)
+#pragma unroll
+    for (int i = 0; i < (SMALL ? EPT : 1); ++i) dreg[i] = pal[DPAL_MAX * min(id[i] >> 30, 2u) + ((code[i / 8] >> (4 * (i % 8))) & 15u)];
+  const unsigned gv = tid < ng ? G[tid] : 0u;  // the first ghost
+
+  double rzold = 1.0;
   int it = 0;
-  for (;;) {
-    // z = M⁻¹ r in Float32
+  while (rr > thr && it < a.maxit) {
+    // z = M⁻¹ r in Float32; T holds r
 #pragma unroll
     for (int i = 0; i < EPT; ++i) id[i] = (unsigned)fresh((int)id[i]);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i)
-      if (id[i] >> 28) T[tcol(id[i])] = (float)r[i];
-    __syncthreads();
-    ypass(a.yb[py][0][0], a.yb[py][1][0]);
+    ypass(yf[0], yf[1], ff);
     for (int m = w; m < mt; m += nw) {
       // 16 y modes: z forward, the projector, z back; k = 16 g + 4 lk + u of the rows (zero past them)
-      v4f Bx[ZT], By[ZT], Bz[ZT];
       const int lf = fresh(l), lr = lf & 15, lk = lf >> 4;
       const float *Tq = T + 16 * m + lr;
-#pragma unroll
-      for (int g = 0; g < ZT; ++g)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int k = 16 * g + 4 * lk + u;
-          const float vx = Tq[min(k, lz - 1) * ST], vy = Tq[(CY + min(k, lz - 1)) * ST], vz = Tq[(lz + min(k, lze - 1)) * ST];
-          Bx[g][u] = k < lz ? vx : 0.0f;
-          By[g][u] = k < lz ? vy : 0.0f;
-          Bz[g][u] = k < lze ? vz : 0.0f;
-        }
       v4f acc[3][ZT];
 #pragma unroll
-      for (int t = 0; t < ZT; ++t) {
-        acc[0][t] = acc[1][t] = acc[2][t] = v4f{0, 0, 0, 0};
+      for (int t = 0; t < ZT; ++t) acc[0][t] = acc[1][t] = acc[2][t] = v4f{0, 0, 0, 0};
 #pragma unroll
-        for (int g = 0; g < ZT; ++g) {
-          const v4f Av = *(const v4f *)(a.zb[pz][0][0] + (16 * t + lr) * a.zp + 16 * g + 4 * lk);
-          const v4f Au = *(const v4f *)(a.zb[pz][1][0] + (16 * t + lr) * a.zp + 16 * g + 4 * lk);
+      for (int g = 0; g < ZT; ++g) {
+        // a component's rows at a time, the fragments of both node components once
+        auto rows = [&](int row0, int cnt) {
+          v4f B;
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Av[u], Bx[g][u], acc[0][t], 0, 0, 0);
-            acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Av[u], By[g][u], acc[1][t], 0, 0, 0);
-            acc[2][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(Au[u], Bz[g][u], acc[2][t], 0, 0, 0);
+            const int k = 16 * g + 4 * lk + u;
+            const float v = Tq[(row0 + min(k, cnt - 1)) * ST];
+            B[u] = k < cnt ? v : 0.0f;
           }
+          return B;
+        };
+        v4f A[ZT];
+#pragma unroll
+        for (int t = 0; t < ZT; ++t) A[t] = ZREG ? zr[0] : zfrag(0, t, g, lf);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          const v4f B = rows(c == 0 ? 0 : (c == 1 ? CY : lz), c == 2 ? lze : lz);
+          if (c == 2)
+#pragma unroll
+            for (int t = 0; t < ZT; ++t) A[t] = ZREG ? zr[1] : zfrag(1, t, g, lf);
+#pragma unroll
+          for (int t = 0; t < ZT; ++t)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[t][u], B[u], acc[c][t], 0, 0, 0);
         }
+        if (ZT > 1) __builtin_amdgcn_sched_barrier(0);  // the registers of one group at a time
       }
       {
         const int my = 2 * (16 * m + lr) + py;
-        const float k1 = a.sfx[mx], k2 = my < q.ny ? a.sfy[my] : 0.0f;
+        const float k1 = a.sfx[mx], k2 = my < q.ny ? a.sfy[my] : 0.0f, af = (float)a.a;
         const bool live = my < q.ny, hx = mx > 0, hy = my > 0;
 #pragma unroll
         for (int t = 0; t < ZT; ++t)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
+            // (I + aK)^{-1} = P_L + P_T / (1 + a |k|²) = (I + a k kᵀ) / (1 + a |k|²) (implicit.jl:67-78); a component
+            // without the mode is zero
             const int mz = 2 * (16 * t + 4 * lk + e) + pz;
-            if (!live || mz >= q.nz) continue;
-            const float k3 = a.sfz[mz], k2s = k1 * k1 + k2 * k2 + k3 * k3;
-            const bool hz = mz > 0;
-            float x1 = hx ? acc[0][t][e] : 0.0f, y1 = hy ? acc[1][t][e] : 0.0f, z1 = hz ? acc[2][t][e] : 0.0f;
-            if (k2s != 0) {  // (I + aK)^{-1} = P_L + P_T / (1 + a |k|²) (implicit.jl:67-78)
-              const float dd = (k1 * x1 + k2 * y1 + k3 * z1) / k2s, f = 1.0f / (1.0f + (float)a.a * k2s);
-              if (hx) x1 = k1 * dd + f * (x1 - k1 * dd);
-              if (hy) y1 = k2 * dd + f * (y1 - k2 * dd);
-              if (hz) z1 = k3 * dd + f * (z1 - k3 * dd);
-            }
-            acc[0][t][e] = x1;
-            acc[1][t][e] = y1;
-            acc[2][t][e] = z1;
+            const bool in = live && mz < q.nz;
+            const float k3 = in ? kz[16 * t + 4 * lk + e] : 0.0f, f = 1.0f / (1.0f + af * (k1 * k1 + k2 * k2 + k3 * k3));
+            const float x1 = hx ? acc[0][t][e] : 0.0f, y1 = hy ? acc[1][t][e] : 0.0f, z1 = mz > 0 ? acc[2][t][e] : 0.0f;
+            const float dd = af * (k1 * x1 + k2 * y1 + k3 * z1);
+            acc[0][t][e] = hx ? f * (x1 + k1 * dd) : 0.0f;
+            acc[1][t][e] = hy ? f * (y1 + k2 * dd) : 0.0f;
+            acc[2][t][e] = mz > 0 ? f * (z1 + k3 * dd) : 0.0f;
+            if (ZT > 1 && e % 2) __builtin_amdgcn_sched_barrier(0);
           }
       }
       __builtin_amdgcn_wave_barrier();  // the tile's columns are read: their rows take the result
@@ -553,7 +654,7 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
           v4f o = v4f{0, 0, 0, 0};
 #pragma unroll
           for (int g = 0; g < ZT; ++g) {
-            const v4f A = *(const v4f *)(a.zb[pz][c == 2 ? 1 : 0][1] + (16 * t + lr) * a.zp + 16 * g + 4 * lk);
+            const v4f A = ZREG ? zr[c == 2 ? 3 : 2] : zfrag(c == 2 ? 3 : 2, t, g, lf);
 #pragma unroll
             for (int u = 0; u < 4; ++u) o = __builtin_amdgcn_mfma_f32_16x16x4f32(A[u], acc[c][g][u], o, 0, 0, 0);
           }
@@ -563,102 +664,95 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
             if (k < rows) To[k * ST] = o[e];
           }
         }
+        if (ZT > 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if (!SMALL) fr = first(yr[0], yr[1]);
     __syncthreads();
-    ypass(a.yb[py][0][1], a.yb[py][1][1]);
+    ypass(yr[0], yr[1], fr);
     // the dots and the direction
     float z[EPT];
     double rz = 0.0, rzo = 0.0;
 #pragma unroll
     for (int i = 0; i < EPT; ++i) {
       z[i] = 0.0f;
-      if (id[i] >> 28) {
-        z[i] = T[tcol(id[i])];
-        const double wr = (double)(1u << ((id[i] >> 22) & 3u)) * r[i];
-        rz += wr * (double)z[i];
-        rzo += wr * (double)zo[i];
+      if (tid + nth * i < n) {
+        z[i] = T[(id[i] >> 14) & 16383u];
+        const double wr = weight(id[i]) * r[i];
+        rz = fma(wr, (double)z[i], rz);
+        rzo = fma(wr, (double)zo[i], rzo);
         zo[i] = z[i];
       }
     }
     sum_of(0, rz);
     sum_of(1, rzo);
+    auto ghost_z = [&](unsigned v) { return (v >> 28) & 2u ? -(double)T[(v >> 14) & 16383u] : (double)T[(v >> 14) & 16383u]; };
+    const double gz = ghost_z(gv), gp = P[gv & 16383u];
+    double pold[SMALL ? EPT : 1];
+    if (SMALL)
+#pragma unroll
+      for (int i = 0; i < (SMALL ? EPT : 1); ++i) pold[i] = P[id[i] & 16383u];
     __syncthreads();
     rz = total(0);
-    rzo = total(1);
-    const double beta = it > 0 ? (rz - rzo) / rzold : 0.0;
+    const double beta = it > 0 ? (rz - total(1)) / rzold : 0.0;
     rzold = rz;
 #pragma unroll
     for (int i = 0; i < EPT; ++i)
-      if (id[i] >> 28) {
-        const int e = tid + nth * i;
-        P[e] = it > 0 ? (double)z[i] + beta * P[e] : (double)z[i];
+      if (tid + nth * i < n) {
+        double *p = P + (id[i] & 16383u);
+        *p = fma(beta, SMALL ? pold[SMALL ? i : 0] : *p, (double)z[i]);
       }
+    if (gv >> 28) P[gv & 16383u] = fma(beta, gp, gz);
+    for (int g = tid + nth; g < ng; g += nth) {
+      const unsigned v = G[g];
+      double *p = P + (v & 16383u);
+      if (v >> 28) *p = fma(beta, *p, ghost_z(v));
+    }
     __syncthreads();
-    // Q = (D + aK) P on the half domain
+    // Q = (D + aK) P on the half domain: the ghosts make every place alike.  Edges along y and z: the same with
+    // the directions swapped (da across the edge in the plane, db along it).
     double Q[EPT], pq = 0.0;
 #pragma unroll
     for (int i = 0; i < EPT; ++i) {
       Q[i] = 0.0;
-      const unsigned v = (unsigned)fresh((int)id[i]);
-      if (v >> 28) {
-        const int j = v & 1023, k = (v >> 10) & 1023, c = (v >> 20) & 3;
-        const double *PX = P + j + ly * k, *PY = P + oY + j + le * k, *PZ = P + oZ + j + ly * k;
-        // curl components at edge offsets (dj, dk) of the element: hz and hx need the node past the edge
-        // along y, hy and hx along z
-        auto hzv = [&](int dj) {
-          const double up = j + dj + 1 < ly ? PX[dj + 1] : gy.gn * PX[dj];
-          return sv * PY[dj] - (up - PX[dj]);
-        };
-        auto hyv = [&](int dk) {
-          const double up = k + dk + 1 < lz ? PX[ly * (dk + 1)] : gz.gn * PX[ly * dk];
-          return (up - PX[ly * dk]) - sv * PZ[ly * dk];
-        };
-        auto hxv = [&](int dj, int dk) {
-          const double *z0 = PZ + dj + ly * dk, *y0 = PY + dj + le * dk;
-          const double zu = j + dj + 1 < ly ? z0[1] : gy.gn * z0[0], yu = k + dk + 1 < lz ? y0[le] : gz.gn * y0[0];
-          return (zu - z0[0]) - (yu - y0[0]);
-        };
-        double cur, pc;
+      if (tid + nth * i < n) {
+        const unsigned v = (unsigned)fresh((int)id[i]), c = v >> 30;
+        const double *A = P + (v & 16383u);
+        const double p0 = A[0];
+        double cur;
         if (c == 0) {
-          const double hzm = j > 0 ? hzv(-1) : 0.0, hzc = j < le ? hzv(0) : gy.ge * hzm;
-          const double hym = k > 0 ? hyv(-1) : 0.0, hyc = k < lze ? hyv(0) : gz.ge * hym;
-          cur = (hzc - hzm) - (hyc - hym);
-          pc = PX[0];
-        } else if (c == 1) {
-          const double hxm = k > 0 ? hxv(0, -1) : 0.0, hxc = k < lze ? hxv(0, 0) : gz.ge * hxm;
-          cur = (hxc - hxm) + sv * hzv(0);
-          pc = PY[0];
+          const double *Y = A + pY, *Z = A + pZ;
+          cur = fma(sv, Y[0] - Y[-1], (p0 - A[1]) + (p0 - A[-1])) + fma(sv, Z[0] - Z[-RS], (p0 - A[RS]) + (p0 - A[-RS]));
         } else {
-          const double hxm = j > 0 ? hxv(-1, 0) : 0.0, hxc = j < le ? hxv(0, 0) : gy.ge * hxm;
-          cur = -(sv * hyv(0)) - (hxc - hxm);
-          pc = PZ[0];
+          const int da = c == 1 ? RS : 1, db = c == 1 ? 1 : RS;
+          const double *B = A + (c == 1 ? pY : -pY), *X = A - (c == 1 ? pY : pZ);
+          cur = ((p0 - A[da]) + (p0 - A[-da])) + ((B[db] - B[0]) - (B[db - da] - B[-da])) + sv * fma(sv, p0, X[0] - X[db]);
         }
-        Q[i] = pal[DPAL_MAX * c + ((v >> 24) & 15u)] * pc + ca * cur;
-        pq += (double)(1u << ((v >> 22) & 3u)) * (pc * Q[i]);
+        Q[i] = fma(SMALL ? dreg[SMALL ? i : 0] : pal[DPAL_MAX * c + ((code[i / 8] >> (4 * (i % 8))) & 15u)], p0, ca * cur);
+        pq = fma(weight(v) * p0, Q[i], pq);
       }
     }
     sum_of(2, pq);
-    double dv[EPT];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) dv[i] = (it > 0 && (id[i] >> 28)) ? a.X[base + tid + nth * i] : 0.0;
     __syncthreads();
     const double al = rz / total(2);
     rr = 0.0;
 #pragma unroll
     for (int i = 0; i < EPT; ++i)
-      if (id[i] >> 28) {
-        const int e = tid + nth * i;
-        a.X[base + e] = dv[i] + al * P[e];
-        r[i] -= al * Q[i];
-        rr += (double)(1u << ((id[i] >> 22) & 3u)) * (r[i] * r[i]);
+      if (tid + nth * i < n) {
+        d[i] = fma(al, P[id[i] & 16383u], d[i]);
+        r[i] = fma(-al, Q[i], r[i]);
+        rr = fma(weight(id[i]) * r[i], r[i], rr);
       }
     ++it;
     sum_of(3, rr);
+    put_r();
+    if (!SMALL) ff = first(yf[0], yf[1]);
     __syncthreads();
     rr = total(3);
-    if (!(rr > thr) || it >= a.maxit) break;
   }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i)
+    if (tid + nth * i < n) a.X[base + tid + nth * i] = d[i];
   if (tid == 0) atomicMax(a.d.fl + FL_IT, it);
 }
 
@@ -669,11 +763,11 @@ struct CgPick {
   int threads, ept, zt, sm;
   size_t lds;
 };
-static CgPick cg_pick(const SectCG &a0, int &np, int &trows) {
+static CgPick cg_pick(const SectCG &a0, int &np, int &trows, int &ng) {
   CgPick k{};
   const SectDims &q = a0.q;
   int n = 0, ntile = 0;
-  trows = 0;
+  np = trows = ng = 0;
   for (int s = 0; s < 4; ++s) {
     const int py = s >> 1, pz = s & 1, lz = q.hz[0][pz], lze = q.hz[1][pz], CY = lz + lze;
     if (q.hy[0][py] < 1 || q.hy[1][py] < 1 || lz < 1 || lze < 1) return k;
@@ -682,10 +776,12 @@ static CgPick cg_pick(const SectCG &a0, int &np, int &trows) {
     const int mt = cdiv(q.hy[0][py], 16), nt = cdiv(CY, 16) + cdiv(lz, 16);
     ntile = std::max(ntile, mt * nt);
     trows = std::max(trows, CY + 16 * cdiv(lz, 16));
+    np = std::max(np, (2 * (lz + 2) + lze + 2) * (q.hy[0][py] + 2));
+    ng = std::max(ng, 3 * (q.hy[0][py] + lz) + 2 * (q.hy[1][py] + lze) + 2);
   }
-  np = (n + 1) / 2 * 2;
+  np = (np + 1) / 2 * 2;
   k.zt = cdiv(q.hz[0][0], 16);
-  const int epts[4] = {2, 4, 8, 11};
+  const int epts[6] = {2, 4, 6, 8, 10, 11};
   for (int e : epts) {
     const int th = 64 * std::max(4, cdiv(n, 64 * e));
     if (th > SECT_T) continue;
@@ -695,18 +791,20 @@ static CgPick cg_pick(const SectCG &a0, int &np, int &trows) {
   }
   if (!k.threads) return k;
   k.sm = cdiv(ntile, k.threads / 64);
-  k.lds = (size_t)np * sizeof(double) + (size_t)trows * (a0.yp + 4) * sizeof(float);
-  k.ok = k.zt <= 3 && k.sm <= 6 && k.lds + 1024 <= SECT_LDS_MAX;
-  k.sm = k.sm <= 3 ? 3 : 6;
+  const size_t nT = (size_t)trows * (a0.yp + 4);
+  k.lds = (size_t)np * sizeof(double) + nT * sizeof(float) + (size_t)ng * sizeof(unsigned) + (size_t)q.hz[0][0] * sizeof(float);
+  // 14 bits hold a place in P and in T
+  k.ok = k.zt <= 3 && k.sm <= 6 && np <= 16384 && nT <= 16384 && k.lds + 1024 <= SECT_LDS_MAX;
+  k.sm = k.sm <= 2 ? 2 : (k.sm <= 4 ? 4 : 6);
   return k;
 }
 bool sect_cg_fits(const SectCG &a) {
-  int np, tr;
-  return cg_pick(a, np, tr).ok;
+  int np, tr, ng;
+  return cg_pick(a, np, tr, ng).ok;
 }
 hipError_t launch_sect_cg(SectCG a, hipStream_t s) {
   if (g_rec) return hipErrorNotSupported;
-  const CgPick k = cg_pick(a, a.np, a.trows);
+  const CgPick k = cg_pick(a, a.np, a.trows, a.ng);
   if (!k.ok) return hipErrorInvalidValue;
   const dim3 grid(4 * a.q.nx), blk(k.threads);
 #define TDGL_CG(E, Z, M)                                              \
@@ -714,9 +812,11 @@ hipError_t launch_sect_cg(SectCG a, hipStream_t s) {
     TDGL_LAUNCH((k_sect_cg<E, Z, M>), grid, blk, k.lds, s, a);        \
     return hipGetLastError();                                         \
   }
-#define TDGL_CG_E(E) TDGL_CG(E, 1, 3) TDGL_CG(E, 2, 3) TDGL_CG(E, 3, 3) TDGL_CG(E, 1, 6) TDGL_CG(E, 2, 6) TDGL_CG(E, 3, 6)
-  TDGL_CG_E(2) TDGL_CG_E(4) TDGL_CG_E(8) TDGL_CG_E(11)
+#define TDGL_CG_Z(E, Z) TDGL_CG(E, Z, 2) TDGL_CG(E, Z, 4) TDGL_CG(E, Z, 6)
+#define TDGL_CG_E(E) TDGL_CG_Z(E, 1) TDGL_CG_Z(E, 2) TDGL_CG_Z(E, 3)
+  TDGL_CG_E(2) TDGL_CG_E(4) TDGL_CG_E(6) TDGL_CG_E(8) TDGL_CG_E(10) TDGL_CG_E(11)
 #undef TDGL_CG_E
+#undef TDGL_CG_Z
 #undef TDGL_CG
   return hipErrorInvalidValue;
 }

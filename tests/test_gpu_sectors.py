@@ -38,9 +38,10 @@ def _core(errs):
 
 # nodes per axis n = cells + 2 buf - 1: three nodes, odd and even counts, half extents at and past whole
 # 16-point tiles (31, 32 | 33, 34 nodes), one to three z tiles (half 16, 17, 33, 46), each elements-a-thread instance
-# (2, 4, 8, 11 x 512) and the largest sector (40 x 46 nodes)
+# (2, 4, 6, 8, 10, 11 x 512), more ghosts than threads (90 x 4 half nodes) and the largest sector (40 x 46 nodes)
 SIZES = [(2, 2, 2, 1), (5, 4, 3, 2), (9, 13, 8, 2), (20, 12, 28, 2), (17, 29, 30, 2), (33, 30, 31, 2), (34, 31, 29, 2), (12, 60, 28, 2),
-         (6, 28, 62, 2), (70, 66, 13, 2), (9, 76, 88, 2)]
+         (6, 28, 62, 2), (70, 66, 13, 2), (4, 92, 32, 2), (4, 120, 36, 2),
+         (4, 140, 44, 2), (3, 177, 5, 2), (9, 76, 88, 2)]
 
 
 @pytest.mark.parametrize("nx,ny,nz,buf", SIZES)
