@@ -162,7 +162,9 @@ typedef struct {
    * residual and solution sit around inner PCG solves in Float32 (their vectors, operator and the
    * folded Float32 preconditioner): each round solves A d = b − A x to pcg_inner_tol of its starting
    * residual, x += d, until ||b − A x|| <= pcg_tol ||b|| in FP64.  A captured cycle holds pcg_rounds
-   * rounds (1..16).  Needs pcg_f32 and the folded preconditioner; 0 keeps the reference's solver. */
+   * rounds (1..16).  Needs pcg_f32 and the folded preconditioner; 0 keeps the reference's solver.
+   * Where D is constant along x and mirror-symmetric the solve goes by sectors with or without it: every
+   * vector is then FP64, the tolerance holds in FP64, and pcg_rounds and pcg_inner_tol shape nothing. */
   int32_t pcg_refine;
   int32_t pcg_rounds;
   double pcg_inner_tol;

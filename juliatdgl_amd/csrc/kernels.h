@@ -719,6 +719,7 @@ struct SectCG {
   const double *pal;        // DPAL_MAX values a component
   double ca, a;             // curl-curl coefficient of the operator, a of the preconditioner
   double share;             // 1 / the number of sectors
+  double tight;             // the tolerance a sector stops at, of the solve's
   int maxit;
   int np, trows, ng;        // set by the launcher: P's places, T's rows, ghosts
 };

@@ -357,7 +357,7 @@ hipError_t launch_sect_inv(SectX p, hipStream_t s) {
 // (branches at every edge) and with d in global memory: 955 us there, now 812; 82 to 54 us on 100 x 52 x 28 nodes,
 // 126 to 78 on 83 x 49 x 21, 38 to 26 on 57 x 31 x 13.
 // The sums are FP64, in a fixed order: the same bits every time.
-// Where it stops: a sector's share of (SECT_TIGHT tol ||b||)² is half an equal share and half its share of
+// Where it stops: a sector's share of (tight tol ||b||)² is half an equal share and half its share of
 // the first residual, so the sectors' residuals together are below the tolerance, no sector iterates for
 // the others and one that holds almost nothing stops at once.  What is left is spread over the sectors and
 // not where the general iteration leaves it, and at the tolerance itself the fields came out up to nine
@@ -365,7 +365,6 @@ hipError_t launch_sect_inv(SectX p, hipStream_t s) {
 // cycles of 96x48x24 cells, 9.2e-8 against 2.8e-8 after one of 53x27x9); at an eighth of it they are nearer
 // (1.5e-8 on 53x27x9, 3.3e-8 against 2.0e-7 on 144x17x21, 9e-11 against 6e-10 with KWT) or as near (5.4e-9
 // against 2.5e-9 and 7.1e-9, full length and folded, on 96x48x24), for 15 % more iterations.
-constexpr double SECT_TIGHT = 0.125;
 // the same value, which the compiler does not know to be: what is derived from it is formed where it is used
 // and not kept in registers through the iterations
 __device__ __forceinline__ int fresh(int v) {
@@ -506,7 +505,7 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   put_r();
   __syncthreads();
   rr = total(0);
-  const double thr = SECT_TIGHT * SECT_TIGHT * 0.5 * tolb * tolb * (a.share + rr / a.d.sc[SC_RR]);
+  const double thr = a.tight * a.tight * 0.5 * tolb * tolb * (a.share + rr / a.d.sc[SC_RR]);
   const float imt = 1.0f / (float)mt;
   // one pass of the y products over the rows of T: rows x basis, in place
   struct First {

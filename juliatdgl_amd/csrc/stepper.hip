@@ -1500,6 +1500,11 @@ SectCG sect_cg(tdgl_handle *h) {
   a.ca = h->d.sxy / (h->d.dx * h->d.dy);
   a.a = h->d.a;
   a.share = 1.0 / (4.0 * h->sq.nx);
+  // k_sect_cg says why an eighth.  The last Float32 solve of a refinement leaves its residual well below the
+  // tolerance: 4.8e-10 to 3.9e-8 from a solution to the rounding over five grids of 16 to 64 cells across, where
+  // an eighth left 1.2e-9 to 1.5e-8 (up to five times more), a 32nd up to 1.2 times more and a 128th a ninth
+  // to a half as much or less, for four iterations more than an eighth
+  a.tight = h->d.pcg_refine ? 1.0 / 128 : 1.0 / 8;
   a.maxit = h->d.pcg_maxit;
   return a;
 }
@@ -1547,8 +1552,8 @@ int implicit_pcg_sect(tdgl_handle *h) {
 // kernel has written b = φₑ − θ and the partials of b·b, and scaled φ by D.  Eager: the host
 // reads the flags between batches of iterations.  Captured: `budget` iterations, each gated.
 int implicit_pcg(tdgl_handle *h) {
-  if (h->refine) return implicit_pcg_refine(h);
   if (h->sect) return implicit_pcg_sect(h);
+  if (h->refine) return implicit_pcg_refine(h);
   const tdgl_desc &d = h->d;
   const bool fast = d.pcg_fast || d.pcg_f32;
   const bool f32 = d.pcg_f32 != 0;
@@ -2486,13 +2491,32 @@ int general_setup(tdgl_handle *h) {
   return fold_setup(h);
 }
 
+// the refinement around Float32 inner solves: their vectors, D in Float32
+int refine_setup(tdgl_handle *h) {
+  const long long n = h->g.n;
+  Vec3f *fv[7] = {&h->f32v.d, &h->f32v.r, &h->f32v.z, &h->f32v.zold, &h->f32v.Pnew, &h->f32v.Pold, &h->f32v.Q};
+  for (Vec3f *v : fv)
+    for (int c = 0; c < 3; ++c) {
+      ALLOC(v->c[c], n);
+      CHK(upload_vec(h, v->c[c], std::vector<float>((size_t)n, 0.0f)));
+    }
+  for (int c = 0; c < 3; ++c) {
+    std::vector<double> dd((size_t)n);
+    CHK(hcopy(h, dd.data(), h->D[c], (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
+    ALLOC(h->D32[c], n);
+    CHK(upload_vec(h, h->D32[c], std::vector<float>(dd.begin(), dd.end())));
+    h->f32v.D[c] = h->D32[c];
+  }
+  return 0;
+}
+
 // The solve by sectors where it applies: the Float32-preconditioned PCG with the same coefficient in every
 // direction, D constant along x and equal to its mirror images in y and z on the unknowns (what
 // link_conductivity gives, implicit.jl:126-140), at most DPAL_MAX values of D a component, and a sector that
 // fits a workgroup.  The variables that shape the general iteration select it, as TDGL_HIP_SECT=0 does.
 int sect_setup(tdgl_handle *h) {
   const tdgl_desc &d = h->d;
-  if (d.field_mode != TDGL_FIELD_PCG || !d.pcg_f32 || d.pcg_refine) return 0;
+  if (d.field_mode != TDGL_FIELD_PCG || !d.pcg_f32) return 0;
   const char *off = std::getenv("TDGL_HIP_SECT");
   if (off && off[0] == '0') return 0;
   for (const char *v : {"TDGL_HIP_BUDGET", "TDGL_HIP_FOLD", "TDGL_HIP_QPLANE", "TDGL_HIP_QPARTS", "TDGL_HIP_ZQ_WAVES", "TDGL_HIP_PLANE",
@@ -2980,26 +3004,15 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
       }
     }
     CHK(sect_setup(h));
-    // a solve by sectors runs no general iteration (the tuner, which times it, sets it up then)
-    if (!h->sect) CHK(general_setup(h));
+    // a solve by sectors runs no general iteration (the tuner, which times it, sets it up then); a refinement
+    // is refused where that has no folds, whichever solves
+    if (!h->sect || d.pcg_refine) CHK(general_setup(h));
     if (d.field_mode == TDGL_FIELD_PCG && d.pcg_refine) {
-      // FP64 iterative refinement around Float32 inner solves: their vectors, D in Float32
       if (!h->fold || !d.pcg_f32 || !(d.pcg_fast || d.pcg_f32))
         return fail(TDGL_E_UNSUPPORTED, "the refinement needs the folded Float32 preconditioner (pcg_f32)");
       if (d.pcg_rounds < 1 || d.pcg_rounds > 16) return fail(TDGL_E_ARG, "pcg_rounds must be 1..16");
-      Vec3f *fv[7] = {&h->f32v.d, &h->f32v.r, &h->f32v.z, &h->f32v.zold, &h->f32v.Pnew, &h->f32v.Pold, &h->f32v.Q};
-      for (Vec3f *v : fv)
-        for (int c = 0; c < 3; ++c) {
-          ALLOC(v->c[c], n);
-          CHK(upload_vec(h, v->c[c], std::vector<float>((size_t)n, 0.0f)));
-        }
-      for (int c = 0; c < 3; ++c) {
-        std::vector<double> dd((size_t)n);
-        CHK(hcopy(h, dd.data(), h->D[c], (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-        ALLOC(h->D32[c], n);
-        CHK(upload_vec(h, h->D32[c], std::vector<float>(dd.begin(), dd.end())));
-        h->f32v.D[c] = h->D32[c];
-      }
+      // (a solve by sectors keeps its vectors in FP64 and needs none of them)
+      if (!h->sect) CHK(refine_setup(h));
       h->refine = true;
       h->rounds = d.pcg_rounds;
     }
@@ -3327,6 +3340,10 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
   h->sect = false;
   if (!h->general) {
     CHK(general_setup(h));
+    CHK(flush(h));
+  }
+  if (h->refine && !h->f32v.D[0]) {
+    CHK(refine_setup(h));
     CHK(flush(h));
   }
   PL(K_VEC, launch_copies(backup_list(h, true), h->s));

@@ -64,6 +64,20 @@ def test_sectors_match_the_general_iteration(nx, ny, nz, buf, monkeypatch):
     assert sa["rollbacks"] == 0
 
 
+def test_refinement_goes_by_sectors(monkeypatch):
+    """pcg_refine where the sectors apply, against its Float32 inner solves: the bound of
+    test_sectors_match_the_general_iteration."""
+    gr = Grid.make(33, 20, 9, dx=0.5, buf=2)
+    st = make_stepper(mgb2(), gr, box_masks(gr), sigma_vac=0.01, pcg_tol=1e-12, pcg_refine=True)
+    H, HJ = 0.03, st.selffield(0.3)
+    s0 = seeded_state(st.model, st.grid, st.masks, H, seed=4)
+    a, na, _ = _run(st, s0, H, HJ, 3, monkeypatch, True, calls=2)
+    b, nb, _ = _run(st, s0, H, HJ, 3, monkeypatch, False, calls=2)
+    assert (na, nb) == (1, 0)
+    errs = compare_states(a, b)
+    assert _core(errs) <= 1e-8, errs
+
+
 def test_sectors_repeat_to_the_bit(monkeypatch):
     """The sums of a sector run in a fixed order: two handles give the same bits, replayed or launched."""
     gr = Grid.make(33, 20, 9, dx=0.5, buf=2)
