@@ -186,6 +186,7 @@ struct GhostArgs {
   int nb;
 };
 hipError_t launch_ghosts(const Geo &g, const GhostArgs &a, hipStream_t s);
+hipError_t launch_curl_ghosts(const Geo &g, const CurlArgs &a, const GhostArgs &gh, uint64_t *tick, hipStream_t s);
 
 // device-to-device copies of up to 48 arrays in one launch
 struct CopyList {

@@ -158,7 +158,7 @@ struct tdgl_handle {
   int qplane = 1;              // TDGL_HIP_QPLANE=0: the quarter x-y transforms on k_plane_mf1 / k_plane_mf
   int qparts = 1;              // k_qplane's blocks a quarter plane (its m tiles split; TDGL_HIP_QPARTS)
   int zq_waves = 8;        // the quarter z pass: 4 or 8 waves a block on the vector ALUs, 0 on the matrix cores (k_zmodes_mf)
-  int merge = 1;           // the bands' stages and the field pass in common launches (TDGL_HIP_MERGE=0: each its own)
+  int merge = 1;           // the bands' stages and the field pass, and the curl and the ghosts, in common launches (TDGL_HIP_MERGE=0: each its own)
   int stxcd = 1;           // the stencil kernels' blocks in XCD runs (TDGL_HIP_STENCILXCD=0: the hardware's order)
   float *zqb[4] = {};      // its padded z bases (ZQ_BASES)
   float *zqmf = nullptr;   // the same as k_zmodes_mf's image (zmodes_mf_image floats)
@@ -1996,13 +1996,17 @@ int step_once(tdgl_handle *h) {
   ca.dydz = d.dy * d.dz;
   ca.dzdx = d.dz * d.dx;
   ca.dxdy = d.dx * d.dy;
-  PL(K_CURL, launch_curl(h->g, ca, h->s));
   GhostArgs ga{};
   for (int mu = 0; mu < d.nbands; ++mu) ga.F[mu] = h->F[mu];
   for (int c = 0; c < 3; ++c) ga.U[c] = h->U[c];
   ga.nb = d.nbands;
-  PL(K_GHOSTS, launch_ghosts(h->g, ga, h->s));
-  if (h->noise) PL(K_VEC, launch_noise_tick(h->nctr, h->s));
+  if (!g_rec && !h->prof && h->merge) {
+    LCHK(launch_curl_ghosts(h->g, ca, ga, h->noise ? h->nctr : nullptr, h->s));
+  } else {
+    PL(K_CURL, launch_curl(h->g, ca, h->s));
+    PL(K_GHOSTS, launch_ghosts(h->g, ga, h->s));
+    if (h->noise) PL(K_VEC, launch_noise_tick(h->nctr, h->s));
+  }
   // advance! (field.jl:248-263): F equals G outside the block, so G <- F is a swap
   for (int mu = 0; mu < d.nbands; ++mu) std::swap(h->G[mu], h->F[mu]);
   for (int c = 0; c < 3; ++c) {

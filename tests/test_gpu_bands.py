@@ -1,5 +1,5 @@
-"""The bands' stages and the field pass in common launches (k_bands) against a launch each
-(TDGL_HIP_MERGE=0): the same bits.  Needs a HIP device."""
+"""The bands' stages and the field pass (k_bands), and the curl, the ghosts and the noise clock
+(k_curl_ghosts), in common launches against a launch each (TDGL_HIP_MERGE=0): the same bits.  Needs a HIP device."""
 import numpy as np
 import pytest
 
