@@ -560,6 +560,7 @@ struct PcgArgs {
   Pcg32 f;           // the Float32 vectors (the refinement's inner solves)
   int gate_fl;       // resid32, xupdate: the flag that gates them
   int norm_only;     // resid32: only the partials of ||b − A x||²
+  int dx0;           // resid: D is constant along x (read at the first node of a row) and nothing needs Q
   int ovf_fl;        // finish: the flag that tells an unfinished solve (ACT[act_slot] when 0)
   // D as a palette (pap): byte k of Dcode[node] indexes Dpal[k] (FP64) / Dpal32[k] (Float32); null
   // without (each component of D takes at most DPAL_MAX values: the bar's σn and the padding's σvac)
@@ -571,6 +572,7 @@ constexpr int DPAL_MAX = 16;  // values per component of D in the palette (held 
 int pcg_box_blocks(const Geo &g, int kc);
 int box_kc(const Geo &g);
 hipError_t launch_pcg_start(const PcgArgs &a, hipStream_t s);    // nb, warm start or zero source
+hipError_t launch_bands_start(BandsArgs a, const PcgArgs &p, hipStream_t s);  // with a stage of the bands
 hipError_t launch_pcg_resid(const PcgArgs &a, hipStream_t s);    // Q = A x, r = b − Q, r·r
 hipError_t launch_pcg_p(const PcgArgs &a, hipStream_t s);        // β, P = z + βP, zold = z
 hipError_t launch_pcg_ap(const PcgArgs &a, hipStream_t s);       // Q = A P, p·Ap

@@ -539,22 +539,7 @@ hipError_t launch_field(const Geo &g, const FieldArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// A stage of every band that has one and, with the first stage, the field pass: launch-bound grids pay one
-// launch (about 5 us in a captured chain) where they paid one a band and one for the field.  The field's
-// blocks come first (they are the longer ones); each part keeps its own order of blocks on the XCDs, so
-// every node's and every partial's bits are those of the separate launches.  A step: 35.2 -> 28.4 us on 12x8x4
-// cells, 76 -> 61 us with three bands on 148x60x10, 219 -> 203 us (128x64x16, KWT), 249 -> 235 us (75x41x13, open);
-// 552 -> 538 us on 256x128x32, where the launches are bound by HBM, and never slower.
-__global__ void __launch_bounds__(256) k_bands(Geo g, BandsArgs a) {
-  int b = blockIdx.x;
-  if (b < a.fp) {
-    if (b >= a.fb) return;
-    const int nx = cdiv_d(g.Nx + 1, 64), ny = cdiv_d(g.Ny + 1, 4);
-    const int l = a.f.xcd ? xcd_run(b, a.fb) : b;
-    field_body(g, a.f, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, g.Nz + 1});
-    return;
-  }
-  b -= a.fp;
+__device__ __forceinline__ void bands_block(const Geo &g, const BandsArgs &a, int b) {
   const int q = b / a.sp;
   b -= q * a.sp;
   if (b >= a.sb) return;
@@ -563,17 +548,39 @@ __global__ void __launch_bounds__(256) k_bands(Geo g, BandsArgs a) {
   const int l = st.xcd ? xcd_run(b, a.sb) : b;
   stage_body(g, st, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, g.z2 - g.z1});
 }
+// the blocks of the parts, a.fb of the first given
+static void bands_blocks(const Geo &g, BandsArgs &a) {
+  const int ni = g.x2 - g.x1, nj = g.y2 - g.y1, nk = g.z2 - g.z1;
+  a.sb = (ni > 0 && nj > 0 && nk > 0) ? cdiv(ni, 64) * cdiv(nj, 4) * nk : 0;
+  a.fp = 8 * cdiv(a.fb, 8);
+  a.sp = 8 * std::max(1, cdiv(a.sb, 8));
+}
+
+// A stage of every band that has one and, with the first stage, the field pass: launch-bound grids pay one
+// launch (about 5 us in a captured chain) where they paid one a band and one for the field.  The field's
+// blocks come first (they are the longer ones); each part keeps its own order of blocks on the XCDs, so
+// every node's and every partial's bits are those of the separate launches.  A step: 35.2 -> 28.4 us on 12x8x4
+// cells, 76 -> 61 us with three bands on 148x60x10, 219 -> 203 us (128x64x16, KWT), 249 -> 235 us (75x41x13, open);
+// 552 -> 538 us on 256x128x32, where the launches are bound by HBM, and never slower.
+__global__ void __launch_bounds__(256) k_bands(Geo g, BandsArgs a) {
+  const int b = blockIdx.x;
+  if (b < a.fp) {
+    if (b >= a.fb) return;
+    const int nx = cdiv_d(g.Nx + 1, 64), ny = cdiv_d(g.Ny + 1, 4);
+    const int l = a.f.xcd ? xcd_run(b, a.fb) : b;
+    field_body(g, a.f, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, g.Nz + 1});
+    return;
+  }
+  bands_block(g, a, b - a.fp);
+}
 static_assert(sizeof(Geo) + sizeof(BandsArgs) <= 4096, "kernel arguments");
 
 hipError_t launch_bands(const Geo &g, BandsArgs a, hipStream_t s) {
   if (g_rec) return hipErrorNotSupported;
   if (a.ns < 0 || a.ns > TDGL_MAX_BANDS) return hipErrorInvalidValue;
   if (a.field && a.f.part && field_blocks(g) > MAX_PART) return hipErrorInvalidValue;
-  const int ni = g.x2 - g.x1, nj = g.y2 - g.y1, nk = g.z2 - g.z1;
   a.fb = a.field ? field_blocks(g) : 0;
-  a.sb = (ni > 0 && nj > 0 && nk > 0) ? cdiv(ni, 64) * cdiv(nj, 4) * nk : 0;
-  a.fp = 8 * cdiv(a.fb, 8);
-  a.sp = 8 * std::max(1, cdiv(a.sb, 8));
+  bands_blocks(g, a);
   const int nb = a.fp + a.ns * a.sp;
   if (nb == 0) return hipSuccess;
   TDGL_LAUNCH(k_bands, dim3(nb), dim3(64, 4, 1), 0, s, g, a);
@@ -3388,18 +3395,21 @@ struct BoxIdx {
 // With `xcd`, the hardware's block order is taken through xcd_run: each XCD receives a contiguous
 // run of the (x, y, level) order, so that the neighbours whose halos a stencil block shares mostly
 // sit behind the same L2.  The block's partial slot is its place in that order either way.
-__device__ __forceinline__ BoxIdx box_idx(const Geo &g, int kc, int xcd) {
+__device__ __forceinline__ BoxIdx box_at(const Geo &g, int kc, int b) {
   const int gx = cdiv_d(g.Nx - 1, 64), gy = cdiv_d(g.Ny - 1, 4);
-  const int b = xcd ? xcd_run((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
   BoxIdx r;
   r.bid = b;
   const int bx = b % gx, by = (b / gx) % gy, bz = b / (gx * gy);
-  r.i = 2 + bx * 64 + (int)(threadIdx.x & 63);
-  r.j = 2 + by * 4 + (int)(threadIdx.x >> 6);
+  const int t = (int)(threadIdx.x + threadIdx.y * blockDim.x);
+  r.i = 2 + bx * 64 + (t & 63);
+  r.j = 2 + by * 4 + (t >> 6);
   r.k = 2 + bz * kc;
   r.nk = min(kc, g.Nz - 1 - bz * kc);
   r.c = g.at(r.i, r.j, r.k);
   return r;
+}
+__device__ __forceinline__ BoxIdx box_idx(const Geo &g, int kc, int xcd) {
+  return box_at(g, kc, xcd ? xcd_run((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x);
 }
 // level q of a block (its k + q)
 __device__ __forceinline__ BoxIdx box_level(const Geo &g, BoxIdx b, int q) {
@@ -3478,7 +3488,8 @@ __device__ __forceinline__ void apply3(const PcgArgs &a, const double *P0, const
                                        int j, int k, int c, double q[3], double pc[3]) {
   double v[NSTEN];
   gather24(P0, P1, P2, c, a.g.px, a.g.px * a.g.py, v);
-  const double dv[3] = {a.D[0][c], a.D[1][c], a.D[2][c]};
+  const int cd = a.dx0 ? c - i + 2 : c;
+  const double dv[3] = {a.D[0][cd], a.D[1][cd], a.D[2][cd]};
   apply3v<double>(a, v, dv, i, j, k, q);
   pc[0] = v[P0C];
   pc[1] = v[P1C];
@@ -3493,10 +3504,7 @@ __device__ __forceinline__ int box_load_c(const Geo &g, const BoxIdx &b) { retur
 
 // _pcg_zero_update! (implicit.jl:251-271) when the source is zero, else the warm start of
 // _implicit_curl_fast! (:391-402); nb from the field kernel's partials
-__global__ void __launch_bounds__(RED_T) k_pcg_start(PcgArgs a) {
-  __shared__ double sh[8];
-  const int tid = threadIdx.x;
-  const BoxIdx b0 = box_idx(a.g, a.kc, a.xcd);
+__device__ __forceinline__ void pcg_start_body(const PcgArgs &a, const BoxIdx b0, double *sh, int tid) {
   const bool live = box_live(a.g, b0);
   // the first level's values are requested before the partials are summed
   const int cl = box_load_c(a.g, b0);
@@ -3537,6 +3545,35 @@ __global__ void __launch_bounds__(RED_T) k_pcg_start(PcgArgs a) {
     }
   }
 }
+__global__ void __launch_bounds__(RED_T) k_pcg_start(PcgArgs a) {
+  __shared__ double sh[8];
+  pcg_start_body(a, box_idx(a.g, a.kc, a.xcd), sh, threadIdx.x);
+}
+
+// A later stage of the bands with the start of the solve, whose blocks come first: the start waits for the
+// field's partials only, which the first stage's launch wrote.
+// A step: 79.4 -> 76.0 us (57 x 31 x 13 nodes), 168 -> 164 (132 x 68 x 20), 1433 -> 1405 (272 x 144 x 48, with what
+// k_pcg_resid no longer moves: 66 -> 51 us there without Q and with one D a row).
+__global__ void __launch_bounds__(256) k_bands_start(BandsArgs a, PcgArgs p) {
+  __shared__ double sh[8];
+  int b = blockIdx.x;
+  if (b < a.fp) {
+    if (b < a.fb) pcg_start_body(p, box_at(p.g, p.kc, p.xcd ? xcd_run(b, a.fb) : b), sh, (int)(threadIdx.x + 64 * threadIdx.y));
+    return;
+  }
+  bands_block(p.g, a, b - a.fp);
+}
+static_assert(sizeof(BandsArgs) + sizeof(PcgArgs) <= 4096, "kernel arguments");
+hipError_t launch_bands_start(BandsArgs a, const PcgArgs &p, hipStream_t s) {
+  if (g_rec) return hipErrorNotSupported;
+  if (a.ns < 0 || a.ns > TDGL_MAX_BANDS || a.field || p.kc < 1 || p.kc > p.g.Nz - 1) return hipErrorInvalidValue;
+  const Geo &g = p.g;
+  a.fb = pcg_box_blocks(g, p.kc);
+  if (a.fb > MAX_PART) return hipErrorInvalidValue;
+  bands_blocks(g, a);
+  TDGL_LAUNCH(k_bands_start, dim3(a.fp + a.ns * a.sp), dim3(64, 4, 1), 0, s, a, p);
+  return hipGetLastError();
+}
 
 // the start of the iterations: Q = A x, r = b − Q and the partials of r·r (implicit.jl:407-410)
 __global__ void __launch_bounds__(RED_T) k_pcg_resid(PcgArgs a) {
@@ -3553,7 +3590,7 @@ __global__ void __launch_bounds__(RED_T) k_pcg_resid(PcgArgs a) {
       apply3(a, a.x.c[0], a.x.c[1], a.x.c[2], b.i, b.j, b.k, b.c, qv, pc);
       for (int comp = 0; comp < 3; ++comp) {
         if (!a.rg.in(comp, b.i, b.j, b.k)) continue;
-        a.Q.c[comp][b.c] = qv[comp];
+        if (!a.dx0) a.Q.c[comp][b.c] = qv[comp];
         const double rv = bv[comp] - qv[comp];
         a.r.c[comp][b.c] = rv;
         s += rv * rv;

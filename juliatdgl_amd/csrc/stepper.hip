@@ -744,8 +744,10 @@ bool bands_merge(const tdgl_handle *h) {
   return true;
 }
 
+PcgArgs pcg_start_args(tdgl_handle *h);
+
 // update_bands! (bands.jl:330-346) of all bands side by side, stage after stage, the field pass with the first
-int update_bands_merged(tdgl_handle *h, const FieldArgs &fa) {
+int update_bands_merged(tdgl_handle *h, const FieldArgs &fa, bool &started) {
   const tdgl_desc &d = h->d;
   const cplx *A[TDGL_MAX_BANDS], *B[TDGL_MAX_BANDS];
   int smax = 1;
@@ -768,6 +770,11 @@ int update_bands_merged(tdgl_handle *h, const FieldArgs &fa) {
       ba.st[ba.ns++] = rkl_stage(h, mu, ns, j, A[mu], B[mu], C);
       A[mu] = B[mu];
       B[mu] = C;
+    }
+    if (j == 2 && d.field_mode == TDGL_FIELD_PCG) {
+      LCHK(launch_bands_start(ba, pcg_start_args(h), h->s));
+      started = true;
+      continue;
     }
     LCHK(launch_bands(h->g, ba, h->s));
   }
@@ -1369,6 +1376,16 @@ int pcg32_iteration(tdgl_handle *h, int q) {
   return sep_folded_tail(h, o, nullptr, cv);
 }
 
+// the start of a solve: ||b||, the extrapolated guess
+PcgArgs pcg_start_args(tdgl_handle *h) {
+  PcgArgs a = pcg_args(h);
+  a.warm = h->warm;
+  a.extrap = h->d.pcg_extrap && h->d.pcg_fast;
+  a.have2 = h->have2;
+  a.nparts_in = field_blocks(h->g);
+  return a;
+}
+
 // One round of the refinement: r32 = b − A x (FP64), the round's check and the fold of r32, the
 // Float32 solve A d = r32 from d = 0 (its first preconditioner, then `budget` gated iterations, or
 // eagerly while active), x += d.  Round 0 is gated by NZ, the others by OACT.
@@ -1413,16 +1430,12 @@ int refine_round(tdgl_handle *h, int round) {
 // limit.  Eager: rounds while the check says so.  Captured: `rounds` rounds, each with `budget`
 // gated inner iterations, then a last FP64 check; a solve still above the tolerance overflows
 // (the cycle is rolled back and stepped eagerly).
-int implicit_pcg_refine(tdgl_handle *h) {
+int implicit_pcg_refine(tdgl_handle *h, bool started) {
   const tdgl_desc &d = h->d;
   const bool extrap = d.pcg_extrap && d.pcg_fast;
   const int *nz = h->pd.fl + FL_NZ;
-  PcgArgs a = pcg_args(h);
-  a.warm = h->warm;
-  a.extrap = extrap;
-  a.have2 = h->have2;
-  a.nparts_in = field_blocks(h->g);
-  PL(K_VEC, launch_pcg_start(a, h->s));
+  PcgArgs a = pcg_start_args(h);
+  if (!started) PL(K_VEC, launch_pcg_start(a, h->s));
   if (!h->warm) {  // cold start: x = M⁻¹ b in Float64
     SepOut o{&h->x, false, 0};
     CHK(sep_solve(h, h->B, o, nz, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
@@ -1513,22 +1526,19 @@ SectCG sect_cg(tdgl_handle *h) {
 // iteration's, the residual to the sectors, the flexible CG of every sector to its own convergence in one
 // launch, the solution's increment back (x += d, φ = θ + x).  Nothing is gated by a budget of iterations,
 // and the host waits for nothing.
-int implicit_pcg_sect(tdgl_handle *h) {
+int implicit_pcg_sect(tdgl_handle *h, bool started) {
   const tdgl_desc &d = h->d;
   const bool extrap = d.pcg_extrap && d.pcg_fast;
   const int *nz = h->pd.fl + FL_NZ;
-  PcgArgs a = pcg_args(h);
-  a.warm = h->warm;
-  a.extrap = extrap;
-  a.have2 = h->have2;
-  a.nparts_in = field_blocks(h->g);
-  PL(K_VEC, launch_pcg_start(a, h->s));
+  PcgArgs a = pcg_start_args(h);
+  if (!started) PL(K_VEC, launch_pcg_start(a, h->s));
   if (!h->warm) {  // cold start: x = M⁻¹ b in Float64
     SepOut o{&h->x, false, 0};
     CHK(sep_solve(h, h->B, o, nz, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
   }
   h->have2 = h->warm && extrap;
   h->warm = true;
+  a.dx0 = 1;
   PL(K_APPLYA, launch_pcg_resid(a, h->s));
   SectX f = sect_x(h, false);
   for (int c = 0; c < 3; ++c) f.v[c] = node_view(h, h->r.c[c]);
@@ -1551,21 +1561,17 @@ int implicit_pcg_sect(tdgl_handle *h) {
 // implicit_curl!(s, ::PCGSolver) / _implicit_curl_fast! (implicit.jl:279-446), after the field
 // kernel has written b = φₑ − θ and the partials of b·b, and scaled φ by D.  Eager: the host
 // reads the flags between batches of iterations.  Captured: `budget` iterations, each gated.
-int implicit_pcg(tdgl_handle *h) {
-  if (h->sect) return implicit_pcg_sect(h);
-  if (h->refine) return implicit_pcg_refine(h);
+int implicit_pcg(tdgl_handle *h, bool started) {
+  if (h->sect) return implicit_pcg_sect(h, started);
+  if (h->refine) return implicit_pcg_refine(h, started);
   const tdgl_desc &d = h->d;
   const bool fast = d.pcg_fast || d.pcg_f32;
   const bool f32 = d.pcg_f32 != 0;
   const bool extrap = d.pcg_extrap && d.pcg_fast;
   const bool flexible = fast && f32;
   const int *nz = h->pd.fl + FL_NZ;
-  PcgArgs a = pcg_args(h);
-  a.warm = h->warm;
-  a.extrap = fast && extrap;
-  a.have2 = h->have2;
-  a.nparts_in = field_blocks(h->g);
-  PL(K_VEC, launch_pcg_start(a, h->s));
+  PcgArgs a = pcg_start_args(h);
+  if (!started) PL(K_VEC, launch_pcg_start(a, h->s));
   if (!h->warm) {  // cold start: x = M⁻¹ b in Float64
     SepOut o{&h->x, false, 0};
     CHK(sep_solve(h, h->B, o, nz, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
@@ -1922,6 +1928,7 @@ int step_once(tdgl_handle *h) {
   if (d.selffield_bc == TDGL_BC_OPEN) CHK(open_update(h));
   if (d.qp_mode != TDGL_QP_NONE) CHK(qp_potential(h));
   const bool merge = bands_merge(h);
+  bool started = false;
   if (!merge) CHK(update_bands(h));
   FieldArgs fa{};
   fa.xcd = h->stxcd;
@@ -1960,14 +1967,14 @@ int step_once(tdgl_handle *h) {
     fa.nz = noise_args(h);
   }
   if (merge)
-    CHK(update_bands_merged(h, fa));
+    CHK(update_bands_merged(h, fa, started));
   else
     PL(K_FIELD, launch_field(h->g, fa, h->s));
   if (d.field_mode == TDGL_FIELD_SEPARABLE) {
     SepOut o{nullptr, true, 0};
     CHK(sep_solve(h, h->B, o, nullptr, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
   } else if (d.field_mode == TDGL_FIELD_PCG) {
-    CHK(implicit_pcg(h));
+    CHK(implicit_pcg(h, started));
   }
   CurlArgs ca{};
   ca.xcd = h->stxcd;
