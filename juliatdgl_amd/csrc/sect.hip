@@ -351,11 +351,12 @@ hipError_t launch_sect_inv(SectX p, hipStream_t s) {
 // L2, its first groups asked for before the barrier), then each wave takes 16 y modes through the z transform,
 // the projector and the inverse z transform in registers (a forward tile leaves in a lane the modes its inverse
 // takes as operand), then the inverse y products.
-// Bound: on 272 x 144 x 48 nodes the matrix products of an iteration are 11.8 k cycles of the 42 k it takes a
-// block there (two share a CU), the rest LDS reads of the stencil, FP64 sums and what ten elements a thread spill
-// past 128 registers; on small planes the chain of ten barriers an iteration, 10 k cycles.  Before the ghosts
-// (branches at every edge) and with d in global memory: 955 us there, now 812; 82 to 54 us on 100 x 52 x 28 nodes,
-// 126 to 78 on 83 x 49 x 21, 38 to 26 on 57 x 31 x 13.
+// Bound: on 272 x 144 x 48 nodes the matrix products of an iteration are 11.8 k cycles of the 38 k it takes a
+// block there (two share a CU), the rest the issue of the stencil's LDS reads, FP64 sums and what ten elements a
+// thread spill past 128 registers; on small planes the issue of the instructions of two blocks and ten barriers an
+// iteration, 7 to 13 k cycles.  Branches at every edge and d in global memory at first: 955 us on those nodes, 82 us
+// on 100 x 52 x 28, 126 us on 83 x 49 x 21, 38 us on 57 x 31 x 13; with the ghosts 812, 54, 78 and 26; with
+// the y tiles known when compiled (MT; 0: any) 762, 46, 65 and 22, and 75 to 63 on 132 x 68 x 20.
 // The sums are FP64, in a fixed order: the same bits every time.
 // Where it stops: a sector's share of (tight tol ||b||)² is half an equal share and half its share of
 // the first residual, so the sectors' residuals together are below the tolerance, no sector iterates for
@@ -389,7 +390,7 @@ __device__ __forceinline__ double wave_sum63(double v) {
   return dpp_add<0x143, 0xc>(v);
 }
 
-template <int EPT, int ZT, int SM>
+template <int EPT, int ZT, int SM, int MT>
 __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   if (!sect_active(a.d)) return;
   extern __shared__ __align__(16) unsigned char cg_smem[];
@@ -406,8 +407,8 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   double *P = (double *)cg_smem;
   float *T = (float *)(P + a.np);
   unsigned *G = (unsigned *)(T + a.trows * (a.yp + 4));
-  const int ST = a.yp + 4, CY = lz + lze;
-  const int mt = (ly + 15) / 16, nt1 = (CY + 15) / 16, nt2 = (lz + 15) / 16, ntile = mt * (nt1 + nt2);
+  const int yp = MT ? 16 * MT : a.yp, ST = (MT ? 16 * MT : a.yp) + 4, CY = lz + lze;
+  const int mt = MT ? MT : (ly + 15) / 16, nt1 = (CY + 15) / 16, nt2 = (lz + 15) / 16, ntile = mt * (nt1 + nt2);
   // P: component c at pc[c] + (k + 1) RS + j + 1, a ring of ghost places around each
   const int RS = ly + 2, pY = (lz + 2) * RS, pZ = 2 * pY;
   auto pat = [&](int c, int j, int k) { return (c == 0 ? 0 : (c == 1 ? pY : pZ)) + (k + 1) * RS + j + 1; };
@@ -513,7 +514,7 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   };
   auto tile = [&](int t, int &m, int &nt) __attribute__((always_inline)) {
     const int tt = w + nw * t;
-    nt = __builtin_amdgcn_readfirstlane((int)(((float)tt + 0.5f) * imt));
+    nt = MT ? tt / max(MT, 1) : __builtin_amdgcn_readfirstlane((int)(((float)tt + 0.5f) * imt));
     m = tt - nt * mt;
     return tt < ntile;
   };
@@ -521,24 +522,25 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
     First f{v4f{0, 0, 0, 0}, v4f{0, 0, 0, 0}};
     int m, nt;
     if (tile(0, m, nt)) {
-      const float *A = (nt < nt1 ? BV : BU) + 16 * m * a.yp + fresh(lr) * a.yp + 4 * lk;
+      const float *A = (nt < nt1 ? BV : BU) + 16 * m * yp + fresh(lr) * yp + 4 * lk;
       f.a = *(const v4f *)A;
       f.b = *(const v4f *)(A + 16 * min(1, mt - 1));
     }
     return f;
   };
   auto ypass = [&](const float *BV, const float *BU, const First f) __attribute__((always_inline)) {
-    const int la = fresh(lr) * a.yp + 4 * lk, lb = fresh(lr) * ST + 4 * lk;
+    const int la = fresh(lr) * yp + 4 * lk, lb = fresh(lr) * ST + 4 * lk;
     v4f acc[SM];
 #pragma unroll
     for (int t = 0; t < SM; ++t) {
       acc[t] = v4f{0, 0, 0, 0};
       int m, nt;
       if (tile(t, m, nt)) {
-        const float *A = (nt < nt1 ? BV : BU) + 16 * m * a.yp + la;
+        const float *A = (nt < nt1 ? BV : BU) + 16 * m * yp + la;
         const float *B = T + (nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1)) * ST + lb;
         // the basis comes through L2: two groups of sixteen ahead
         v4f av = t ? *(const v4f *)A : f.a, an = t ? *(const v4f *)(A + 16 * min(1, mt - 1)) : f.b;
+#pragma unroll(MT ? MT : 1)
         for (int g = 0; g < mt; ++g) {
           const v4f aq = *(const v4f *)(A + 16 * min(g + 2, mt - 1));
           const v4f bv = *(const v4f *)(B + 16 * g);
@@ -573,6 +575,20 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   if (ZREG)
 #pragma unroll
     for (int i = 0; i < 4; ++i) zr[i] = zfrag(i, 0, 0, l);
+  // the projector's factors, one tile a wave
+  constexpr bool PREG = ZREG && EPT <= 2 && MT > 0 && MT <= 4;
+  float pf[4] = {}, pk[4] = {}, pk2 = 0.0f;
+  if (PREG) {
+    const int my = 2 * (16 * w + lr) + py;
+    const float k1 = a.sfx[mx], af = (float)a.a;
+    pk2 = my < q.ny ? a.sfy[my] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int mz = 2 * (4 * lk + e) + pz;
+      pk[e] = my < q.ny && mz < q.nz ? a.sfz[mz] : 0.0f;
+      pf[e] = 1.0f / (1.0f + af * (k1 * k1 + pk2 * pk2 + pk[e] * pk[e]));
+    }
+  }
   double dreg[SMALL ? EPT : 1] = {};
   if (SMALL)
 #pragma unroll
@@ -624,7 +640,7 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
       }
       {
         const int my = 2 * (16 * m + lr) + py;
-        const float k1 = a.sfx[mx], k2 = my < q.ny ? a.sfy[my] : 0.0f, af = (float)a.a;
+        const float k1 = a.sfx[mx], k2 = PREG ? pk2 : (my < q.ny ? a.sfy[my] : 0.0f), af = (float)a.a;
         const bool live = my < q.ny, hx = mx > 0, hy = my > 0;
 #pragma unroll
         for (int t = 0; t < ZT; ++t)
@@ -634,7 +650,8 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
             // without the mode is zero
             const int mz = 2 * (16 * t + 4 * lk + e) + pz;
             const bool in = live && mz < q.nz;
-            const float k3 = in ? kz[16 * t + 4 * lk + e] : 0.0f, f = 1.0f / (1.0f + af * (k1 * k1 + k2 * k2 + k3 * k3));
+            const float k3 = PREG ? pk[e] : (in ? kz[16 * t + 4 * lk + e] : 0.0f);
+            const float f = PREG ? pf[e] : 1.0f / (1.0f + af * (k1 * k1 + k2 * k2 + k3 * k3));
             const float x1 = hx ? acc[0][t][e] : 0.0f, y1 = hy ? acc[1][t][e] : 0.0f, z1 = mz > 0 ? acc[2][t][e] : 0.0f;
             const float dd = af * (k1 * x1 + k2 * y1 + k3 * z1);
             acc[0][t][e] = hx ? f * (x1 + k1 * dd) : 0.0f;
@@ -794,7 +811,6 @@ static CgPick cg_pick(const SectCG &a0, int &np, int &trows, int &ng) {
   k.lds = (size_t)np * sizeof(double) + nT * sizeof(float) + (size_t)ng * sizeof(unsigned) + (size_t)q.hz[0][0] * sizeof(float);
   // 14 bits hold a place in P and in T
   k.ok = k.zt <= 3 && k.sm <= 6 && np <= 16384 && nT <= 16384 && k.lds + 1024 <= SECT_LDS_MAX;
-  k.sm = k.sm <= 2 ? 2 : (k.sm <= 4 ? 4 : 6);
   return k;
 }
 bool sect_cg_fits(const SectCG &a) {
@@ -806,12 +822,17 @@ hipError_t launch_sect_cg(SectCG a, hipStream_t s) {
   const CgPick k = cg_pick(a, a.np, a.trows, a.ng);
   if (!k.ok) return hipErrorInvalidValue;
   const dim3 grid(4 * a.q.nx), blk(k.threads);
-#define TDGL_CG(E, Z, M)                                              \
-  if (k.ept == E && k.zt == Z && k.sm == M) {                         \
-    TDGL_LAUNCH((k_sect_cg<E, Z, M>), grid, blk, k.lds, s, a);        \
-    return hipGetLastError();                                         \
+#define TDGL_CG(E, Z, M, T)                                              \
+  if (k.ept == E && k.zt == Z && k.sm <= M && (T == 0 || a.yp == 16 * T)) { \
+    TDGL_LAUNCH((k_sect_cg<E, Z, M, T>), grid, blk, k.lds, s, a);        \
+    return hipGetLastError();                                            \
   }
-#define TDGL_CG_Z(E, Z) TDGL_CG(E, Z, 2) TDGL_CG(E, Z, 4) TDGL_CG(E, Z, 6)
+  // the y tiles known when compiled, for the planes that are near square
+  TDGL_CG(2, 1, 2, 1) TDGL_CG(2, 1, 2, 2) TDGL_CG(2, 1, 2, 3) TDGL_CG(2, 1, 2, 4) TDGL_CG(4, 1, 2, 2) TDGL_CG(4, 1, 2, 3)
+  TDGL_CG(4, 1, 2, 4) TDGL_CG(4, 1, 2, 5) TDGL_CG(6, 1, 2, 3) TDGL_CG(6, 1, 2, 5)
+  TDGL_CG(6, 1, 2, 4) TDGL_CG(2, 2, 2, 1) TDGL_CG(4, 2, 2, 2) TDGL_CG(6, 2, 2, 2) TDGL_CG(6, 2, 4, 3) TDGL_CG(8, 2, 4, 3)
+  TDGL_CG(10, 2, 4, 4) TDGL_CG(10, 2, 4, 5)
+#define TDGL_CG_Z(E, Z) TDGL_CG(E, Z, 2, 0) TDGL_CG(E, Z, 6, 0)
 #define TDGL_CG_E(E) TDGL_CG_Z(E, 1) TDGL_CG_Z(E, 2) TDGL_CG_Z(E, 3)
   TDGL_CG_E(2) TDGL_CG_E(4) TDGL_CG_E(6) TDGL_CG_E(8) TDGL_CG_E(10) TDGL_CG_E(11)
 #undef TDGL_CG_E
