@@ -211,7 +211,8 @@ typedef struct {
   int32_t pcg_budget;   /* PCG iterations per solve in the captured cycle (a solve by sectors runs to its end on
                            the device whatever they are: what the general iteration would hold) */
   int64_t captures;     /* graphs captured and instantiated (the last four are kept and replayed) */
-  int32_t folded;       /* 1: the Float32 preconditioner runs its parity-folded transforms */
+  int32_t folded;       /* 1: the Float32 preconditioner (or the separable solve) runs its parity-folded
+                         * transforms; 2: the separable solve goes by sectors */
 } tdgl_stats;
 
 typedef struct tdgl_handle tdgl_handle;

@@ -634,7 +634,7 @@ hipError_t launch_meter_finish(const MeterArgs &a, double *rec, double *rung, hi
 // off[r+1]-1 of a 1D grid, which it takes as its own grid of dims[3r] x dims[3r+1] x dims[3r+2]
 // blocks (the grid its single-run launch would have), with its own Geo and argument struct.
 enum { BK_STAGE = 0, BK_FIELD, BK_TX, BK_TX2, BK_CURL, BK_GHOSTS, BK_METER, BK_METERFIN, BK_PLANE, BK_ZMODES, BK_FOLD, BK_UNFOLD,
-       BK_ZMODESQ, BK_QPLANE, BK_N };
+       BK_ZMODESQ, BK_QPLANE, BK_SECTF, BK_SECTS, BK_SECTI, BK_N };
 struct BatchTab {
   const int *off;    // n + 1 block offsets
   const int *dims;   // 3 per run
@@ -642,6 +642,30 @@ struct BatchTab {
   const void *args;  // per run: the kind's argument struct
   int n;
 };
+// A kernel body's block: its place in its run's grid and that grid's size
+struct Blk {
+  int x, y, z, nx, ny, nz;
+};
+// The run of a batched launch's block b (the last r with off[r] <= b: runs of no blocks are
+// passed over) and the block's place in that run's grid
+struct BatchIdx {
+  int r;
+  Blk b;
+};
+__device__ __forceinline__ BatchIdx batch_idx(const BatchTab &t, int b = -1) {
+  if (b < 0) b = blockIdx.x;
+  int lo = 0, hi = t.n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (t.off[mid] <= b)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  const int l = b - t.off[lo];
+  const int nx = t.dims[3 * lo], ny = t.dims[3 * lo + 1], nz = t.dims[3 * lo + 2];
+  return BatchIdx{lo, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, nz}};
+}
 struct MeterFinArgs {
   MeterArgs a;
   double *rec, *rung;
@@ -661,6 +685,8 @@ struct Recorder {
   std::vector<BatchRec> recs;
 };
 extern thread_local Recorder *g_rec;
+hipError_t record(int kind, const Geo &g, const void *args, size_t bytes, int variant = 0, bool has_grid = false,
+                  dim3 grid = dim3(0, 0, 0), size_t lds = 0);
 size_t batch_args_size(int kind);
 dim3 batch_grid(int kind, const Geo &g, const void *args);  // the single-run grid of a record
 hipError_t launch_batch(int kind, int variant, size_t lds, const BatchTab &t, int blocks, hipStream_t s);
@@ -703,6 +729,7 @@ struct SectX {
   int jg, kg;               // set by the launcher
 };
 bool sect_x_fits(const SectX &p);
+int sect_x_blocks(const SectX &p);
 hipError_t launch_sect_fwd(SectX p, hipStream_t s);
 hipError_t launch_sect_inv(SectX p, hipStream_t s);
 // the flexible CG of every sector, each in one block (k_sect_cg): A d = r from d = 0
@@ -727,6 +754,21 @@ struct SectCG {
   int np, trows, ng;        // set by the launcher: P's places, T's rows, ghosts
 };
 bool sect_cg_fits(const SectCG &a);
+// the separable solve of every sector in FP64 (k_sect_sep), in place
+struct SectSep {
+  SectDims q;
+  double *S;
+  const double *s[3];       // singular values
+  // half-size bases as SectCG's, in FP64
+  const double *yb[2][2][2], *zb[2][2][2];
+  int yp, zp;
+  double a;
+  int trows;                // set by the launcher
+};
+bool sect_sep_fits(const SectSep &a);
+hipError_t launch_sect_sep(SectSep a, hipStream_t s);
+hipError_t launch_sect_inv_sep(SectX p, hipStream_t s);  // φ = θ + x
+hipError_t launch_sect_batch(int kind, int variant, size_t lds, const BatchTab &t, int blocks, hipStream_t s);
 hipError_t launch_sect_cg(SectCG a, hipStream_t s);
 hipError_t launch_pcg_cycle_reset(PcgDev d, hipStream_t s);
 

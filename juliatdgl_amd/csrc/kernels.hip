@@ -11,8 +11,7 @@ namespace tdgl {
 thread_local ProfPair *prof_pair = nullptr;
 thread_local Recorder *g_rec = nullptr;
 
-static hipError_t record(int kind, const Geo &g, const void *args, size_t bytes, int variant = 0, bool has_grid = false,
-                         dim3 grid = dim3(0, 0, 0), size_t lds = 0) {
+hipError_t record(int kind, const Geo &g, const void *args, size_t bytes, int variant, bool has_grid, dim3 grid, size_t lds) {
   BatchRec r;
   r.kind = kind;
   r.variant = variant;
@@ -25,10 +24,6 @@ static hipError_t record(int kind, const Geo &g, const void *args, size_t bytes,
   return hipSuccess;
 }
 
-// A kernel body's block: its place in its run's grid and that grid's size
-struct Blk {
-  int x, y, z, nx, ny, nz;
-};
 __device__ __forceinline__ Blk hw_blk() {
   return Blk{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.x, (int)gridDim.y, (int)gridDim.z};
 }
@@ -45,27 +40,6 @@ __device__ __forceinline__ Blk hw_blk_xcd() {
   const int l = xcd_run((int)blockIdx.x + nx * ((int)blockIdx.y + ny * (int)blockIdx.z), nx * ny * nz);
   return Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, nz};
 }
-// The run of a batched launch's block b (the last r with off[r] <= b: runs of no blocks are
-// passed over) and the block's place in that run's grid
-struct BatchIdx {
-  int r;
-  Blk b;
-};
-__device__ __forceinline__ BatchIdx batch_idx(const BatchTab &t, int b = -1) {
-  if (b < 0) b = blockIdx.x;
-  int lo = 0, hi = t.n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (t.off[mid] <= b)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  const int l = b - t.off[lo];
-  const int nx = t.dims[3 * lo], ny = t.dims[3 * lo + 1], nz = t.dims[3 * lo + 2];
-  return BatchIdx{lo, Blk{l % nx, (l / nx) % ny, l / (nx * ny), nx, ny, nz}};
-}
-
 // ============================================================================ band stage
 // Rate of the frame at a block node: the faces copy the interior (precedence x, y, z), so the
 // value at any block node is the one of the nearest interior node (bands.jl:224-232).
@@ -4062,6 +4036,9 @@ size_t batch_args_size(int kind) {
     case BK_UNFOLD: return sizeof(UnfoldPass);
     case BK_ZMODESQ: return sizeof(ZModesQ64);
     case BK_QPLANE: return sizeof(QPass64);
+    case BK_SECTF:
+    case BK_SECTI: return sizeof(SectX);
+    case BK_SECTS: return sizeof(SectSep);
     default: return 0;
   }
 }
@@ -4156,6 +4133,9 @@ hipError_t launch_batch(int kind, int variant, size_t lds, const BatchTab &t, in
         }
       }
       break;
+    case BK_SECTF:
+    case BK_SECTS:
+    case BK_SECTI: return launch_sect_batch(kind, variant, lds, t, blocks, s);
     default: return launch_batch_meter(kind, t, blocks, s);
   }
   return hipGetLastError();

@@ -322,12 +322,19 @@ static void sx_grid(SectX &p, int &blocks, int &threads, size_t &lds) {
   threads = 64 * std::min(SX_WAVES, std::max(4, mt));
   lds = sx_lds(mt);
 }
+int sect_x_blocks(const SectX &p0) {
+  SectX p = p0;
+  int nb, nt;
+  size_t lds;
+  sx_grid(p, nb, nt, lds);
+  return nb;
+}
 hipError_t launch_sect_fwd(SectX p, hipStream_t s) {
-  if (g_rec) return hipErrorNotSupported;
   if (!sect_x_fits(p)) return hipErrorInvalidValue;
   int nb, nt;
   size_t lds;
   sx_grid(p, nb, nt, lds);
+  if (g_rec) return (p.gate || p.nparts) ? hipErrorNotSupported : record(BK_SECTF, Geo{}, &p, sizeof p, nt, true, dim3(nb), lds);
   TDGL_LAUNCH(k_sect_fwd, dim3(nb), dim3(nt), lds, s, p);
   return hipGetLastError();
 }
@@ -338,6 +345,234 @@ hipError_t launch_sect_inv(SectX p, hipStream_t s) {
   size_t lds;
   sx_grid(p, nb, nt, lds);
   TDGL_LAUNCH(k_sect_inv, dim3(nb), dim3(nt), lds, s, p);
+  return hipGetLastError();
+}
+
+__global__ void __launch_bounds__(64 * SX_WAVES, 5) k_sect_inv_sep(SectX p) { sect_inv_body<false>(p, (int)blockIdx.x, true); }
+hipError_t launch_sect_inv_sep(SectX p, hipStream_t s) {
+  if (!sect_x_fits(p)) return hipErrorInvalidValue;
+  int nb, nt;
+  size_t lds;
+  sx_grid(p, nb, nt, lds);
+  if (g_rec) return record(BK_SECTI, Geo{}, &p, sizeof p, nt, true, dim3(nb), lds);
+  TDGL_LAUNCH(k_sect_inv_sep, dim3(nb), dim3(nt), lds, s, p);
+  return hipGetLastError();
+}
+__global__ void __launch_bounds__(64 * SX_WAVES, 5) k_sect_fwd_b(BatchTab t) {
+  const BatchIdx q = batch_idx(t);
+  sect_fwd_body(((const SectX *)t.args)[q.r], q.b.x);
+}
+__global__ void __launch_bounds__(64 * SX_WAVES, 5) k_sect_inv_b(BatchTab t) {
+  const BatchIdx q = batch_idx(t);
+  sect_inv_body<false>(((const SectX *)t.args)[q.r], q.b.x, true);
+}
+
+// ---------------------------------------------------------------------------- the separable solve of a sector
+// One block per sector and mode, in FP64 and in place: the y products (16 x 16 x 4 tiles, rows of T by the
+// half-size basis, the basis from L2), the z products by component and 16 y modes a wave, (I + aK)^-1 by element
+// over all threads, the inverse z and y products.  T's rows are the z columns of X, Z and Y as in k_sect_cg.
+// Bound: the matrix products, 2 (Ly / 2) + 2 (Lz / 2) flop an element and direction.  With the z products, the
+// projector and their inverse of 16 y modes in one wave's registers (five waves of eight at work, two FP64 divisions
+// an element one behind the other) that part alone took 66 k of 155 k cycles.
+// 257 x 129 x 33 nodes: fold, quarter planes, z pass and unfold took 363 us, the three launches here 237 (this one 140; three
+// blocks a CU, the basis loads and products of their passes).
+template <int ZT, int SM>
+__device__ __forceinline__ void sect_sep_body(const SectSep &a, int b) {
+  extern __shared__ __align__(16) unsigned char cg_smem[];
+  const int tid = threadIdx.x, nth = blockDim.x, nw = nth >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lr = l & 15, lk = l >> 4;
+  const int s = b & 3, mx = b >> 2, py = s >> 1, pz = s & 1;
+  const SectDims &q = a.q;
+  const int n = q.size[s], ly = q.hy[0][py], le = q.hy[1][py], lz = q.hz[0][pz], lze = q.hz[1][pz];
+  const int oY = q.oc[1][s], oZ = q.oc[2][s];
+  const int yp = a.yp, ST = yp + 2, CY = lz + lze;
+  const int mt = (ly + 15) / 16, nt1 = (CY + 15) / 16, nt2 = (lz + 15) / 16, ntile = mt * (nt1 + nt2);
+  double *T = (double *)cg_smem;
+  for (int t = tid; t < a.trows * ST; t += nth) T[t] = 0.0;
+  const size_t base = (size_t)q.off[s] + (size_t)mx * n;
+  const float iy = 1.0f / (float)ly, ie = 1.0f / (float)le;
+  auto tat = [&](int e) {
+    const int c = e < oY ? 0 : (e < oZ ? 1 : 2), f = e - (c == 0 ? 0 : (c == 1 ? oY : oZ)), row = c == 1 ? le : ly;
+    const int k = (int)(((float)f + 0.5f) * (c == 1 ? ie : iy)), j = f - k * row;
+    return (c == 0 ? k : (c == 1 ? CY + k : lz + k)) * ST + j;
+  };
+  __syncthreads();
+  for (int e0 = tid; e0 < n; e0 += 4 * nth) {
+    double v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = a.S[base + min(e0 + u * nth, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + u * nth;
+      if (e < n) T[tat(e)] = (mx == 0 && e < oY) ? 0.0 : v[u];  // no edge mode of wave number 0
+    }
+  }
+  __syncthreads();
+  const float imt = 1.0f / (float)mt;
+  auto ypass = [&](const double *BV, const double *BU) __attribute__((always_inline)) {
+    v4d acc[SM];
+#pragma unroll
+    for (int t = 0; t < SM; ++t) {
+      acc[t] = v4d{0, 0, 0, 0};
+      const int tt = w + nw * t;
+      if (tt < ntile) {
+        const int nt = __builtin_amdgcn_readfirstlane((int)(((float)tt + 0.5f) * imt)), m = tt - nt * mt;
+        const double *B = (nt < nt1 ? BV : BU) + (size_t)(16 * m + lr) * yp + 4 * lk;
+        const double *A = T + ((nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1)) + lr) * ST + 4 * lk;
+        v4d bb = ld4d(B), bn = ld4d(B + 16 * min(1, mt - 1));
+        for (int g = 0; g < mt; ++g) {
+          const v4d b2 = ld4d(B + 16 * min(g + 2, mt - 1));
+          const v4d av = ld4d(A + 16 * g);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bb[u], acc[t], 0, 0, 0);
+          bb = bn;
+          bn = b2;
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < SM; ++t) {
+      const int tt = w + nw * t;
+      if (tt < ntile) {
+        const int nt = __builtin_amdgcn_readfirstlane((int)(((float)tt + 0.5f) * imt)), m = tt - nt * mt;
+        const int row0 = nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1), rows = nt < nt1 ? CY : CY + lz;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (row0 + lk + 4 * e < rows) T[(row0 + lk + 4 * e) * ST + 16 * m + lr] = acc[t][e];
+      }
+    }
+    __syncthreads();
+  };
+  ypass(a.yb[py][0][0], a.yb[py][1][0]);
+  // z forward and back, 16 y modes of a component a wave at a time, in place: the rows hold the z modes in between,
+  // the edges' (none for wave number 0) from row 0 on
+  const int sh = pz == 0 ? 1 : 0;
+  auto zpass = [&](int back) __attribute__((always_inline)) {
+    for (int o = w; o < 3 * mt; o += nw) {
+      const int c = __builtin_amdgcn_readfirstlane((int)(((float)o + 0.5f) * imt)), m = o - c * mt;
+      const int rows = c == 2 ? lze : lz, shi = c == 2 && back ? sh : 0, sho = c == 2 && !back ? sh : 0;
+      double *Tq = T + (c == 0 ? 0 : (c == 1 ? CY : lz)) * ST + 16 * m + lr;
+      const double *Z = a.zb[pz][c == 2][back] + (size_t)lr * a.zp + 4 * lk;
+      v4d A[ZT][ZT], acc[ZT];
+#pragma unroll
+      for (int t = 0; t < ZT; ++t) {
+        acc[t] = v4d{0, 0, 0, 0};
+#pragma unroll
+        for (int g = 0; g < ZT; ++g) A[t][g] = ld4d(Z + (size_t)16 * t * a.zp + 16 * g);
+      }
+#pragma unroll
+      for (int g = 0; g < ZT; ++g) {
+        double B[4];  // rows past the component's meet the zeros of the basis
+#pragma unroll
+        for (int u = 0; u < 4; ++u) B[u] = Tq[min(max(16 * g + 4 * lk + u - shi, 0), rows - 1) * ST];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int t = 0; t < ZT; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[t][g][u], B[u], acc[t], 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < ZT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 16 * t + lk + 4 * e - sho;
+          if (r >= 0 && r < rows) Tq[r * ST] = acc[t][e];
+        }
+    }
+    __syncthreads();
+  };
+  zpass(0);
+  {
+    const double k1 = a.s[0][mx];
+    const bool hx = mx > 0;
+    for (int t = tid; t < ly * lz; t += nth) {
+      // (I + aK)^{-1} = P_L + P_T / (1 + a |k|²) (implicit.jl:67-78); a component without the mode is zero
+      const int r = (int)(((float)t + 0.5f) * iy), p = t - r * ly, my = 2 * p + py, mz = 2 * r + pz;
+      const bool hy = my > 0, hz = mz > 0;
+      const double k2 = a.s[1][my], k3 = a.s[2][mz], k2s = k1 * k1 + k2 * k2 + k3 * k3;
+      double *X = T + r * ST + p, *Y = X + CY * ST, *Z = X + (lz - sh) * ST;
+      const double x1 = hx ? *X : 0.0, y1 = hy ? *Y : 0.0, z1 = hz ? *Z : 0.0;
+      double dd = 0.0, f = 1.0;
+      if (k2s != 0) {
+        dd = (k1 * x1 + k2 * y1 + k3 * z1) / k2s;
+        f = 1.0 / (1.0 + a.a * k2s);
+      }
+      *X = hx ? k1 * dd + f * (x1 - k1 * dd) : 0.0;
+      *Y = hy ? k2 * dd + f * (y1 - k2 * dd) : 0.0;
+      if (hz) *Z = k3 * dd + f * (z1 - k3 * dd);
+    }
+  }
+  __syncthreads();
+  zpass(1);
+  ypass(a.yb[py][0][1], a.yb[py][1][1]);
+  for (int e = tid; e < n; e += nth) a.S[base + e] = T[tat(e)];
+}
+template <int ZT, int SM>
+__global__ void __launch_bounds__(512, 4) k_sect_sep(SectSep a) {
+  sect_sep_body<ZT, SM>(a, (int)blockIdx.x);
+}
+template <int ZT, int SM>
+__global__ void __launch_bounds__(512, 4) k_sect_sep_b(BatchTab t) {
+  const BatchIdx q = batch_idx(t);
+  sect_sep_body<ZT, SM>(((const SectSep *)t.args)[q.r], q.b.x);
+}
+// z tiles, y tiles a wave (0: does not fit), LDS
+static int sep_pick(SectSep &a, int &zt, size_t &lds) {
+  const SectDims &q = a.q;
+  int ntile = 0;
+  a.trows = 0;
+  zt = cdiv(q.hz[0][0], 16);
+  for (int s = 0; s < 4; ++s) {
+    const int py = s >> 1, pz = s & 1, lz = q.hz[0][pz], lze = q.hz[1][pz], CY = lz + lze;
+    if (q.hy[0][py] < 1 || q.hy[1][py] < 1 || lz < 1 || lze < 1) return 0;
+    ntile = std::max(ntile, cdiv(q.hy[0][py], 16) * (cdiv(CY, 16) + cdiv(lz, 16)));
+    // the products read whole tiles of rows past the last component
+    a.trows = std::max({a.trows, CY + 16 * cdiv(lz, 16), CY + 16 * zt, 16 * cdiv(CY, 16)});
+  }
+  const int sm = cdiv(ntile, 8);
+  lds = (size_t)a.trows * (a.yp + 2) * sizeof(double);
+  if (zt > 3 || sm > 8 || lds + 1024 > SECT_LDS_MAX) return 0;
+  return sm <= 4 ? 4 : 8;
+}
+bool sect_sep_fits(const SectSep &a0) {
+  SectSep a = a0;
+  int zt;
+  size_t lds;
+  return sep_pick(a, zt, lds) > 0;
+}
+#define TDGL_SEP_ALL TDGL_SEP(1, 4) TDGL_SEP(2, 4) TDGL_SEP(3, 4) TDGL_SEP(1, 8) TDGL_SEP(2, 8) TDGL_SEP(3, 8)
+hipError_t launch_sect_sep(SectSep a, hipStream_t s) {
+  int zt;
+  size_t lds;
+  const int sm = sep_pick(a, zt, lds);
+  if (!sm) return hipErrorInvalidValue;
+  const dim3 grid(4 * a.q.nx);
+  if (g_rec) return record(BK_SECTS, Geo{}, &a, sizeof a, 10 * zt + sm, true, grid, lds);
+  switch (10 * zt + sm) {
+#define TDGL_SEP(z, m) \
+  case 10 * z + m: TDGL_LAUNCH((k_sect_sep<z, m>), grid, dim3(512), lds, s, a); break;
+    TDGL_SEP_ALL
+#undef TDGL_SEP
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+hipError_t launch_sect_batch(int kind, int variant, size_t lds, const BatchTab &t, int blocks, hipStream_t s) {
+  if (kind == BK_SECTF || kind == BK_SECTI) {
+    if (variant < 64 || variant > 64 * SX_WAVES) return hipErrorInvalidValue;
+    if (kind == BK_SECTF)
+      TDGL_LAUNCH(k_sect_fwd_b, dim3(blocks), dim3(variant), lds, s, t);
+    else
+      TDGL_LAUNCH(k_sect_inv_b, dim3(blocks), dim3(variant), lds, s, t);
+    return hipGetLastError();
+  }
+  switch (variant) {
+#define TDGL_SEP(z, m) \
+  case 10 * z + m: TDGL_LAUNCH((k_sect_sep_b<z, m>), dim3(blocks), dim3(512), lds, s, t); break;
+    TDGL_SEP_ALL
+#undef TDGL_SEP
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

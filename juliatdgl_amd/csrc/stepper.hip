@@ -175,6 +175,8 @@ struct tdgl_handle {
   SectDims sq{};
   double *sxB[2][2][2] = {};   // x half bases [0 V, 1 U][parity][0 forward, 1 back], zero-padded to whole tiles
   float *syb[2][2][2] = {}, *szb[2][2][2] = {};  // SectCG::yb, zb
+  double *sydb[2][2][2] = {}, *szdb[2][2][2] = {};  // SectSep::yb, zb
+  bool sepsect = false;        // the separable solve by sectors (k_sect_sep)
   int syp = 0, szp = 0;
   unsigned char *scode[3] = {};
   double *spal = nullptr;
@@ -1147,8 +1149,43 @@ int sep_solve_folded64(tdgl_handle *h, const Vec3 &in, const SepOut &o) {
   return 0;
 }
 
+SectX sect_x(tdgl_handle *h, bool inv);
+SectSep sect_sep(tdgl_handle *h) {
+  SectSep a{};
+  a.q = h->sq;
+  a.S = h->T1;
+  for (int ax = 0; ax < 3; ++ax) a.s[ax] = h->sd[ax];
+  for (int par = 0; par < 2; ++par)
+    for (int w = 0; w < 2; ++w)
+      for (int t = 0; t < 2; ++t) {
+        a.yb[par][w][t] = h->sydb[par][w][t];
+        a.zb[par][w][t] = h->szdb[par][w][t];
+      }
+  a.yp = h->syp;
+  a.zp = h->szp;
+  a.a = h->d.a;
+  return a;
+}
+// φ = θ + (I + aK)^-1 in by sectors: the x transform folded in all three axes, each (mode, y parity, z parity) in
+// one block's LDS, and back
+int sep_solve_sect(tdgl_handle *h, const Vec3 &in) {
+  SectX f = sect_x(h, false);
+  for (int c = 0; c < 3; ++c) f.v[c] = node_view(h, in.c[c]);
+  f.S = h->T1;
+  PL(K_TX, launch_sect_fwd(f, h->s));
+  PL(K_MODES, launch_sect_sep(sect_sep(h), h->s));
+  SectX b = sect_x(h, true);
+  for (int c = 0; c < 3; ++c) {
+    b.v[c] = node_view(h, h->ph[c]);
+    b.th[c] = node_view(h, h->th[c]);
+  }
+  b.S = h->T1;
+  PL(K_TX, launch_sect_inv_sep(b, h->s));
+  return 0;
+}
 int sep_solve(tdgl_handle *h, const Vec3 &in, const SepOut &o, const int *gate, bool f32, Conv conv) {
   if (f32 && h->fold) return sep_solve_folded(h, in, o, gate, conv);
+  if (!f32 && h->sepsect && !h->tx_only && !gate && conv.mode == CONV_NONE && o.addth && !o.dot && !o.out32) return sep_solve_sect(h, in);
   if (!f32 && h->fold64 && !h->tx_only && !gate && conv.mode == CONV_NONE && !o.dot && !o.out32)
     return sep_solve_folded64(h, in, o);
   void *Ta = f32 ? (void *)h->T32a : (void *)h->T1;
@@ -2521,6 +2558,95 @@ int refine_setup(tdgl_handle *h) {
   return 0;
 }
 
+// the half-size bases of the sectors along x, zero-padded to whole tiles
+template <class Put>
+void sect_x_tables(tdgl_handle *h, Put &&put) {
+  const Bases b = make_bases(h->sq.nx);
+  for (int w = 0; w < 2; ++w) {
+    const std::vector<double> &M = w == 0 ? b.V : b.U;
+    const int L = h->sq.nx - w, Lh = (L + 1) / 2;
+    // the x passes pad to the tiles of the component's own extent
+    const int LP = 16 * cdiv(Lh, 16);
+    for (int par = 0; par < 2; ++par)
+      for (int t = 0; t < 2; ++t) {
+        std::vector<double> m((size_t)LP * LP, 0.0);
+        for (int i = 0; i < Lh; ++i)
+          for (int cc = 0; cc < Lh; ++cc) {
+            const int col = 2 * cc + par;
+            if (col >= L) continue;
+            const double v = M[i + (size_t)L * col];
+            m[t == 0 ? (size_t)cc * LP + i : (size_t)i * LP + cc] = v;
+          }
+        put(&h->sxB[w][par][t], m.data(), m.size() * sizeof(double));
+      }
+  }
+}
+// along y and z (SectCG::yb, zb and SectSep's)
+template <class T, class Put>
+void sect_yz_tables(tdgl_handle *h, T *(&yb)[2][2][2], T *(&zb)[2][2][2], Put &&put) {
+  const SectDims &q = h->sq;
+  for (int ax = 1; ax < 3; ++ax) {
+    const int nn = ax == 1 ? q.ny : q.nz, np = ax == 1 ? h->syp : h->szp;
+    const int(*hh)[2] = ax == 1 ? q.hy : q.hz;
+    const Bases b = make_bases(nn);
+    for (int par = 0; par < 2; ++par)
+      for (int w = 0; w < 2; ++w) {
+        std::vector<T> f((size_t)np * np, (T)0), g((size_t)np * np, (T)0);
+        for (int m = 0; 2 * m + par < nn; ++m) {
+          const int k = 2 * m + par;  // the wave number; edges: its column k - 1 (none for 0)
+          if (w == 1 && k == 0) continue;
+          for (int j = 0; j < hh[w][par]; ++j) {
+            const double v = w == 0 ? b.V[j + (size_t)nn * k] : b.U[j + (size_t)(nn - 1) * (k - 1)];
+            const bool centre = w == 0 ? (nn % 2 == 1 && par == 0 && j == hh[0][0] - 1) : (nn % 2 == 0 && par == 1 && j == hh[1][1] - 1);
+            f[(size_t)m * np + j] = (T)(centre ? v : 2.0 * v);
+            g[(size_t)j * np + m] = (T)v;
+          }
+        }
+        T **dst = ax == 1 ? yb[par][w] : zb[par][w];
+        put(&dst[0], f.data(), f.size() * sizeof(T));
+        put(&dst[1], g.data(), g.size() * sizeof(T));
+      }
+  }
+}
+
+// The separable solve by sectors where the planes are too large for the one-round FP64 kernel (wide), a sector fits
+// a workgroup and the x passes have blocks for the chip (SECT_SEP_BLOCKS; TDGL_HIP_SECT=1: from three nodes on, =0:
+// never; the variables that shape the other solves keep them).  Us a step of two bands, quarters against sectors, by
+// the x passes' blocks: 62.0 / 72.7 (161x30x8 cells, 30 blocks), 157 / 168 (200x100x16, 189), 169 / 171 (200x60x32, 204),
+// 197 / 210 (250x100x20, 231), 163 / 170 (150x128x18, 270), 228 / 212 (200x100x24, 273), 197 / 180 (180x60x44, 276),
+// 118 / 93 (60x200x14, 312), 225 / 193 (170x100x30, 336), 294 / 288 (200x100x32, 357), 584 / 459 (256x128x32, 459),
+// 1431 / 747 (256x128x60, 837).
+constexpr int SECT_SEP_BLOCKS = 300;
+int sepsect_setup(tdgl_handle *h, bool wide) {
+  const tdgl_desc &d = h->d;
+  const char *off = std::getenv("TDGL_HIP_SECT");
+  const bool force = off && off[0] == '1';
+  for (const char *v : {"TDGL_HIP_FOLD64", "TDGL_HIP_PLANE", "TDGL_HIP_ZCOL", "TDGL_HIP_ZQ_WAVES"})
+    if (std::getenv(v)) return 0;
+  if ((off && off[0] == '0') || !(wide || force) || d.Nx - 1 < 2 || d.Ny - 1 < 3 || d.Nz - 1 < 3) return 0;
+  h->sq = sect_dims(d.Nx - 1, d.Ny - 1, d.Nz - 1);
+  h->syp = 16 * cdiv(h->sq.hy[0][0], 16);
+  h->szp = 16 * cdiv(h->sq.hz[0][0], 16);
+  if (!force && sect_x_blocks(sect_x(h, false)) < SECT_SEP_BLOCKS) return 0;
+  if (!sect_x_fits(sect_x(h, false)) || !sect_sep_fits(sect_sep(h)) || (size_t)h->sq.total > h->t12cap) return 0;
+  std::vector<unsigned char> all;
+  std::vector<std::pair<void *, size_t>> tabs;
+  auto put = [&](void *where, const void *src, size_t bytes) {
+    const size_t o = (all.size() + 255) / 256 * 256;
+    all.resize(o + bytes);
+    std::memcpy(&all[o], src, bytes);
+    tabs.push_back({where, o});
+  };
+  sect_x_tables(h, put);
+  sect_yz_tables<double>(h, h->sydb, h->szdb, put);
+  unsigned char *dev = nullptr;
+  ALLOC(dev, all.size());
+  CHK(upload_vec(h, dev, all));
+  for (const auto &t : tabs) *(void **)t.first = dev + t.second;
+  h->sepsect = true;
+  return 0;
+}
+
 // The solve by sectors where it applies: the Float32-preconditioned PCG with the same coefficient in every
 // direction, D constant along x and equal to its mirror images in y and z on the unknowns (what
 // link_conductivity gives, implicit.jl:126-140), at most DPAL_MAX values of D a component, and a sector that
@@ -2578,49 +2704,8 @@ int sect_setup(tdgl_handle *h) {
     std::memcpy(&all[o], src, bytes);
     tabs.push_back({where, o});
   };
-  {
-    const Bases b = make_bases(n[0]);
-    for (int w = 0; w < 2; ++w) {
-      const std::vector<double> &M = w == 0 ? b.V : b.U;
-      const int L = n[0] - w, Lh = (L + 1) / 2;
-      // the x passes pad to the tiles of the component's own extent
-      const int LP = 16 * cdiv(Lh, 16);
-      for (int par = 0; par < 2; ++par)
-        for (int t = 0; t < 2; ++t) {
-          std::vector<double> m((size_t)LP * LP, 0.0);
-          for (int i = 0; i < Lh; ++i)
-            for (int cc = 0; cc < Lh; ++cc) {
-              const int col = 2 * cc + par;
-              if (col >= L) continue;
-              const double v = M[i + (size_t)L * col];
-              m[t == 0 ? (size_t)cc * LP + i : (size_t)i * LP + cc] = v;
-            }
-          put(&h->sxB[w][par][t], m.data(), m.size() * sizeof(double));
-        }
-    }
-  }
-  for (int ax = 1; ax < 3; ++ax) {
-    const int nn = n[ax], np = ax == 1 ? h->syp : h->szp;
-    const int(*hh)[2] = ax == 1 ? q.hy : q.hz;
-    const Bases b = make_bases(nn);
-    for (int par = 0; par < 2; ++par)
-      for (int w = 0; w < 2; ++w) {
-        std::vector<float> f((size_t)np * np, 0.0f), g((size_t)np * np, 0.0f);
-        for (int m = 0; 2 * m + par < nn; ++m) {
-          const int k = 2 * m + par;  // the wave number; edges: its column k - 1 (none for 0)
-          if (w == 1 && k == 0) continue;
-          for (int j = 0; j < hh[w][par]; ++j) {
-            const double v = w == 0 ? b.V[j + (size_t)nn * k] : b.U[j + (size_t)(nn - 1) * (k - 1)];
-            const bool centre = w == 0 ? (nn % 2 == 1 && par == 0 && j == hh[0][0] - 1) : (nn % 2 == 0 && par == 1 && j == hh[1][1] - 1);
-            f[(size_t)m * np + j] = (float)(centre ? v : 2.0 * v);
-            g[(size_t)j * np + m] = (float)v;
-          }
-        }
-        float **dst = ax == 1 ? h->syb[par][w] : h->szb[par][w];
-        put(&dst[0], f.data(), f.size() * sizeof(float));
-        put(&dst[1], g.data(), g.size() * sizeof(float));
-      }
-  }
+  sect_x_tables(h, put);
+  sect_yz_tables<float>(h, h->syb, h->szb, put);
   for (int c = 0; c < 3; ++c) put(&h->scode[c], code[c].data(), code[c].size());
   put(&h->spal, pal.data(), pal.size() * sizeof(double));
   unsigned char *dev = nullptr;
@@ -2956,7 +3041,8 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
     const bool fold64_pays = l0max > 160 || l1max > 96;
     const bool fold64_on = gf64 ? gf64[0] == '1' : fold64_pays;
     if (d.field_mode == TDGL_FIELD_SEPARABLE && !(zc && zc[0] == '0')) h->zcols = 1;
-    if (d.field_mode == TDGL_FIELD_SEPARABLE && h->plane64 && fold64_on && d.Nz - 1 >= 2 && d.Nz - 1 <= ZQ64_NZ_MAX) {
+    if (d.field_mode == TDGL_FIELD_SEPARABLE) CHK(sepsect_setup(h, fold64_pays));
+    if (!h->sepsect && d.field_mode == TDGL_FIELD_SEPARABLE && h->plane64 && fold64_on && d.Nz - 1 >= 2 && d.Nz - 1 <= ZQ64_NZ_MAX) {
       int qe[12][3];
       const Quarters q = quarters_of(rg, qe);
       if (plane_fits<double>(qe, 12) && fold_blocks(q) <= MAX_PART && (size_t)q.total <= h->t12cap) {
@@ -3825,7 +3911,7 @@ int tdgl_get_stats(tdgl_handle *h, tdgl_stats *st) {
     if (m > 0) st->pcg_budget = m;
   }
   st->captures = h->captures;
-  st->folded = (h->fold || h->fold64) ? 1 : 0;
+  st->folded = h->sepsect ? 2 : (h->fold || h->fold64) ? 1 : 0;
   st->steps = h->steps;
   st->calls = h->calls;
   st->pcg_iters = h->pcg_iters;
@@ -4128,7 +4214,7 @@ int tdgl_batch_create(tdgl_handle *const *hs, int32_t n, tdgl_batch **out) {
   b->dev = hs[0]->dev;
   const char *ge = std::getenv("TDGL_HIP_GRAPH");  // =0: the batched launches from the host (profiling)
   b->graphs = !(ge && ge[0] == '0');
-  for (int r = 1; r < n; ++r) b->tx_only |= hs[r]->plane64 != hs[0]->plane64 || hs[r]->fold64 != hs[0]->fold64;
+  for (int r = 1; r < n; ++r) b->tx_only |= hs[r]->plane64 != hs[0]->plane64 || hs[r]->fold64 != hs[0]->fold64 || hs[r]->sepsect != hs[0]->sepsect;
   auto bail = [&](int rc) {
     tdgl_batch_destroy(b);
     return rc;
