@@ -45,6 +45,16 @@ def kernel_bytes(st, name: str, launches: int, nsteps: int, stats: dict) -> floa
     nodes = (gr.Nx + 1) * (gr.Ny + 1) * (gr.Nz + 1)
     rng = (gr.Nx - 2) * (gr.Ny - 1) * (gr.Nz - 1) + (gr.Nx - 1) * (gr.Ny - 2) * (gr.Nz - 1) + \
         (gr.Nx - 1) * (gr.Ny - 1) * (gr.Nz - 2)
+    sect = stats.get("sect")
+    if name == "pcg_sectors":
+        return 16.0 * rng * launches  # r in, d out: the iterations stay in LDS and registers
+    if sect == "pcg" and name in ("sep_transform_f64", "pcg_apply_A", "pcg_vector"):
+        # the x transforms (r in, sectors out; sectors, θ and x in, x and φ out), the residual (x, b in, r out), the
+        # start (x and the one before, in and out)
+        return {"sep_transform_f64": 28.0, "pcg_apply_A": 24.0, "pcg_vector": 32.0}[name] * rng * launches
+    if sect == "sep" and name in ("sep_transform_f64", "sep_modes"):
+        # the x transforms (b in, sectors out; sectors and θ in, φ out), the sectors in place
+        return {"sep_transform_f64": 20.0, "sep_modes": 16.0}[name] * rng * launches
     if name == "band_stage":
         # S, D, the other bands, f, three links (+ Y_{j-2} and Ω on most stages)
         per = 16 + 16 + 16 * (N - 1) + 8 + 48 + 16 + 8
@@ -101,13 +111,25 @@ def quarter_total(gr):
     return sum(4 * h0 * h1 * e2 for h0, h1, e2 in quarters(gr))
 
 
-def kernel_flops(st, name: str, launches: int, folded: bool = False) -> float:
+def solved_by_sectors(prof, folded: int):
+    """"pcg" or "sep" where the field solve went by sectors, else None."""
+    if prof["pcg_sectors"][0]:
+        return "pcg"
+    return "sep" if folded == 2 else None
+
+
+def kernel_flops(st, name: str, launches: int, folded: bool = False, sect=None) -> float:
     """Algorithmic flops of the launches of one kernel class: a fused x-y transform launch of the
     separable solve multiplies every element by an (Lx x Lx) then an (Ly x Ly) matrix, 2 (Lx + Ly)
     flop per element; folded, each of the four quarters of a component by its half-size bases,
     2 (ceil(Lx/2) + ceil(Ly/2)) flop per quarter element (half the work).  The folded Float32
     preconditioner's z pass takes every quarter element by an (Lz x Lz) matrix forward and back,
-    4 Lz flop per element."""
+    4 Lz flop per element.  By sectors the transforms are the x axis' alone, folded: Lx flop per element, and the
+    separable solve's sectors take 2 (Ly + Lz) flop per element."""
+    if sect and name == "sep_transform_f64":
+        return launches * sum(1.0 * ex[0] * ex[1] * ex[2] * ex[0] for ex in ranges(st.grid))
+    if sect == "sep" and name == "sep_modes":
+        return launches * sum(2.0 * ex[0] * ex[1] * ex[2] * (ex[1] + ex[2]) for ex in ranges(st.grid))
     if name == "sep_modes" and folded and st.field_mode == 2:
         return launches * sum(4 * h0 * h1 * e2 * 4.0 * e2 for h0, h1, e2 in quarters(st.grid))
     if name == "sep_transform_f32" and folded:
@@ -118,7 +140,7 @@ def kernel_flops(st, name: str, launches: int, folded: bool = False) -> float:
     return 0.0
 
 
-def cycle_bytes_per_node_step(st, iters_per_step: float) -> float:
+def cycle_bytes_per_node_step(st, iters_per_step: float, sect=None) -> float:
     """B_alg per padded node and step of the whole step (every array a fused phase touches counted
     once): the bands' stages, supercurrent + field increment, the PCG (per iteration with the
     Float32 preconditioner) and links + curl, as tabulated for this path."""
@@ -126,7 +148,10 @@ def cycle_bytes_per_node_step(st, iters_per_step: float) -> float:
     N = st.N
     band = 2 * (16 * (N + 1) + 8 + 72) + 152 * (s - 2)
     field = 16 * N + 192
-    if st.field_mode == 2 and getattr(st, "pcg_refine", False):
+    if sect:
+        # by sectors: the x transforms around the sectors' pass, and for the PCG the start and the residual
+        pcg = 24 * (4 + 3 + 2 + 2 + 5) if sect == "pcg" else 24 * (2 + 2 + 3)
+    elif st.field_mode == 2 and getattr(st, "pcg_refine", False):
         # Float32 inner iterations (their vectors, operator and D at half the bytes of the FP64
         # ones: 176 for 288), and about three FP64 rounds a step (residual, check, x += d)
         pcg = 300 + 176 * iters_per_step + 3 * 150
@@ -333,10 +358,10 @@ def cpu_sample(name, st, dev, H, HJ, nsteps):
             "single_thread": {"value": v1, "cores": 1, "seconds": d1}, "cpu_model": model}
 
 
-def roofline(st, dom, nl, ms, nsteps, iters, workload, folded=False):
+def roofline(st, dom, nl, ms, nsteps, iters, workload, folded=False, sect=None):
     avg_s = ms / nl / 1e3
-    byts = kernel_bytes(st, dom, nl, nsteps, {"iters_per_solve": iters / nsteps, "folded": folded}) / nl
-    flops = kernel_flops(st, dom, nl, folded) / nl
+    byts = kernel_bytes(st, dom, nl, nsteps, {"iters_per_solve": iters / nsteps, "folded": folded, "sect": sect}) / nl
+    flops = kernel_flops(st, dom, nl, folded, sect) / nl
     peak = FP32_MFMA_PEAK if dom in ("sep_transform_f32", "sep_modes") else FP64_PEAK
     if byts > 0 and (flops == 0 or flops / byts < peak / HBM_PEAK):
         roof = {"bound": "hbm", "achieved": byts / avg_s / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
@@ -344,7 +369,9 @@ def roofline(st, dom, nl, ms, nsteps, iters, workload, folded=False):
                 "avg_launch_us": avg_s * 1e6,
                 "note": "algorithmic bytes: each array the launch must touch counted once (FP64 node-shaped vectors, "
                         "FP32 quarters); durations from HIP events recorded at each launch's start and end over the "
-                        "same number of cycles as the timed region"}
+                        "same number of cycles as the timed region" +
+                        ("; the launch holds every iteration of the solve in LDS and registers: the bound is the "
+                         "issue of its stencil, products and sums" if dom == "pcg_sectors" else "")}
     else:
         roof = {"bound": "mfma", "achieved": flops / avg_s / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                 "frac": flops / avg_s / peak, "traffic": None, "kernel": dom, "flops_per_launch": flops,
@@ -431,7 +458,13 @@ def run_workload(name, steps, warmup, profile=True, cpu_steps=0, profile_out=Non
                 print(f"[bench]   {kname:20s} {nl:8d} launches {ms:10.3f} ms ({100 * ms / tot:5.1f}%) "
                       f"{1e3 * ms / nl:8.2f} us/launch", file=sys.stderr)
         dom, (nl, ms) = rows[0]
-        out["roofline"] = roofline(st, dom, nl, ms, nsteps, iters, name, bool(st1.get("folded", 0)))
+        sect = solved_by_sectors(prof, int(st1.get("folded", 0)))
+        out["roofline"] = roofline(st, dom, nl, ms, nsteps, iters, name, bool(st1.get("folded", 0)), sect)
+        out["config"]["solved_by_sectors"] = sect
+        if sect:
+            balg = cycle_bytes_per_node_step(st, iters / nsteps, sect)
+            out["config"]["b_alg_per_node_step"] = balg
+            out["config"]["hbm_roofline_frac_cycle"] = balg * nodes * LMAX * steps / wall / HBM_PEAK
         out["config"]["folded_preconditioner"] = bool(st1.get("folded", 0))
         out["config"]["kernel_ms_per_cycle"] = {k: v[1] / steps for k, v in prof.items() if v[0]}
         # every class with algorithmic bytes: its average launch against the HBM peak (and the
@@ -441,12 +474,12 @@ def run_workload(name, steps, warmup, profile=True, cpu_steps=0, profile_out=Non
             if not nl_k:
                 continue
             b = kernel_bytes(st, kname, nl_k, nsteps, {"iters_per_solve": iters / nsteps,
-                                                       "folded": bool(st1.get("folded", 0))}) / nl_k
+                                                       "folded": bool(st1.get("folded", 0)), "sect": sect}) / nl_k
             if b <= 0:
                 continue
             us = 1e3 * ms_k / nl_k
             row = {"us_per_launch": us, "bytes_per_launch": b, "GB_s": b / us / 1e3, "hbm_frac": b / us / 1e3 / (HBM_PEAK / 1e9)}
-            f = kernel_flops(st, kname, nl_k, bool(st1.get("folded", 0))) / nl_k
+            f = kernel_flops(st, kname, nl_k, bool(st1.get("folded", 0)), sect) / nl_k
             if f > 0:
                 pk = FP32_MFMA_PEAK if kname in ("sep_transform_f32", "sep_modes") else FP64_PEAK
                 row["TFLOP_s"] = f / us / 1e6
