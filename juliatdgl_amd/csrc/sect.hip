@@ -1,4 +1,4 @@
-// sect.hip — the insulating PCG solved sector by sector.
+// sect.hip — the insulating PCG, and the separable solve of large planes, sector by sector.
 //
 // The conductivity of the field solve is constant along x and mirror-symmetric in y and z (the bar and
 // its padding, implicit.jl:126-140), so A = D + aK keeps three symmetries that the general PCG does not
@@ -8,16 +8,16 @@
 // enough for one workgroup's LDS and registers: k_sect_fwd takes the residual to the sectors, k_sect_cg
 // runs the whole flexible CG of a sector in one launch, k_sect_inv takes the solution back.  The general
 // iteration's six launches and 860 MB of HBM traffic (290 us on 256x128x32 cells, 20 to 24 a step; 50 us,
-// launch-bound, on 96x48x24) become one launch a solve, whose iterations leave the CU only for the bases and
-// the solution: a time step took 7.86 -> 1.97 ms on 256x128x32 cells, 458 -> 193 us on 96x48x24, 610 -> 224 us on
-// 128x64x16 with KWT, 327 -> 117 us on 53x27x9.
+// launch-bound, on 96x48x24) become one launch a solve, whose iterations leave the CU only for the bases:
+// a time step took 7.86 -> 1.35 ms on 256x128x32 cells, 458 -> 132 us on 96x48x24, 610 -> 155 us on 128x64x16 with
+// KWT, 327 -> 77 us on 53x27x9 (with the open boundary's and the launches' own savings).
 //
 // A sector holds values on the half domain (the rest follows by parity): component c of mode mx at
 // (j, k), j fastest, X (c = 0) then Y then Z.  With (py, pz) the parities of the sector's y and z wave
 // numbers, a component is node-like (cosine) along an axis other than its own and edge-like (sine, the
 // opposite parity) along its own.  A half axis of n nodes holds ceil(n/2) (even) or floor(n/2) (odd)
 // nodes and ceil(n/2) - 1 or floor(n/2) edges; sums over a whole axis weigh each point by 2, a centre
-// point by 1.  A difference across the centre takes the mirrored value (SectGhost).
+// point by 1.  A difference across the centre takes the mirrored value (the ghosts of k_sect_cg).
 #include "kernels.h"
 
 namespace tdgl {
