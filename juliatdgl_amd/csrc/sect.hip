@@ -625,6 +625,12 @@ __device__ __forceinline__ double wave_sum63(double v) {
   return dpp_add<0x143, 0xc>(v);
 }
 
+// The y tiles a wave holds at once: one or two, or up to four, in one round; a plane with more goes in rounds of whole
+// row groups (a tile reads and writes the rows of its own group only).  One instance of up to six tiles spilled 510 to
+// 940 B a lane and was slower than the general iteration on some planes; a step with it, now and by the general
+// iteration: 1265 / 444 / 1031 us (200x250x4 cells, buf 2), 1722 / 677 / 1587 (200x110x34), 1081 / 586 / 986 (8x640x5,
+// rounds), 699 / 383 / 684 (16x60x88); 4244 / 1661 / 9309 us on 256x128x33 cells, buf 8.
+constexpr int SECT_SM = 4;
 template <int EPT, int ZT, int SM, int MT>
 __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   if (!sect_active(a.d)) return;
@@ -747,16 +753,19 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   struct First {
     v4f a, b;  // the first tile's first two groups of the basis
   };
-  auto tile = [&](int t, int &m, int &nt) __attribute__((always_inline)) {
-    const int tt = w + nw * t;
+  // tile t of this wave in the round of row groups that starts at tile t0
+  constexpr int SA = SM > SECT_SM ? SECT_SM : SM;  // accumulators a wave
+  const int per = SM > SECT_SM ? mt * (SECT_SM * nw / mt) : ntile;
+  auto tile = [&](int t0, int t, int &m, int &nt) __attribute__((always_inline)) {
+    const int tt = t0 + w + nw * t;
     nt = MT ? tt / max(MT, 1) : __builtin_amdgcn_readfirstlane((int)(((float)tt + 0.5f) * imt));
     m = tt - nt * mt;
-    return tt < ntile;
+    return tt < (SM > SECT_SM ? min(t0 + per, ntile) : ntile);
   };
   auto first = [&](const float *BV, const float *BU) __attribute__((always_inline)) {
     First f{v4f{0, 0, 0, 0}, v4f{0, 0, 0, 0}};
     int m, nt;
-    if (tile(0, m, nt)) {
+    if (tile(0, 0, m, nt)) {
       const float *A = (nt < nt1 ? BV : BU) + 16 * m * yp + fresh(lr) * yp + 4 * lk;
       f.a = *(const v4f *)A;
       f.b = *(const v4f *)(A + 16 * min(1, mt - 1));
@@ -765,39 +774,43 @@ __global__ void __launch_bounds__(SECT_T, 4) k_sect_cg(SectCG a) {
   };
   auto ypass = [&](const float *BV, const float *BU, const First f) __attribute__((always_inline)) {
     const int la = fresh(lr) * yp + 4 * lk, lb = fresh(lr) * ST + 4 * lk;
-    v4f acc[SM];
+    int t0 = 0;
+    do {
+      v4f acc[SA];
 #pragma unroll
-    for (int t = 0; t < SM; ++t) {
-      acc[t] = v4f{0, 0, 0, 0};
-      int m, nt;
-      if (tile(t, m, nt)) {
-        const float *A = (nt < nt1 ? BV : BU) + 16 * m * yp + la;
-        const float *B = T + (nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1)) * ST + lb;
-        // the basis comes through L2: two groups of sixteen ahead
-        v4f av = t ? *(const v4f *)A : f.a, an = t ? *(const v4f *)(A + 16 * min(1, mt - 1)) : f.b;
+      for (int t = 0; t < SA; ++t) {
+        acc[t] = v4f{0, 0, 0, 0};
+        int m, nt;
+        if (tile(t0, t, m, nt)) {
+          const float *A = (nt < nt1 ? BV : BU) + 16 * m * yp + la;
+          const float *B = T + (nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1)) * ST + lb;
+          // the basis comes through L2: two groups of sixteen ahead
+          const bool asked = t == 0 && (SM <= SECT_SM || t0 == 0);
+          v4f av = asked ? f.a : *(const v4f *)A, an = asked ? f.b : *(const v4f *)(A + 16 * min(1, mt - 1));
 #pragma unroll(MT ? MT : 1)
-        for (int g = 0; g < mt; ++g) {
-          const v4f aq = *(const v4f *)(A + 16 * min(g + 2, mt - 1));
-          const v4f bv = *(const v4f *)(B + 16 * g);
+          for (int g = 0; g < mt; ++g) {
+            const v4f aq = *(const v4f *)(A + 16 * min(g + 2, mt - 1));
+            const v4f bv = *(const v4f *)(B + 16 * g);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc[t], 0, 0, 0);
-          av = an;
-          an = aq;
+            for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc[t], 0, 0, 0);
+            av = an;
+            an = aq;
+          }
         }
       }
-    }
-    __syncthreads();
+      __syncthreads();
 #pragma unroll
-    for (int t = 0; t < SM; ++t) {
-      int m, nt;
-      if (tile(t, m, nt)) {
-        const int col0 = nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1);
-        if (col0 + lr < (nt < nt1 ? CY : CY + lz)) *(v4f *)(T + col0 * ST + 16 * m + lb) = acc[t];
+      for (int t = 0; t < SA; ++t) {
+        int m, nt;
+        if (tile(t0, t, m, nt)) {
+          const int col0 = nt < nt1 ? 16 * nt : CY + 16 * (nt - nt1);
+          if (col0 + lr < (nt < nt1 ? CY : CY + lz)) *(v4f *)(T + col0 * ST + 16 * m + lb) = acc[t];
+        }
       }
-    }
+      t0 += per;
+    } while (SM > SECT_SM && t0 < ntile);
     __syncthreads();
   };
-
   const float *const yf[2] = {a.yb[py][0][0], a.yb[py][1][0]}, *const yr[2] = {a.yb[py][0][1], a.yb[py][1][1]};
   First ff = first(yf[0], yf[1]), fr = ff;
   if (SMALL) fr = first(yr[0], yr[1]);
@@ -1017,7 +1030,7 @@ struct CgPick {
 static CgPick cg_pick(const SectCG &a0, int &np, int &trows, int &ng) {
   CgPick k{};
   const SectDims &q = a0.q;
-  int n = 0, ntile = 0;
+  int n = 0, ntile = 0, mtm = 0;
   np = trows = ng = 0;
   for (int s = 0; s < 4; ++s) {
     const int py = s >> 1, pz = s & 1, lz = q.hz[0][pz], lze = q.hz[1][pz], CY = lz + lze;
@@ -1026,6 +1039,7 @@ static CgPick cg_pick(const SectCG &a0, int &np, int &trows, int &ng) {
     n = std::max(n, q.size[s]);
     const int mt = cdiv(q.hy[0][py], 16), nt = cdiv(CY, 16) + cdiv(lz, 16);
     ntile = std::max(ntile, mt * nt);
+    mtm = std::max(mtm, mt);
     trows = std::max(trows, CY + 16 * cdiv(lz, 16));
     np = std::max(np, (2 * (lz + 2) + lze + 2) * (q.hy[0][py] + 2));
     ng = std::max(ng, 3 * (q.hy[0][py] + lz) + 2 * (q.hy[1][py] + lze) + 2);
@@ -1045,7 +1059,8 @@ static CgPick cg_pick(const SectCG &a0, int &np, int &trows, int &ng) {
   const size_t nT = (size_t)trows * (a0.yp + 4);
   k.lds = (size_t)np * sizeof(double) + nT * sizeof(float) + (size_t)ng * sizeof(unsigned) + (size_t)q.hz[0][0] * sizeof(float);
   // 14 bits hold a place in P and in T
-  k.ok = k.zt <= 3 && k.sm <= 6 && np <= 16384 && nT <= 16384 && k.lds + 1024 <= SECT_LDS_MAX;
+  // a round of the y products takes whole row groups
+  k.ok = k.zt <= 3 && k.sm <= 6 && mtm <= SECT_SM * (k.threads / 64) && np <= 16384 && nT <= 16384 && k.lds + 1024 <= SECT_LDS_MAX;
   return k;
 }
 bool sect_cg_fits(const SectCG &a) {
@@ -1062,12 +1077,14 @@ hipError_t launch_sect_cg(SectCG a, hipStream_t s) {
     TDGL_LAUNCH((k_sect_cg<E, Z, M, T>), grid, blk, k.lds, s, a);        \
     return hipGetLastError();                                            \
   }
-  // the y tiles known when compiled, for the planes that are near square
+  // the y tiles known when compiled, for sectors of one and two z tiles whose elements a thread go with that count on
+  // planes up to twice as wide as deep or so; the others take the generic instance of their tiles a wave (of 5088 and
+  // 5160 elements, 32 iterations: 964 us with, 1046 without)
   TDGL_CG(2, 1, 2, 1) TDGL_CG(2, 1, 2, 2) TDGL_CG(2, 1, 2, 3) TDGL_CG(2, 1, 2, 4) TDGL_CG(4, 1, 2, 2) TDGL_CG(4, 1, 2, 3)
   TDGL_CG(4, 1, 2, 4) TDGL_CG(4, 1, 2, 5) TDGL_CG(6, 1, 2, 3) TDGL_CG(6, 1, 2, 5)
   TDGL_CG(6, 1, 2, 4) TDGL_CG(2, 2, 2, 1) TDGL_CG(4, 2, 2, 2) TDGL_CG(6, 2, 2, 2) TDGL_CG(6, 2, 4, 3) TDGL_CG(8, 2, 4, 3)
   TDGL_CG(10, 2, 4, 4) TDGL_CG(10, 2, 4, 5)
-#define TDGL_CG_Z(E, Z) TDGL_CG(E, Z, 2, 0) TDGL_CG(E, Z, 6, 0)
+#define TDGL_CG_Z(E, Z) TDGL_CG(E, Z, 2, 0) TDGL_CG(E, Z, 4, 0) TDGL_CG(E, Z, 6, 0)
 #define TDGL_CG_E(E) TDGL_CG_Z(E, 1) TDGL_CG_Z(E, 2) TDGL_CG_Z(E, 3)
   TDGL_CG_E(2) TDGL_CG_E(4) TDGL_CG_E(6) TDGL_CG_E(8) TDGL_CG_E(10) TDGL_CG_E(11)
 #undef TDGL_CG_E

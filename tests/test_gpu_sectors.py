@@ -38,10 +38,11 @@ def _core(errs):
 
 # nodes per axis n = cells + 2 buf - 1: three nodes, odd and even counts, half extents at and past whole
 # 16-point tiles (31, 32 | 33, 34 nodes), one to three z tiles (half 16, 17, 33, 46), each elements-a-thread instance
-# (2, 4, 6, 8, 10, 11 x 512), more ghosts than threads (90 x 4 half nodes) and the largest sector (40 x 46 nodes)
+# (2, 4, 6, 8, 10, 11 x 512), more ghosts than threads (90 x 4 half nodes), the largest sector (40 x 46 nodes), and y tiles
+# in rounds: 5 and 6 a wave of 12 x 3, 7 x 5 and 21 x 2
 SIZES = [(2, 2, 2, 1), (5, 4, 3, 2), (9, 13, 8, 2), (20, 12, 28, 2), (17, 29, 30, 2), (33, 30, 31, 2), (34, 31, 29, 2), (12, 60, 28, 2),
          (6, 28, 62, 2), (70, 66, 13, 2), (4, 92, 32, 2), (4, 120, 36, 2),
-         (4, 140, 44, 2), (3, 177, 5, 2), (9, 76, 88, 2)]
+         (4, 140, 44, 2), (3, 177, 5, 2), (9, 76, 88, 2), (3, 360, 14, 2), (4, 220, 30, 2), (2, 640, 5, 2)]
 
 
 @pytest.mark.parametrize("nx,ny,nz,buf", SIZES)
@@ -145,3 +146,29 @@ def test_sectors_match_the_oracle(tol, maxit, bound, monkeypatch):
     errs = compare_states(got, o.get_state())
     print(f"[gpu] sectors against the oracle, tol {tol:g}: {_core(errs):.2e}", flush=True)
     assert _core(errs) <= bound, errs
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(200, 110, 34), (200, 250, 4), (8, 640, 5), (16, 60, 88)])
+def test_sectors_are_no_slower_than_the_general_iteration(nx, ny, nz, monkeypatch):
+    """Planes of three to six y tiles a wave: a step by sectors takes no longer than the general iteration's (half of it,
+    measured; the best of four calls a side)."""
+    from juliatdgl_amd.hip import HipStepper
+    gr = Grid.make(nx, ny, nz, dx=0.5, buf=2)
+    best = {}
+    for sect in ("0", None):
+        if sect:
+            monkeypatch.setenv("TDGL_HIP_SECT", sect)
+        else:
+            monkeypatch.delenv("TDGL_HIP_SECT", raising=False)
+        st = make_stepper(mgb2(), gr, box_masks(gr), sigma_vac=0.01)
+        d = HipStepper(st)
+        d.upload(seeded_state(st.model, st.grid, st.masks, 0.03, seed=1))
+        ms = []
+        for _ in range(6):
+            t = d.stats()["device_ms"]
+            d.step(6, 0.03, st.selffield(0.3))
+            ms.append((d.stats()["device_ms"] - t) / 6)
+        d.close()
+        best[sect] = min(ms[2:])
+    print(f"[gpu] {nx}x{ny}x{nz}: general {1e3 * best['0']:.0f} us a step, sectors {1e3 * best[None]:.0f}", flush=True)
+    assert best[None] <= best["0"]
