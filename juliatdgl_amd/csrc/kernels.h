@@ -678,11 +678,13 @@ struct BatchRec {
   bool has_grid;  // grid and lds as the launcher chose them (else batch_grid, no dynamic LDS)
   dim3 grid;
   size_t lds;
+  int phase;      // of its step sequence (Recorder::phase)
   Geo g;
   std::vector<unsigned char> args;
 };
 struct Recorder {
   std::vector<BatchRec> recs;
+  int phase = 0;  // even: the launches every run makes alike; odd: a run's own solve of the field
 };
 extern thread_local Recorder *g_rec;
 hipError_t record(int kind, const Geo &g, const void *args, size_t bytes, int variant = 0, bool has_grid = false,

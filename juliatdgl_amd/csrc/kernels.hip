@@ -18,6 +18,7 @@ hipError_t record(int kind, const Geo &g, const void *args, size_t bytes, int va
   r.has_grid = has_grid;
   r.grid = grid;
   r.lds = lds;
+  r.phase = g_rec->phase;
   r.g = g;
   r.args.assign((const unsigned char *)args, (const unsigned char *)args + bytes);
   g_rec->recs.push_back(std::move(r));

@@ -177,6 +177,7 @@ struct tdgl_handle {
   float *syb[2][2][2] = {}, *szb[2][2][2] = {};  // SectCG::yb, zb
   double *sydb[2][2][2] = {}, *szdb[2][2][2] = {};  // SectSep::yb, zb
   bool sepsect = false;        // the separable solve by sectors (k_sect_sep)
+  bool folds64 = false;        // the transforms of the separable solve are the folded ones (also where it goes by sectors)
   int syp = 0, szp = 0;
   unsigned char *scode[3] = {};
   double *spal = nullptr;
@@ -2009,7 +2010,9 @@ int step_once(tdgl_handle *h) {
     PL(K_FIELD, launch_field(h->g, fa, h->s));
   if (d.field_mode == TDGL_FIELD_SEPARABLE) {
     SepOut o{nullptr, true, 0};
+    if (g_rec) ++g_rec->phase;
     CHK(sep_solve(h, h->B, o, nullptr, false, Conv{CONV_NONE, nullptr, nullptr, 0}));
+    if (g_rec) ++g_rec->phase;
   } else if (d.field_mode == TDGL_FIELD_PCG) {
     CHK(implicit_pcg(h, started));
   }
@@ -3041,11 +3044,13 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
     const bool fold64_pays = l0max > 160 || l1max > 96;
     const bool fold64_on = gf64 ? gf64[0] == '1' : fold64_pays;
     if (d.field_mode == TDGL_FIELD_SEPARABLE && !(zc && zc[0] == '0')) h->zcols = 1;
-    if (d.field_mode == TDGL_FIELD_SEPARABLE) CHK(sepsect_setup(h, fold64_pays));
-    if (!h->sepsect && d.field_mode == TDGL_FIELD_SEPARABLE && h->plane64 && fold64_on && d.Nz - 1 >= 2 && d.Nz - 1 <= ZQ64_NZ_MAX) {
+    if (d.field_mode == TDGL_FIELD_SEPARABLE) {
       int qe[12][3];
       const Quarters q = quarters_of(rg, qe);
-      if (plane_fits<double>(qe, 12) && fold_blocks(q) <= MAX_PART && (size_t)q.total <= h->t12cap) {
+      h->folds64 = h->plane64 && fold64_on && d.Nz - 1 >= 2 && d.Nz - 1 <= ZQ64_NZ_MAX && plane_fits<double>(qe, 12) &&
+                   fold_blocks(q) <= MAX_PART && (size_t)q.total <= h->t12cap;
+      CHK(sepsect_setup(h, fold64_pays));
+      if (h->folds64 && !h->sepsect) {
         h->q = q;
         const int nn[2] = {d.Nx - 1, d.Ny - 1};
         for (int ax = 0; ax < 2; ++ax) {
@@ -3954,10 +3959,14 @@ struct LaunchPlan {
   size_t lds;
   size_t off, dims, g, args;
   int pos;  // the position in the step sequence: the instances of one position are independent
+  int phase, branch, branches;  // of a phase whose runs take several paths: this path's branch
 };
-// The steps of a call are recorded once per run (the launches its own step would make, with the
-// single-axis passes of the separable solve), checked to be the same sequence of kernels in
-// every run, laid out as one table per launch (block offsets, each run's grid, Geo and argument
+// The steps of a call are recorded once per run (the launches its own step would make; the
+// single-axis passes of the separable solve where the runs' transforms differ), checked to be the
+// same sequence of kernels in every run but for the solve of the field, which each run makes by its
+// own path (a branch of the graph each: 170x100x30 cells by sectors and 170x100x20 by the folds take 385 us a step,
+// 418 with a fork and join a launch; 621 when a run by sectors made all take the single-axis passes, 423 when both
+// took the folds; 256x128x32 and 256x128x20 870, 1337 and 1020), laid out as one table per launch (block offsets, each run's grid, Geo and argument
 // struct) and captured as a graph of one batched launch per position; the graph is replayed
 // while the steps per call and every run's parity stay the same.
 struct tdgl_batch {
@@ -3972,7 +3981,7 @@ struct tdgl_batch {
   Block tab{};                 // device tables of the graph's launches
   std::vector<LaunchPlan> plans;  // the launches of gn steps (replayed eagerly under TDGL_HIP_GRAPH=0)
   bool graphs = true;
-  bool tx_only = false;           // the runs differ in their transform passes: single-axis ones in all
+  bool tx_only = false;           // the runs differ in their transforms (folded, planes): single-axis passes in all
   Block mtab{}, mstage{};      // device tables of the meter's launches, their pinned staging
   Block dH{}, hH{};            // (H, HJ) of every run: device, pinned host
   Block drec{}, hrec{};        // the meter's records: device, pinned host
@@ -4078,49 +4087,78 @@ int batch_graph(tdgl_batch *b, int m) {
     restore(h, start);
     if (rc) return fail(rc, "batch: run %d cannot be batched: %s", r, g_err.c_str());
   }
-  const size_t P = rec[0].recs.size();
-  for (int r = 1; r < R; ++r) {
-    if (rec[r].recs.size() != P) return fail(TDGL_E_ARG, "batch: run %d makes %zu launches a call, run 0 %zu", r, rec[r].recs.size(), P);
-    for (size_t q = 0; q < P; ++q)
-      if (rec[r].recs[q].kind != rec[0].recs[q].kind) return fail(TDGL_E_ARG, "batch: run %d differs from run 0 at launch %zu", r, q);
+  // the runs' launches by phase: the phases of a step that every run makes alike hold the same kernels in every run,
+  // the solve of the field each run's own
+  const int phases = rec[0].phase + 1;
+  std::vector<std::vector<std::vector<const BatchRec *>>> seq(R, std::vector<std::vector<const BatchRec *>>(phases));
+  for (int r = 0; r < R; ++r) {
+    if (rec[r].phase + 1 != phases) return fail(TDGL_E_ARG, "batch: run %d makes %d phases a call, run 0 %d", r, rec[r].phase + 1, phases);
+    for (const BatchRec &br : rec[r].recs) seq[r][br.phase].push_back(&br);
   }
-  // one launch per position and kernel instance (the plane and z-mode passes have several)
+  for (int r = 1; r < R; ++r)
+    for (int f = 0; f < phases; f += 2) {
+      const auto &x = seq[r][f], &y = seq[0][f];
+      if (x.size() != y.size()) return fail(TDGL_E_ARG, "batch: run %d makes %zu launches in phase %d, run 0 %zu", r, x.size(), f, y.size());
+      for (size_t q = 0; q < x.size(); ++q)
+        if (x[q]->kind != y[q]->kind) return fail(TDGL_E_ARG, "batch: run %d differs from run 0 at launch %zu of phase %d", r, q, f);
+    }
+  // one launch per position of a path and kernel instance (the plane and z-mode passes have several)
   TabBuild tb;
   std::vector<LaunchPlan> plans;
   std::vector<CurlArgs> curl(R);
-  for (size_t q = 0; q < P; ++q) {
-    const int kind = rec[0].recs[q].kind;
-    std::vector<int> variants;
+  int pos = 0;
+  for (int f = 0; f < phases; ++f) {
+    // the runs by the kernels they launch in this phase: a branch each
+    std::vector<std::vector<int>> paths;
+    auto alike = [&](int r, int o) {
+      const auto &x = seq[r][f], &y = seq[o][f];
+      return x.size() == y.size() &&
+             std::equal(x.begin(), x.end(), y.begin(), [](const BatchRec *u, const BatchRec *v) { return u->kind == v->kind; });
+    };
     for (int r = 0; r < R; ++r) {
-      const BatchRec &br = rec[r].recs[q];
-      if (br.args.size() != batch_args_size(kind)) return fail(TDGL_E_ARG, "batch: launch %zu has the wrong argument size", q);
-      if (std::find(variants.begin(), variants.end(), br.variant) == variants.end()) variants.push_back(br.variant);
+      size_t k = 0;
+      while (k < paths.size() && !alike(r, paths[k][0])) ++k;
+      if (k == paths.size()) paths.emplace_back();
+      paths[k].push_back(r);
     }
-    for (int v : variants) {
-      std::vector<Geo> gs;
-      std::vector<const void *> args;
-      std::vector<dim3> grids;
-      size_t lds = 0;
-      for (int r = 0; r < R; ++r) {
-        const BatchRec &br = rec[r].recs[q];
-        if (br.variant != v) continue;
-        const void *a = br.args.data();
-        if (kind == BK_CURL) {
-          // the field boundary reads the run's (H, HJ) from the batch's array
-          std::memcpy(&curl[r], br.args.data(), sizeof(CurlArgs));
-          curl[r].hp = (double *)b->dH.p + 2 * r;
-          a = &curl[r];
+    for (size_t k = 0; k < paths.size(); ++k)
+      for (size_t q = 0; q < seq[paths[k][0]][f].size(); ++q, ++pos) {
+        const int kind = seq[paths[k][0]][f][q]->kind;
+        std::vector<int> variants;
+        for (int r : paths[k]) {
+          const BatchRec &br = *seq[r][f][q];
+          if (br.args.size() != batch_args_size(kind)) return fail(TDGL_E_ARG, "batch: launch %d has the wrong argument size", pos);
+          if (std::find(variants.begin(), variants.end(), br.variant) == variants.end()) variants.push_back(br.variant);
         }
-        gs.push_back(br.g);
-        args.push_back(a);
-        grids.push_back(br.has_grid ? br.grid : batch_grid(kind, br.g, a));
-        lds = std::max(lds, br.lds);
+        for (int v : variants) {
+          std::vector<Geo> gs;
+          std::vector<const void *> args;
+          std::vector<dim3> grids;
+          size_t lds = 0;
+          for (int r : paths[k]) {
+            const BatchRec &br = *seq[r][f][q];
+            if (br.variant != v) continue;
+            const void *a = br.args.data();
+            if (kind == BK_CURL) {
+              // the field boundary reads the run's (H, HJ) from the batch's array
+              std::memcpy(&curl[r], br.args.data(), sizeof(CurlArgs));
+              curl[r].hp = (double *)b->dH.p + 2 * r;
+              a = &curl[r];
+            }
+            gs.push_back(br.g);
+            args.push_back(a);
+            grids.push_back(br.has_grid ? br.grid : batch_grid(kind, br.g, a));
+            lds = std::max(lds, br.lds);
+          }
+          LaunchPlan lp{};
+          CHK(plan_launch(kind, v, lds, gs, args, grids, tb, lp));
+          lp.pos = pos;
+          lp.phase = f;
+          lp.branch = (int)k;
+          lp.branches = (int)paths.size();
+          plans.push_back(lp);
+        }
       }
-      LaunchPlan lp{};
-      CHK(plan_launch(kind, v, lds, gs, args, grids, tb, lp));
-      lp.pos = (int)q;
-      plans.push_back(lp);
-    }
   }
   Block stage{};
   const int rc = upload_tabs(b, tb, b->tab, stage);
@@ -4139,7 +4177,7 @@ int batch_graph(tdgl_batch *b, int m) {
   for (size_t q = 0; q < plans.size();) {
     size_t e = q;
     while (e < plans.size() && plans[e].pos == plans[q].pos) ++e;
-    width = std::max(width, e - q);
+    width = std::max({width, e - q, (size_t)plans[q].branches});
     q = e;
   }
   if (forks) {
@@ -4155,12 +4193,31 @@ int batch_graph(tdgl_batch *b, int m) {
   }
   HIPCHK(hipStreamBeginCapture(b->s, hipStreamCaptureModeRelaxed));
   hipError_t le = hipSuccess;
+  auto launch = [&](const LaunchPlan &lp, hipStream_t st) {
+    return launch_batch(lp.kind, lp.variant, lp.lds, tab_of(b->tab, lp), lp.blocks, st);
+  };
   for (size_t q = 0; q < plans.size() && le == hipSuccess;) {
     size_t e = q;
+    if (forks && plans[q].branches > 1) {
+      // the paths of a phase side by side, one fork and join for all their launches
+      const int f = plans[q].phase, nb = plans[q].branches;
+      while (e < plans.size() && plans[e].phase == f) ++e;
+      le = hipEventRecord(b->fork, b->s);
+      for (int k = nb - 1; k >= 0 && le == hipSuccess; --k) {
+        hipStream_t st = k ? b->side[k - 1] : b->s;
+        if (k) le = hipStreamWaitEvent(st, b->fork, 0);
+        for (size_t u = q; u < e && le == hipSuccess; ++u)
+          if (plans[u].branch == k) le = launch(plans[u], st);
+        if (k && le == hipSuccess) le = hipEventRecord(b->join[k - 1], st);
+      }
+      for (int k = 1; k < nb && le == hipSuccess; ++k) le = hipStreamWaitEvent(b->s, b->join[k - 1], 0);
+      q = e;
+      continue;
+    }
     while (e < plans.size() && plans[e].pos == plans[q].pos) ++e;
     if (!forks || e - q == 1) {
       for (; q < e && le == hipSuccess; ++q)
-        le = launch_batch(plans[q].kind, plans[q].variant, plans[q].lds, tab_of(b->tab, plans[q]), plans[q].blocks, b->s);
+        le = launch(plans[q], b->s);
       continue;
     }
     // fork: instance k >= 1 on side stream k - 1 after the fork event, the first on s; join
@@ -4169,11 +4226,10 @@ int batch_graph(tdgl_batch *b, int m) {
       const LaunchPlan &lp = plans[q + k];
       hipStream_t st = b->side[k - 1];
       le = hipStreamWaitEvent(st, b->fork, 0);
-      if (le == hipSuccess) le = launch_batch(lp.kind, lp.variant, lp.lds, tab_of(b->tab, lp), lp.blocks, st);
+      if (le == hipSuccess) le = launch(lp, st);
       if (le == hipSuccess) le = hipEventRecord(b->join[k - 1], st);
     }
-    if (le == hipSuccess)
-      le = launch_batch(plans[q].kind, plans[q].variant, plans[q].lds, tab_of(b->tab, plans[q]), plans[q].blocks, b->s);
+    if (le == hipSuccess) le = launch(plans[q], b->s);
     for (size_t k = 1; k < e - q && le == hipSuccess; ++k) le = hipStreamWaitEvent(b->s, b->join[k - 1], 0);
     q = e;
   }
@@ -4214,7 +4270,9 @@ int tdgl_batch_create(tdgl_handle *const *hs, int32_t n, tdgl_batch **out) {
   b->dev = hs[0]->dev;
   const char *ge = std::getenv("TDGL_HIP_GRAPH");  // =0: the batched launches from the host (profiling)
   b->graphs = !(ge && ge[0] == '0');
-  for (int r = 1; r < n; ++r) b->tx_only |= hs[r]->plane64 != hs[0]->plane64 || hs[r]->fold64 != hs[0]->fold64 || hs[r]->sepsect != hs[0]->sepsect;
+  bool sectors = true;  // every run's solve
+  for (int r = 0; r < n; ++r) sectors = sectors && hs[r]->sepsect;
+  for (int r = 1; r < n; ++r) b->tx_only |= hs[r]->plane64 != hs[0]->plane64 || (!sectors && hs[r]->folds64 != hs[0]->folds64);
   auto bail = [&](int rc) {
     tdgl_batch_destroy(b);
     return rc;

@@ -277,7 +277,7 @@ def run_batch(specs: List[RunSpec], work: Callable, workers: int = 8):
 def run_batched(specs: List[RunSpec], work: "Cycles", group: int = 64, workers: int = 8, lanes: int = 1):
     """Every run of `specs` with batched kernels (tdgl_batch_*): groups of `group` runs advanced
     together, one launch per kernel of a step over the group's runs of each path of the separable
-    solve (with or without the parity folds: one batch per path).  With lanes = 1 host threads
+    solve (by sectors, with the parity folds or without: one batch per path).  With lanes = 1 host threads
     set up the next group (stepper, state, upload, meter) while the current one runs; with
     lanes > 1 that many groups step at once, each batch on its own stream (their launches overlap
     on the device, so one batch's slowest blocks do not idle it), each lane setting up its next
@@ -310,9 +310,9 @@ def run_batched(specs: List[RunSpec], work: "Cycles", group: int = 64, workers: 
             batch.close()
 
     def advance(ready):
-        # one batch per path of the separable solve (the parity folds, which a handle takes on planes
-        # too large for the full-length kernel, or not): a batch of one path launches what each run's
-        # own step launches, so every record equals the run's alone
+        # one batch per path of the separable solve (sectors, or the parity folds, which a handle takes on
+        # planes too large for the full-length kernel, or neither): a batch of one path launches what each
+        # run's own step launches, so every record equals the run's alone
         out = {}
         try:
             parts = {}

@@ -80,3 +80,28 @@ def test_batched_sectors(sizes, monkeypatch):
             assert max(v for k, v in errs.items() if not k.startswith(("U", "V"))) <= 1e-12, errs
     for _, d in runs:
         d.close()
+
+
+def test_batched_sectors_beside_folds():
+    """Wide runs, some by sectors and some by the folded transforms, in one batch: each is where its own steps
+    leave it, to the bit."""
+    from juliatdgl_amd.hip import HipBatch
+    sizes, H = [(170, 100, 30), (170, 100, 20), (60, 200, 14)], 0.03
+    print(f"[gpu] batched sectors beside folds {sizes}", flush=True)
+    alone = []
+    for st, d in _steppers(sizes):
+        d.step(4, H, st.selffield(0.3))
+        alone.append((d.download(), d.stats()["folded"]))
+        d.close()
+    assert [f for _, f in alone] == [2, 1, 2]
+    runs = _steppers(sizes)
+    b = HipBatch([d for _, d in runs])
+    for _ in range(2):
+        b.step(2, np.full(len(runs), H), np.array([st.selffield(0.3) for st, _ in runs]))
+    got = [d.download() for _, d in runs]
+    b.close()
+    for _, d in runs:
+        d.close()
+    for (x, _), y in zip(alone, got):
+        for (k, u), (_, v) in zip(x.arrays(), y.arrays()):
+            assert np.array_equal(u, v), k
