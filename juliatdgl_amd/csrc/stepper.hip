@@ -2618,8 +2618,13 @@ void sect_yz_tables(tdgl_handle *h, T *(&yb)[2][2][2], T *(&zb)[2][2][2], Put &&
 // the x passes' blocks: 62.0 / 72.7 (161x30x8 cells, 30 blocks), 157 / 168 (200x100x16, 189), 169 / 171 (200x60x32, 204),
 // 197 / 210 (250x100x20, 231), 163 / 170 (150x128x18, 270), 228 / 212 (200x100x24, 273), 197 / 180 (180x60x44, 276),
 // 118 / 93 (60x200x14, 312), 225 / 193 (170x100x30, 336), 294 / 288 (200x100x32, 357), 584 / 459 (256x128x32, 459),
-// 1431 / 747 (256x128x60, 837).
-constexpr int SECT_SEP_BLOCKS = 300;
+// 1431 / 747 (256x128x60, 837).  300 is the count from which every measured plane gains; at 270 to 276 the deeper ones
+// gain 7 to 9 % and the thin one loses 4 %.  Planes the folds do not take (deeper than ZQ64_NZ_MAX) go by sectors from
+// SECT_SEP_NARROW blocks of k_sect_sep on, below which their few workgroups leave the chip to the planes' passes, planes
+// against sectors: 145 / 150 (4x128x64 cells, 20 blocks), 152 / 156 (8x128x64, 36), 201 / 212 (6x170x80, 28), 151 / 148
+// (12x128x64, 52), 168 / 151 (16x128x64, 68).  Where the folds are what they replace the sectors gain at any width:
+// 129 / 105 (4x128x40), 124 / 107 (8x223x20).
+constexpr int SECT_SEP_BLOCKS = 300, SECT_SEP_NARROW = 48;
 int sepsect_setup(tdgl_handle *h, bool wide) {
   const tdgl_desc &d = h->d;
   const char *off = std::getenv("TDGL_HIP_SECT");
@@ -2630,7 +2635,7 @@ int sepsect_setup(tdgl_handle *h, bool wide) {
   h->sq = sect_dims(d.Nx - 1, d.Ny - 1, d.Nz - 1);
   h->syp = 16 * cdiv(h->sq.hy[0][0], 16);
   h->szp = 16 * cdiv(h->sq.hz[0][0], 16);
-  if (!force && sect_x_blocks(sect_x(h, false)) < SECT_SEP_BLOCKS) return 0;
+  if (!force && (sect_x_blocks(sect_x(h, false)) < SECT_SEP_BLOCKS || (!h->folds64 && 4 * h->sq.nx < SECT_SEP_NARROW))) return 0;
   if (!sect_x_fits(sect_x(h, false)) || !sect_sep_fits(sect_sep(h)) || (size_t)h->sq.total > h->t12cap) return 0;
   std::vector<unsigned char> all;
   std::vector<std::pair<void *, size_t>> tabs;

@@ -105,3 +105,14 @@ def test_batched_sectors_beside_folds():
     for (x, _), y in zip(alone, got):
         for (k, u), (_, v) in zip(x.arrays(), y.arrays()):
             assert np.array_equal(u, v), k
+
+
+@pytest.mark.parametrize("size,by_sectors", [((4, 128, 64), False), ((10, 128, 64), False), ((6, 170, 80), False),
+                                             ((11, 128, 64), True), ((4, 128, 40), True), ((60, 200, 14), True)])
+def test_few_sectors_keep_the_planes(size, by_sectors):
+    """Deep planes, which the folds do not take, go by sectors from 48 workgroups on (12 nodes along x); where the folds
+    are the other way, at any width."""
+    (_, d), = _steppers([size])
+    folded = d.stats()["folded"]
+    d.close()
+    assert (folded == 2) == by_sectors, folded
