@@ -163,8 +163,10 @@ typedef struct {
    * folded Float32 preconditioner): each round solves A d = b − A x to pcg_inner_tol of its starting
    * residual, x += d, until ||b − A x|| <= pcg_tol ||b|| in FP64.  A captured cycle holds pcg_rounds
    * rounds (1..16).  Needs pcg_f32 and the folded preconditioner; 0 keeps the reference's solver.
-   * Where D is constant along x and mirror-symmetric the solve goes by sectors with or without it: every
-   * vector is then FP64, the tolerance holds in FP64, and pcg_rounds and pcg_inner_tol shape nothing. */
+   * Where D is constant along x and mirror-symmetric and pcg_tol is 1e-12 or more the solve goes by sectors
+   * with or without it: r, x and the directions are then FP64, b − A x is formed once and each sector stops
+   * on the residual of its recursion at a 128th of the tolerance (which covers the rounding between the two,
+   * 1.6e-14 ||b|| at most as measured), and pcg_rounds and pcg_inner_tol shape nothing. */
   int32_t pcg_refine;
   int32_t pcg_rounds;
   double pcg_inner_tol;

@@ -2659,9 +2659,14 @@ int sepsect_setup(tdgl_handle *h, bool wide) {
 // direction, D constant along x and equal to its mirror images in y and z on the unknowns (what
 // link_conductivity gives, implicit.jl:126-140), at most DPAL_MAX values of D a component, and a sector that
 // fits a workgroup.  The variables that shape the general iteration select it, as TDGL_HIP_SECT=0 does.
+// A refinement promises ||b − A x|| <= tol ||b|| of the residual itself, and its rounds form it anew in FP64.  The
+// sectors form it once and stop on the residual of their recursion, at a 128th of the tolerance; what rounding
+// leaves between the two came to 4e-15 of ||b|| (33x20x9 cells) to 1.6e-14 (256x128x32), the rounds' own floor to 1.1e-15.
+// Tolerances below REFINE_SECT_TOL, which that gap comes near, keep the rounds.
+constexpr double REFINE_SECT_TOL = 1e-12;
 int sect_setup(tdgl_handle *h) {
   const tdgl_desc &d = h->d;
-  if (d.field_mode != TDGL_FIELD_PCG || !d.pcg_f32) return 0;
+  if (d.field_mode != TDGL_FIELD_PCG || !d.pcg_f32 || (d.pcg_refine && d.pcg_tol < REFINE_SECT_TOL)) return 0;
   const char *off = std::getenv("TDGL_HIP_SECT");
   if (off && off[0] == '0') return 0;
   for (const char *v : {"TDGL_HIP_BUDGET", "TDGL_HIP_FOLD", "TDGL_HIP_QPLANE", "TDGL_HIP_QPARTS", "TDGL_HIP_ZQ_WAVES", "TDGL_HIP_PLANE",

@@ -830,7 +830,8 @@ def make_stepper(md: Model, gr: Grid, mk: Masks, *, implicit=True, substeps=None
     `pcg_refine` (an extension of the PCG solver, with pcg_f32 and the insulating padding): the FP64
     operator, residual and solution refine around Float32 inner PCG solves, each to `pcg_inner_tol`
     of its starting residual, until ||b − A x|| <= pcg_tol ||b||; `pcg_rounds` rounds a captured
-    solve holds (a solve by sectors keeps FP64 vectors throughout and needs neither)."""
+    solve holds (a solve by sectors, at a tolerance of 1e-12 or more, keeps FP64 vectors throughout and
+    needs neither)."""
     for k, v in unsupported.items():
         if v is not None and v is not False:
             raise NotImplementedError(f"Stepper option {k!r} is not run by the HIP stepper")

@@ -75,6 +75,46 @@ def test_refinement_rolls_back_a_short_budget(monkeypatch):
     assert max(core.values()) <= tol, errs
 
 
+@pytest.mark.parametrize("tol", [1e-12, 2e-15])
+def test_refinement_meets_its_tolerance(tol):
+    """||b − A x|| of the returned solution, b from an all-FP64 solve of the same step to 1e-15 and A from its
+    definition: within pcg_tol, and the rounding of that b and of the product (2e-15), also where the tolerance
+    is near the rounding (the rounds then run, not the sectors)."""
+    from juliatdgl_amd.scheme import Grid, box_masks, make_stepper
+    from juliatdgl_amd.state import seeded_state
+    from cases import mgb2
+    from test_oracle_pcg import flat, operator
+    HipStepper = _hip()
+    gr = Grid.make(53, 27, 9, dx=0.5, buf=2)
+    kw = dict(sigma_vac=0.01)
+    st = make_stepper(mgb2(), gr, box_masks(gr), pcg_refine=True, pcg_tol=tol, **kw)
+    H, HJ = 0.03, st.selffield(0.3)
+    print(f"[gpu] refinement's residual, tol {tol:g}", flush=True)
+    a = HipStepper(st)
+    a.upload(seeded_state(st.model, gr, st.masks, H, seed=3))
+    a.step(6, H, HJ)
+    s1, p1 = a.download(), a.get_pcg()
+    a.step(1, H, HJ)
+    x = flat(a.get_pcg().x)
+    a.profile(True)
+    a.step(1, H, HJ)
+    by_sectors = a.profile_get()["pcg_sectors"][0]
+    a.profile(False)
+    a.close()
+    st64 = make_stepper(mgb2(), gr, box_masks(gr), pcg_tol=1e-15, pcg_fast=False, pcg_f32=False, **kw)
+    b = HipStepper(st64)
+    b.upload(s1)
+    b.set_pcg(p1)
+    b.step(1, H, HJ)
+    xs = flat(b.get_pcg().x)
+    b.close()
+    A = operator(st, st.D)
+    res = np.linalg.norm(A @ (xs - x)) / np.linalg.norm(A @ xs)
+    print(f"    ||b - A x|| / ||b|| {res:.2e}, by sectors {by_sectors}", flush=True)
+    assert by_sectors == (1 if tol >= 1e-12 else 0)
+    assert res <= tol + 2e-15
+
+
 def test_refinement_against_all_fp64_on_the_three_band_workload():
     """The three-band anisotropic open-boundary workload (buf 8, tol 1e-8) on 48x24x8 cells: the
     refinement against an all-FP64 run (FP64 preconditioner) after 80 steps; ψ and A agree to the
