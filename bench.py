@@ -111,11 +111,9 @@ def quarter_total(gr):
     return sum(4 * h0 * h1 * e2 for h0, h1, e2 in quarters(gr))
 
 
-def solved_by_sectors(prof, folded: int):
-    """"pcg" or "sep" where the field solve went by sectors, else None."""
-    if prof["pcg_sectors"][0]:
-        return "pcg"
-    return "sep" if folded == 2 else None
+def solved_by_sectors(st, folded: int):
+    """"pcg" or "sep" where the field solve goes by sectors (tdgl_stats.folded), else None."""
+    return ("pcg" if st.field_mode == 2 else "sep") if folded == 2 else None
 
 
 def kernel_flops(st, name: str, launches: int, folded: bool = False, sect=None) -> float:
@@ -432,14 +430,15 @@ def run_workload(name, steps, warmup, profile=True, cpu_steps=0, profile_out=Non
     cells = st.grid.cells
     value = cells * steps / wall
     nodes = (st.grid.Nx + 1) * (st.grid.Ny + 1) * (st.grid.Nz + 1)
-    balg = cycle_bytes_per_node_step(st, iters / nsteps)
+    sect, folded = solved_by_sectors(st, int(st1["folded"])), int(st1["folded"]) == 1
+    balg = cycle_bytes_per_node_step(st, iters / nsteps, sect)
     out = {"value": value, "wall": wall, "steps": steps, "st": st, "nsteps": nsteps, "iters": iters,
            "config": {"workload": desc, "cells": cells, "lmax": LMAX, "pcg_iters_per_step": iters / nsteps,
                       "device_ms_per_cycle": dev_ms / steps, "padded_nodes": nodes, "cell_steps_per_s": value * LMAX,
                       "b_alg_per_node_step": balg,
                       "hbm_roofline_frac_cycle": balg * nodes * LMAX * steps / wall / HBM_PEAK,
                       "ms_per_time_step": 1e3 * wall / nsteps, "timed_rollbacks": rollbacks,
-                      "timed_graph_captures": captures, "pcg_budget": st1.get("pcg_budget"),
+                      "timed_graph_captures": captures, "pcg_budget": st1.get("pcg_budget"), "solved_by_sectors": sect,
                       "tuned": None if tuned is None else {k: tuned[k] for k in ("box_kc", "plane_mt", "zmodes_waves",
                                                                                  "qparts", "fold", "zcol")},
                       **({"pcg_refine": {"inner_tol": st.pcg_inner_tol, "rounds": st.pcg_rounds}}
@@ -458,14 +457,8 @@ def run_workload(name, steps, warmup, profile=True, cpu_steps=0, profile_out=Non
                 print(f"[bench]   {kname:20s} {nl:8d} launches {ms:10.3f} ms ({100 * ms / tot:5.1f}%) "
                       f"{1e3 * ms / nl:8.2f} us/launch", file=sys.stderr)
         dom, (nl, ms) = rows[0]
-        sect = solved_by_sectors(prof, int(st1.get("folded", 0)))
-        out["roofline"] = roofline(st, dom, nl, ms, nsteps, iters, name, bool(st1.get("folded", 0)), sect)
-        out["config"]["solved_by_sectors"] = sect
-        if sect:
-            balg = cycle_bytes_per_node_step(st, iters / nsteps, sect)
-            out["config"]["b_alg_per_node_step"] = balg
-            out["config"]["hbm_roofline_frac_cycle"] = balg * nodes * LMAX * steps / wall / HBM_PEAK
-        out["config"]["folded_preconditioner"] = bool(st1.get("folded", 0))
+        out["roofline"] = roofline(st, dom, nl, ms, nsteps, iters, name, folded, sect)
+        out["config"]["folded_preconditioner"] = folded
         out["config"]["kernel_ms_per_cycle"] = {k: v[1] / steps for k, v in prof.items() if v[0]}
         # every class with algorithmic bytes: its average launch against the HBM peak (and the
         # transforms against the matrix peak)
@@ -474,12 +467,12 @@ def run_workload(name, steps, warmup, profile=True, cpu_steps=0, profile_out=Non
             if not nl_k:
                 continue
             b = kernel_bytes(st, kname, nl_k, nsteps, {"iters_per_solve": iters / nsteps,
-                                                       "folded": bool(st1.get("folded", 0)), "sect": sect}) / nl_k
+                                                       "folded": folded, "sect": sect}) / nl_k
             if b <= 0:
                 continue
             us = 1e3 * ms_k / nl_k
             row = {"us_per_launch": us, "bytes_per_launch": b, "GB_s": b / us / 1e3, "hbm_frac": b / us / 1e3 / (HBM_PEAK / 1e9)}
-            f = kernel_flops(st, kname, nl_k, bool(st1.get("folded", 0)), sect) / nl_k
+            f = kernel_flops(st, kname, nl_k, folded, sect) / nl_k
             if f > 0:
                 pk = FP32_MFMA_PEAK if kname in ("sep_transform_f32", "sep_modes") else FP64_PEAK
                 row["TFLOP_s"] = f / us / 1e6

@@ -213,8 +213,8 @@ typedef struct {
   int32_t pcg_budget;   /* PCG iterations per solve in the captured cycle (a solve by sectors runs to its end on
                            the device whatever they are: what the general iteration would hold) */
   int64_t captures;     /* graphs captured and instantiated (the last four are kept and replayed) */
-  int32_t folded;       /* 1: the Float32 preconditioner (or the separable solve) runs its parity-folded
-                         * transforms; 2: the separable solve goes by sectors */
+  int32_t folded;       /* what the steps run: 2: the field solve (PCG or separable) goes by sectors; 1: the
+                         * Float32 preconditioner or the separable solve takes its parity-folded transforms */
 } tdgl_stats;
 
 typedef struct tdgl_handle tdgl_handle;
@@ -260,8 +260,9 @@ int tdgl_step_noalloc(tdgl_handle *h, int32_t n, double H, double HJ);
  * and the folds how the preconditioner rounds (each agrees with the others to the PCG tolerance);
  * the m tiles, the vector ALUs' waves, qparts and zcol change no result.  cand[] lists every candidate
  * timed (us per launch of the kernels it shapes; per PCG iteration for fold and zcol).  A stepper whose
- * steps solve by sectors (D constant along x and mirror-symmetric) keeps doing so: of the choices only
- * box_kc, the blocks of its residual kernel, reaches its steps. */
+ * steps solve by sectors (D constant along x and mirror-symmetric) keeps doing so (fold 2): of the choices
+ * only box_kc reaches its steps, and is timed on them (us of the start and the residual); the others are the
+ * general iteration's. */
 #define TDGL_TUNE_MAX 16
 enum { TDGL_TUNE_BOX_KC = 1, TDGL_TUNE_PLANE_MT = 2, TDGL_TUNE_ZMODES_WAVES = 3, TDGL_TUNE_FOLD = 4,
        TDGL_TUNE_ZCOL = 5, TDGL_TUNE_QPARTS = 6 };
@@ -273,7 +274,7 @@ typedef struct {
   int32_t box_kc, plane_mt, zmodes_waves;
   int32_t ncand;
   tdgl_tune_cand cand[TDGL_TUNE_MAX];
-  int32_t fold, zcol;  /* the preconditioner's path chosen */
+  int32_t fold, zcol;  /* the preconditioner's path chosen (fold 2: the steps solve by sectors) */
   int32_t qparts;      /* blocks a folded quarter plane's x-y transform is split over */
 } tdgl_tuning;
 int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out);

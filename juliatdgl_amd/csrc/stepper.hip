@@ -3443,13 +3443,13 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
   HIPCHK(hipMemcpyAsync(h->hp, h->hph, 2 * sizeof(double), hipMemcpyHostToDevice, h->s));
   const HostSnap start = snap(h);
   const int last_iters = h->last_iters;
-  // the shapes are the general iteration's, also where the steps solve by sectors (which have none to choose)
+  // where the steps solve by sectors their box levels are timed on those steps; the other shapes are the general
+  // iteration's (a solve by sectors has none of them), which a tune sets up and times all the same
   struct SectScope {
     tdgl_handle *h;
     bool on;
     ~SectScope() { h->sect = on; }
   } sect_scope{h, h->sect};
-  h->sect = false;
   if (!h->general) {
     CHK(general_setup(h));
     CHK(flush(h));
@@ -3473,7 +3473,8 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
     h->last_iters = last_iters;
     PL(K_VEC, launch_pcg_cycle_reset(h->pd, h->s));
     CHK(tdgl_profile_enable(h, 1));
-    const int rc = steps_eager(h, 1);
+    // by sectors a step launches the box kernels (the start and the residual) once each: four steps
+    const int rc = steps_eager(h, h->sect ? 4 : 1);
     tdgl_profile p{};
     const int rc2 = rc ? rc : tdgl_profile_get(h, &p);
     (void)tdgl_profile_enable(h, 0);
@@ -3491,7 +3492,7 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
     return 0;
   };
   int rc = 0;
-  // the PCG's levels per block: the operator and the vector update per iteration
+  // the PCG's levels per block: the operator and the vector update per iteration, or the residual and the start
   const int kc0 = h->box_kc;
   int best_kc = kc0;
   double best = 1e300;
@@ -3506,6 +3507,7 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
     }
   }
   h->box_kc = best_kc;
+  h->sect = false;
   // m tiles per block of the one-round x-y kernel, timed on the full-length path that launches it
   // (a folded handle's x-y launches are the quarter kernel's), unless a refinement keeps the folds
   const int mt0 = h->plane1;
@@ -3612,7 +3614,7 @@ int tdgl_autotune(tdgl_handle *h, double H, double HJ, tdgl_tuning *out) {
   out->box_kc = h->box_kc;
   out->plane_mt = h->plane1;
   out->zmodes_waves = h->zq_waves;
-  out->fold = h->fold ? 1 : 0;
+  out->fold = sect_scope.on ? 2 : h->fold ? 1 : 0;
   out->zcol = h->zcols;
   out->qparts = h->qparts;
   return 0;
@@ -3926,7 +3928,7 @@ int tdgl_get_stats(tdgl_handle *h, tdgl_stats *st) {
     if (m > 0) st->pcg_budget = m;
   }
   st->captures = h->captures;
-  st->folded = h->sepsect ? 2 : (h->fold || h->fold64) ? 1 : 0;
+  st->folded = (h->sepsect || h->sect) ? 2 : (h->fold || h->fold64) ? 1 : 0;
   st->steps = h->steps;
   st->calls = h->calls;
   st->pcg_iters = h->pcg_iters;

@@ -1,6 +1,7 @@
 """tdgl_autotune: the state, the PCG history and the open boundary come back as they were after the
 tuner's timed steps, every candidate it names was timed, and the steps after a tune agree with the
-steps of an untuned handle.  The PCG box kernels' levels per block decide how the reductions' block
+steps of an untuned handle, by sectors (which the cases take by default) and with the general
+iteration (TDGL_HIP_SECT=0).  The PCG box kernels' levels per block decide how the reductions' block
 partials are summed and the preconditioner's folds how it rounds, so the two agree to the case's
 tolerance against the oracle, not bit for bit; the m tiles, the z pass's waves and its columns or
 x-runs change no bit (test_gpu_parity's kernel-variant test).  Needs a HIP device."""
@@ -12,14 +13,17 @@ from cases import compare_states, make_case, seed_state
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("sect", ["default", "0"])
 @pytest.mark.parametrize("name", ["kwt10_pcg", "pcg_wide_f32", "open_kwt_pcg", "qp_two_kwt_pcg"])
-def test_tune_restores_state_and_steps_agree(name):
+def test_tune_restores_state_and_steps_agree(name, sect, monkeypatch):
     from juliatdgl_amd.hip import HipStepper, device_count
     if device_count() < 1:
         pytest.fail("no HIP device visible")
+    if sect != "default":
+        monkeypatch.setenv("TDGL_HIP_SECT", sect)
     st, tol = make_case(name)
     s0, pcg, H, HJ = seed_state(st)
-    print(f"[gpu] tdgl_autotune on {name}", flush=True)
+    print(f"[gpu] tdgl_autotune on {name}, sectors {sect}", flush=True)
     a = HipStepper(st)
     b = HipStepper(st)
     try:
@@ -56,11 +60,16 @@ def test_tune_restores_state_and_steps_agree(name):
             assert 1 in timed["fold"]
         else:
             assert t["zcol"] in timed["zcol"]
+        # the steps go by sectors, tuned or not, unless the general iteration is asked for
         assert a.stats()["folded"] == t["fold"]
+        assert (t["fold"] == 2) == (b.stats()["folded"] == 2) == (sect == "default")
         a.step(12, H, HJ)
         b.step(12, H, HJ)
         errs = compare_states(a.download(), b.download())
         worst = max(errs.values())
+        a.profile(True)
+        a.step(1, H, HJ)
+        assert a.profile_get()["pcg_sectors"][0] == (sect == "default")
         print(f"[gpu]   tuned {t['box_kc'], t['plane_mt'], t['zmodes_waves'], t['fold'], t['zcol']}: worst {worst:.2e}",
               flush=True)
         assert worst <= tol, errs
