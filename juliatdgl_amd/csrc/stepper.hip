@@ -123,8 +123,9 @@ struct tdgl_handle {
   cplx *U[3] = {}, *V[3] = {};
   double *J[3] = {}, *h[3] = {};
   // workspace
-  cplx *W[TDGL_MAX_BANDS] = {}, *W2[TDGL_MAX_BANDS] = {};  // per band, so that bands step side by side
-  double *Om[TDGL_MAX_BANDS] = {};   // the frame's rate, per band for the same reason
+  cplx *W[TDGL_MAX_BANDS] = {}, *W2[TDGL_MAX_BANDS] = {};  // per band where the bands step side by side (apart), else one
+  double *Om[TDGL_MAX_BANDS] = {};   // the frame's rate, likewise
+  bool apart = false;
   // masks and tables
   double *f = nullptr, *tau[3] = {}, *D[3] = {};
   double *bar[6] = {};
@@ -734,18 +735,22 @@ StageArgs euler_stage(tdgl_handle *h, int mu) {
   return a;
 }
 
-// Whether the bands' stages and the field pass go into common launches: Euler steps and stages without SK-ROCK's
-// source or the low-pass sweeps of a noisy frame (which put other launches between them), launched by themselves
-// (not recorded for a batch, not timed one by one)
-bool bands_merge(const tdgl_handle *h) {
+// Whether the bands' stages and the field pass can go into common launches: Euler steps and stages without SK-ROCK's
+// source or the low-pass sweeps of a noisy frame (which put other launches between them).  Each band then has its own
+// work arrays, up to APART_NODES nodes (40 B a node and band more than one set, 5.4 GB there for three); past that one
+// set serves the bands in turn, where a launch saved is a thousandth of the stages' time.
+constexpr long long APART_NODES = 1LL << 26;
+bool bands_apart(const tdgl_handle *h) {
   const tdgl_desc &d = h->d;
-  if (g_rec || h->prof || !h->merge || frame_first(h) == FRAME_RAW) return false;
+  if (!h->merge || h->g.n > APART_NODES || frame_first(h) == FRAME_RAW) return false;
   for (int mu = 0; mu < d.nbands; ++mu) {
     if (h->noise && d.noise_sk[mu]) return false;
     if (d.stages[mu] == 0 && d.nsub[mu] != 1) return false;
   }
   return true;
 }
+// whether a step does: launched by itself (not recorded for a batch, not timed one by one)
+bool bands_merge(const tdgl_handle *h) { return h->apart && !g_rec && !h->prof; }
 
 PcgArgs pcg_start_args(tdgl_handle *h);
 
@@ -2805,19 +2810,20 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
       ALLOC(h->tau[c], n);
     }
     ALLOC(h->f, n);
-    // the bands on substeps one after the other share the first one's
-    for (int mu = 0; mu < d.nbands; ++mu) {
-      if (d.stages[mu] > 0) {
-        ALLOC(h->W[mu], n);
-        ALLOC(h->W2[mu], n);
-      } else if (d.nsub[mu] > 1) {
-        for (int nu = 0; nu < mu && !h->W[mu]; ++nu) h->W[mu] = h->W[nu];
-        if (!h->W[mu]) ALLOC(h->W[mu], n);
-      }
-    }
-    if (d.rotframe)
-      for (int mu = 0; mu < d.nbands; ++mu) ALLOC(h->Om[mu], n);
     h->noise = d.noise != 0;
+    const char *mg = std::getenv("TDGL_HIP_MERGE");
+    h->merge = mg && mg[0] == '0' ? 0 : 1;
+    h->apart = bands_apart(h);
+    // bands one after the other share the first one's work arrays
+    auto first_of = [&](auto &a, int mu) {
+      for (int nu = 0; nu < mu && !h->apart && !a[mu]; ++nu) a[mu] = a[nu];
+      return !a[mu];
+    };
+    for (int mu = 0; mu < d.nbands; ++mu) {
+      if ((d.stages[mu] > 0 || d.nsub[mu] > 1) && first_of(h->W, mu)) ALLOC(h->W[mu], n);
+      if (d.stages[mu] > 0 && first_of(h->W2, mu)) ALLOC(h->W2[mu], n);
+      if (d.rotframe && first_of(h->Om, mu)) ALLOC(h->Om[mu], n);
+    }
     if (h->noise) {
       ALLOC(h->nctr, 2);
       bool sk = false;
@@ -3026,8 +3032,6 @@ int tdgl_create(const tdgl_desc *desc, tdgl_handle **out) {
     if (qs && qs[0] >= '1' && qs[0] <= '3' && !qs[1]) h->qparts = qs[0] - '0';
     // TDGL_HIP_ZQ_WAVES=4 or 8: the quarter z pass on the vector ALUs with that many waves a block
     // (8 by default), 0: on the matrix cores
-    const char *mg = std::getenv("TDGL_HIP_MERGE");
-    h->merge = mg && mg[0] == '0' ? 0 : 1;
     const char *sx = std::getenv("TDGL_HIP_STENCILXCD");
     h->stxcd = sx && sx[0] == '0' ? 0 : 1;
     const char *zw = std::getenv("TDGL_HIP_ZQ_WAVES");

@@ -173,7 +173,7 @@ def footprint(st: Stepper) -> int:
               + 3 * 2 * 2    # U, V (complex)
               + 3 * 3        # J, h, τ
               + 1 + 3        # f, D
-              + 2 * 2 + 1    # W, W2, Ω
+              + (2 * 2 + 1) * max(1, sum(k > 0 for k in st.rkl))  # W, W2, Ω of every staged band
               + 6 * 2        # separable intermediates (double and float) and sources
               + 12)          # PCG vectors
     if st.field_mode == 2:

@@ -43,3 +43,22 @@ def test_merged_bands_give_the_same_bits(name, monkeypatch):
             d.close()
     for (k, a), (_, b) in zip(outs[0].arrays(), outs[1].arrays()):
         assert np.array_equal(a, b), k
+
+
+@pytest.mark.parametrize("name,own", [("kwt10_pcg", 40), ("kwt10", 40), ("production", 0), ("euler_substeps", 0)])
+def test_bands_in_turn_share_their_work_arrays(name, own, monkeypatch):
+    """A second band's own W, W2 (32 B a node) and frame rate (8 B) are there only where the bands step side by side:
+    with TDGL_HIP_MERGE=0 one set serves all."""
+    from juliatdgl_amd.hip import HipStepper
+    st, _ = make_case(name)
+    print(f"[gpu] work arrays of {name}", flush=True)
+    held = {}
+    for v in ("0", "1"):
+        monkeypatch.setenv("TDGL_HIP_MERGE", v)
+        d = HipStepper(st)
+        held[v] = d.stats()["device_bytes"]
+        d.close()
+    nodes = (st.grid.Nx + 1) * (st.grid.Ny + 1) * (st.grid.Nz + 1)
+    extra = held["1"] - held["0"]
+    print(f"    {extra} B more side by side ({extra / nodes:.1f} a node)", flush=True)
+    assert extra >= own * nodes if own else extra == 0
