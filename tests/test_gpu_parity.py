@@ -71,6 +71,29 @@ def test_hip_matches_oracle(name):
         assert abs(gi - oi) <= max(2, oi // 4), (gi, oi)
 
 
+# the cases whose field solve goes by sectors, which the general iteration (TDGL_HIP_SECT=0) still has to run
+SECTOR_CASES = ["pcg_fast_f32", "pcg_tight_f32", "kwt10_pcg", "qp_two_kwt_pcg", "pcg_wide_f32", "pcg_mf1_f32",
+                "kwt10_mf1_pcg", "open_kwt_pcg"]
+
+
+def _solver(sect, monkeypatch, st):
+    """TDGL_HIP_SECT, and the solver that steps of `st` then take."""
+    if sect != "default":
+        monkeypatch.setenv("TDGL_HIP_SECT", sect)
+    dev = _hip()(st)
+    folded = dev.stats()["folded"]
+    dev.close()
+    assert (folded == 2) == (sect == "default"), (folded, sect)
+
+
+@pytest.mark.parametrize("name", SECTOR_CASES)
+def test_hip_general_iteration_matches_oracle(name, monkeypatch):
+    st, _ = make_case(name)
+    _solver("default", monkeypatch, st)
+    _solver("0", monkeypatch, st)
+    test_hip_matches_oracle(name)
+
+
 GRAPH_CASES = ["production", "euler_substeps", "pcg_fast_f32", "pcg_exact", "kwt10_pcg", "three_aniso", "kwt10_euler",
                "qp_two_kwt_pcg", "qp_three", "open", "open_kwt_pcg"]
 
@@ -264,11 +287,14 @@ def test_hip_open_boundary_resumes_and_is_odd_in_the_current():
     assert np.max(np.abs(p.hz + m.hz)) < 1e-13 and np.max(np.abs(p.hz)) > 1e-4
 
 
-def test_hip_pcg_budget_shrinks_and_changes_nothing(monkeypatch):
+@pytest.mark.parametrize("sect", ["0", "default"])
+def test_hip_pcg_budget_shrinks_and_changes_nothing(sect, monkeypatch):
     """The PCG budget learned from the cold first cycle shrinks once the solves run shorter, and the
-    graph cycles that follow give the eager steps' state to the bit."""
+    graph cycles that follow give the eager steps' state to the bit (by sectors the budget is learnt
+    and gates nothing)."""
     HipStepper = _hip()
     st, _ = make_case("kwt10_pcg")
+    _solver(sect, monkeypatch, st)
     s0, pcg, H, HJ = seed_state(st)
     print("[gpu] PCG budget", flush=True)
     runs = []
@@ -355,15 +381,17 @@ def test_hip_long_runs_match_the_oracle(name, cycles):
     assert max(errs.values()) <= 1e-8, errs
 
 
-def test_pcg_budget_settles_on_a_current_ramp():
+@pytest.mark.parametrize("sect", ["0", "default"])
+def test_pcg_budget_settles_on_a_current_ramp(sect, monkeypatch):
     """Captured cycles while the current steps up every cycle (the solves' lengths move): the
     results equal the eager steps, and the budget neither flips every cycle nor recaptures each
     time (roll backs hold the budget for a few cycles; the last graphs are kept)."""
     from juliatdgl_amd.hip import HipStepper
     _hip()
     st, tol = make_case("kwt10_pcg")
+    _solver(sect, monkeypatch, st)
     s0, pcg, H, _ = seed_state(st)
-    print("[gpu] PCG budget on a current ramp", flush=True)
+    print(f"[gpu] PCG budget on a current ramp, sectors {sect}", flush=True)
     outs, stats = [], []
     for graphs in ("1", "0"):
         import os
@@ -555,7 +583,8 @@ def test_folded_fp64_solve_matches_full_length(name, monkeypatch):
     assert max(core.values()) <= 1e-12, errs
 
 
-def test_open_pcg_step_class_budgets_give_the_same_bits(monkeypatch):
+@pytest.mark.parametrize("sect", ["0", "default"])
+def test_open_pcg_step_class_budgets_give_the_same_bits(sect, monkeypatch):
     """With the open boundary, a call's steps replay one-step graphs whose gated PCG budgets follow
     the steps since the last recomputation of h_δ (the default), against one graph a call with one
     budget (TDGL_HIP_STEPWISE=0) and against steps launched from the host (TDGL_HIP_GRAPH=0): eight
@@ -564,6 +593,7 @@ def test_open_pcg_step_class_budgets_give_the_same_bits(monkeypatch):
     most the single one."""
     HipStepper = _hip()
     st, _ = make_case("open_kwt_pcg")
+    _solver(sect, monkeypatch, st)
     s0, pcg, H, HJ = seed_state(st)
     outs, stats = [], []
     for env in ({}, {"TDGL_HIP_STEPWISE": "0"}, {"TDGL_HIP_GRAPH": "0"}):

@@ -18,13 +18,17 @@ def _hip():
     return HipStepper
 
 
+@pytest.mark.parametrize("sect", ["default", "0"])
 @pytest.mark.parametrize("graph", ["0", "1"])
 @pytest.mark.parametrize("name", ["pcg_fast_f32", "pcg_tight_f32", "kwt10_pcg", "open_kwt_pcg", "qp_two_kwt_pcg",
                                   "pcg_mf1_f32"])
-def test_refinement_matches_the_oracle(name, graph, monkeypatch):
+def test_refinement_matches_the_oracle(name, graph, sect, monkeypatch):
+    """By sectors (default) and by the Float32 inner solves (TDGL_HIP_SECT=0)."""
     from oracle.oracle import Oracle
     HipStepper = _hip()
     monkeypatch.setenv("TDGL_HIP_GRAPH", graph)
+    if sect != "default":
+        monkeypatch.setenv("TDGL_HIP_SECT", sect)
     st, tol = make_case(name, pcg_refine=True)
     s0, pcg, H, HJ = seed_state(st)
     n = 20
@@ -41,6 +45,7 @@ def test_refinement_matches_the_oracle(name, graph, monkeypatch):
     out = dev.download()
     stt = dev.stats()
     dev.close()
+    assert (stt["folded"] == 2) == (sect == "default")
     errs = compare_states(out, ref)
     core = {k: v for k, v in errs.items() if not k.startswith(("U", "V"))}
     worst = max(core, key=core.get)
@@ -115,13 +120,16 @@ def test_refinement_meets_its_tolerance(tol):
     assert res <= tol + 2e-15
 
 
-def test_refinement_against_all_fp64_on_the_three_band_workload():
+@pytest.mark.parametrize("sect", ["default", "0"])
+def test_refinement_against_all_fp64_on_the_three_band_workload(sect, monkeypatch):
     """The three-band anisotropic open-boundary workload (buf 8, tol 1e-8) on 48x24x8 cells: the
     refinement against an all-FP64 run (FP64 preconditioner) after 80 steps; ψ and A agree to the
     solver's tolerance scale."""
     from juliatdgl_amd.configs import open_3band_256x128x32
     from juliatdgl_amd.state import seeded_state
     HipStepper = _hip()
+    if sect != "default":
+        monkeypatch.setenv("TDGL_HIP_SECT", sect)
     outs = []
     for kw in (dict(pcg_refine=True), dict(pcg_f32=False, pcg_fast=False)):
         st, p = open_3band_256x128x32(nx=48, ny=24, nz=8, **kw)
@@ -138,7 +146,8 @@ def test_refinement_against_all_fp64_on_the_three_band_workload():
     assert max(v for k, v in errs.items() if not k.startswith(("U", "V"))) <= 1e-6, errs
 
 
-def test_refinement_onset_bins_against_all_fp64():
+@pytest.mark.parametrize("sect", ["default", "0"])
+def test_refinement_onset_bins_against_all_fp64(sect, monkeypatch):
     """The golden ladder's sample with an insulating buffer (buf 2, σvac/σn = 0.01, PCG tol 1e-10):
     the two-polarity ladders stepped with the refinement have the verdicts, cycles and onset
     brackets of the same ladders stepped with every part of the PCG in FP64, and 400 steps at J = 0.6
@@ -148,6 +157,8 @@ def test_refinement_onset_bins_against_all_fp64():
     from juliatdgl_amd.state import initial_state
     from test_ladder import golden_setup
     HipStepper = _hip()
+    if sect != "default":
+        monkeypatch.setenv("TDGL_HIP_SECT", sect)
     _, _, st0, pr = golden_setup()
     gr = Grid.make(24, 12, 4, dx=0.5, buf=2)
     mk = wedge_masks(gr)
