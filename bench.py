@@ -356,11 +356,16 @@ def cpu_sample(name, st, dev, H, HJ, nsteps):
             "single_thread": {"value": v1, "cores": 1, "seconds": d1}, "cpu_model": model}
 
 
+def matrix_peak(name: str, sect) -> float:
+    """The matrix rate of the precision a transform class runs in (the sectors of the separable solve are FP64)."""
+    return FP32_MFMA_PEAK if name == "sep_transform_f32" or (name == "sep_modes" and sect != "sep") else FP64_PEAK
+
+
 def roofline(st, dom, nl, ms, nsteps, iters, workload, folded=False, sect=None):
     avg_s = ms / nl / 1e3
     byts = kernel_bytes(st, dom, nl, nsteps, {"iters_per_solve": iters / nsteps, "folded": folded, "sect": sect}) / nl
     flops = kernel_flops(st, dom, nl, folded, sect) / nl
-    peak = FP32_MFMA_PEAK if dom in ("sep_transform_f32", "sep_modes") else FP64_PEAK
+    peak = matrix_peak(dom, sect)
     if byts > 0 and (flops == 0 or flops / byts < peak / HBM_PEAK):
         roof = {"bound": "hbm", "achieved": byts / avg_s / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                 "frac": byts / avg_s / HBM_PEAK, "traffic": None, "kernel": dom, "bytes_per_launch": byts,
@@ -368,8 +373,10 @@ def roofline(st, dom, nl, ms, nsteps, iters, workload, folded=False, sect=None):
                 "note": "algorithmic bytes: each array the launch must touch counted once (FP64 node-shaped vectors, "
                         "FP32 quarters); durations from HIP events recorded at each launch's start and end over the "
                         "same number of cycles as the timed region" +
-                        ("; the launch holds every iteration of the solve in LDS and registers: the bound is the "
-                         "issue of its stencil, products and sums" if dom == "pcg_sectors" else "")}
+                        ("; r in and d out only: the launch holds every iteration of the solve in LDS and registers, so "
+                         "this fraction says that it is far from HBM-bound and no more (its issue, matrix and wait cycles: "
+                         "profiles/pcg_sectors_open_3band_256x128x32_sq_counters.txt; its products' flops depend on each "
+                         "sector's iterations, of which the longest is known here)" if dom == "pcg_sectors" else "")}
     else:
         roof = {"bound": "mfma", "achieved": flops / avg_s / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                 "frac": flops / avg_s / peak, "traffic": None, "kernel": dom, "flops_per_launch": flops,
@@ -474,11 +481,13 @@ def run_workload(name, steps, warmup, profile=True, cpu_steps=0, profile_out=Non
             row = {"us_per_launch": us, "bytes_per_launch": b, "GB_s": b / us / 1e3, "hbm_frac": b / us / 1e3 / (HBM_PEAK / 1e9)}
             f = kernel_flops(st, kname, nl_k, folded, sect) / nl_k
             if f > 0:
-                pk = FP32_MFMA_PEAK if kname in ("sep_transform_f32", "sep_modes") else FP64_PEAK
+                pk = matrix_peak(kname, sect)
                 row["TFLOP_s"] = f / us / 1e6
                 row["mfma_frac"] = f / us / 1e6 / (pk / 1e12)
             per[kname] = row
         out["config"]["kernel_roofline"] = per
+        out["config"]["kernel_timing"] = ("each kernel launched and timed apart; the timed cycles run the bands' stages with "
+                                          "the field pass or the PCG's start, and the curl with the ghosts, in common launches")
         if profile_out:
             with open(profile_out, "w") as fh:
                 json.dump({k: {"launches": v[0], "ms": v[1]} for k, v in prof.items()}, fh, indent=1)
