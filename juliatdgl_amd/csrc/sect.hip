@@ -597,10 +597,12 @@ hipError_t launch_sect_batch(int kind, int variant, size_t lds, const BatchTab &
 // the first residual, so the sectors' residuals together are below the tolerance, no sector iterates for
 // the others and one that holds almost nothing stops at once.  What is left is spread over the sectors and
 // not where the general iteration leaves it, and at the tolerance itself the fields came out up to nine
-// times further from a solution to the rounding than that iteration's (2.4e-8 against 2.5e-9 after six
-// cycles of 96x48x24 cells, 9.2e-8 against 2.8e-8 after one of 53x27x9); at an eighth of it they are nearer
-// (1.5e-8 on 53x27x9, 3.3e-8 against 2.0e-7 on 144x17x21, 9e-11 against 6e-10 with KWT) or as near (5.4e-9
-// against 2.5e-9 and 7.1e-9, full length and folded, on 96x48x24), for 15 % more iterations.
+// times further from a solution to the rounding than that iteration's.  At a 16th they are nearer than by either
+// of its preconditioner's paths (folds, full length) on all 28 runs measured: 2.3e-9 against 2.5e-9 and 7.1e-9 after
+// six cycles of 96x48x24 cells, 8.3e-9 against 2.8e-8 and 7.3e-8 after one of 53x27x9, 8.7e-9 against 2.7e-8 and 1.3e-8
+// (43x86x6), 6.9e-11 against 9.0e-10 and 8.7e-10 with KWT (128x64x16).  At an eighth three of them were further by up to
+// twice (5.4e-9 on 96x48x24, 1.6e-8 on 43x86x6, 1.3e-8 against 1.0e-8 on 72x41x8); a 16th takes 4 to 8 % more
+// iterations, a 24th another 3 %.
 // the same value, which the compiler does not know to be: what is derived from it is formed where it is used
 // and not kept in registers through the iterations
 __device__ __forceinline__ int fresh(int v) {

@@ -1556,11 +1556,11 @@ SectCG sect_cg(tdgl_handle *h) {
   a.ca = h->d.sxy / (h->d.dx * h->d.dy);
   a.a = h->d.a;
   a.share = 1.0 / (4.0 * h->sq.nx);
-  // k_sect_cg says why an eighth.  The last Float32 solve of a refinement leaves its residual well below the
+  // k_sect_cg says why a 16th.  The last Float32 solve of a refinement leaves its residual well below the
   // tolerance: 4.8e-10 to 3.9e-8 from a solution to the rounding over five grids of 16 to 64 cells across, where
   // an eighth left 1.2e-9 to 1.5e-8 (up to five times more), a 32nd up to 1.2 times more and a 128th a ninth
   // to a half as much or less, for four iterations more than an eighth
-  a.tight = h->d.pcg_refine ? 1.0 / 128 : 1.0 / 8;
+  a.tight = h->d.pcg_refine ? 1.0 / 128 : 1.0 / 16;
   a.maxit = h->d.pcg_maxit;
   return a;
 }
