@@ -9,8 +9,8 @@
 // runs the whole flexible CG of a sector in one launch, k_sect_inv takes the solution back.  The general
 // iteration's six launches and 860 MB of HBM traffic (290 us on 256x128x32 cells, 20 to 24 a step; 50 us,
 // launch-bound, on 96x48x24) become one launch a solve, whose iterations leave the CU only for the bases:
-// a time step took 7.86 -> 1.35 ms on 256x128x32 cells, 458 -> 132 us on 96x48x24, 610 -> 155 us on 128x64x16 with
-// KWT, 327 -> 77 us on 53x27x9 (with the open boundary's and the launches' own savings).
+// a time step took 7.86 -> 1.42 ms on 256x128x32 cells, 458 -> 136 us on 96x48x24, 610 -> 160 us on 128x64x16 with
+// KWT, 327 -> 78 us on 53x27x9 (with the open boundary's and the launches' own savings).
 //
 // A sector holds values on the half domain (the rest follows by parity): component c of mode mx at
 // (j, k), j fastest, X (c = 0) then Y then Z.  With (py, pz) the parities of the sector's y and z wave
@@ -598,7 +598,7 @@ hipError_t launch_sect_batch(int kind, int variant, size_t lds, const BatchTab &
 // the others and one that holds almost nothing stops at once.  What is left is spread over the sectors and
 // not where the general iteration leaves it, and at the tolerance itself the fields came out up to nine
 // times further from a solution to the rounding than that iteration's.  At a 16th they are nearer than by either
-// of its preconditioner's paths (folds, full length) on all 28 runs measured: 2.3e-9 against 2.5e-9 and 7.1e-9 after
+// of its preconditioner's paths (folds, full length) on all 27 runs measured: 2.3e-9 against 2.5e-9 and 7.1e-9 after
 // six cycles of 96x48x24 cells, 8.3e-9 against 2.8e-8 and 7.3e-8 after one of 53x27x9, 8.7e-9 against 2.7e-8 and 1.3e-8
 // (43x86x6), 6.9e-11 against 9.0e-10 and 8.7e-10 with KWT (128x64x16).  At an eighth three of them were further by up to
 // twice (5.4e-9 on 96x48x24, 1.6e-8 on 43x86x6, 1.3e-8 against 1.0e-8 on 72x41x8); a 16th takes 4 to 8 % more
