@@ -82,18 +82,22 @@ def test_batched_sectors(sizes, monkeypatch):
         d.close()
 
 
-def test_batched_sectors_beside_folds():
-    """Wide runs, some by sectors and some by the folded transforms, in one batch: each is where its own steps
-    leave it, to the bit."""
+@pytest.mark.parametrize("graph", ["1", "0"])
+@pytest.mark.parametrize("sizes,paths", [([(170, 100, 30), (170, 100, 20), (60, 200, 14)], [2, 1, 2]),
+                                         ([(256, 128, 20), (200, 100, 24)], [1, 1])])
+def test_batched_sectors_beside_folds(sizes, paths, graph, monkeypatch):
+    """Wide runs, some by sectors and some by the folded transforms (the last two on different kernels of them), in one
+    batch, replayed or launched from the host: each is where its own steps leave it, to the bit."""
     from juliatdgl_amd.hip import HipBatch
-    sizes, H = [(170, 100, 30), (170, 100, 20), (60, 200, 14)], 0.03
+    H = 0.03
+    monkeypatch.setenv("TDGL_HIP_GRAPH", graph)
     print(f"[gpu] batched sectors beside folds {sizes}", flush=True)
     alone = []
     for st, d in _steppers(sizes):
         d.step(4, H, st.selffield(0.3))
         alone.append((d.download(), d.stats()["folded"]))
         d.close()
-    assert [f for _, f in alone] == [2, 1, 2]
+    assert [f for _, f in alone] == paths
     runs = _steppers(sizes)
     b = HipBatch([d for _, d in runs])
     for _ in range(2):
